@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libchfsi.so")
 SOURCES = ["kernels.hip", "kernels_bloch.hip", "operator.hip", "solver.hip", "bloch.hip",
-           "dense.hip"]
+           "dense.hip", "tensor.hip"]
 ROOT = os.path.dirname(HERE)
 DROPIN_SRC = os.path.join(ROOT, "tests", "cpp", "dropin_solve.cpp")
 DROPIN = os.path.join(HERE, "bin", "dropin_solve")

@@ -17,6 +17,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "operator.hpp"
+#include "tensor.hpp"
 
 namespace chfsi {
 
@@ -80,7 +81,9 @@ chfsi_operator::~chfsi_operator() {
                   d_m_slaves, d_m_vals, d_Mc, d_Gd, d_Hk64, d_Hk32, d_nlCk64, d_nlCtk64,
                   d_nlCk32, d_nlCtk32, d_invJ, d_s_gather64, d_ones_cons64, d_s_gather32,
                   d_ones_cons32, d_own_map, d_own_n, d_nlCto64, d_nlCto32, d_nlCtko64,
-                  d_nlCtko32};
+                  d_nlCtko32, d_ttab64, d_ttab32, d_vq64,
+                  d_vq32, d_nlCp64,
+                  d_nlCp32};
   for (void *p : ptrs)
     if (p) hipFree(p);
   ztab_dev.release();
@@ -251,6 +254,8 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
     cells_sorted.insert(cells_sorted.end(), by_color[k].begin(), by_color[k].end());
     op->color_off[k + 1] = (int)cells_sorted.size();
   }
+  for (int k = 0; k < op->ncolors; ++k)
+    op->max_color_cells = std::max(op->max_color_cells, op->color_off[k + 1] - op->color_off[k]);
   std::vector<uint32_t> map(size_t(Ctot) * ne);
   std::vector<int> touched_color(M, -1);
   std::vector<int> touched_cell(M, -1);
@@ -293,6 +298,18 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
       CHFSI_TRY(dev_upload(&op->d_K, d->cell_stiffness, size_t(C) * ne * ne));
     } else {
       CHFSI_TRY(dev_upload(&op->d_K, d->stiffness, size_t(ne) * ne));
+    }
+    std::vector<double> tab;
+    std::vector<float> tab32;
+    if (!d->cell_stiffness && Ctot == C &&
+        tensor_tables(d->shape_values, d->stiffness, ne, op->nq, &tab, &tab32)) {
+      tensor_shape(ne, op->nq, &op->tn, &op->tq);
+      const int qe = (op->tq + 1) / 2;
+      const size_t nv = size_t(C) * qe * qe * 4 * op->tq;
+      CHFSI_TRY(dev_upload(&op->d_ttab64, tab.data(), tab.size()));
+      CHFSI_TRY(dev_upload(&op->d_ttab32, tab32.data(), tab32.size()));
+      CHFSI_TRY(dev_alloc(&op->d_vq64, nv));
+      CHFSI_TRY(dev_alloc(&op->d_vq32, nv));
     }
     if (d->shape_gradients)
       CHFSI_TRY(dev_upload(&op->d_Gq, d->shape_gradients, size_t(op->nq) * ne * 3));
@@ -538,6 +555,12 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
     }
     CHFSI_TRY(dev_alloc(&op->d_nlC16, nlC.size()));
     CHFSI_HIP(launch_f64_to_bf16(op->d_nlC64, (int64_t)nlC.size(), op->d_nlC16, 0));
+    if (op->tn) {
+      CHFSI_TRY(dev_alloc(&op->d_nlCp64, nlC.size()));
+      CHFSI_TRY(dev_alloc(&op->d_nlCp32, nlC.size()));
+      CHFSI_HIP(launch_tensor_projectors(op->d_nlC64, (int64_t)nlC.size(), op->tn, ne, ne_pad,
+                                         op->d_nlCp64, op->d_nlCp32, 0));
+    }
     CHFSI_TRY(dev_upload(&op->d_proj_ptr, proj_ptr.data(), proj_ptr.size()));
     CHFSI_TRY(dev_upload(&op->d_proj_slots, proj_slots.data(), proj_slots.size()));
     CHFSI_TRY(dev_upload(&op->d_proj_V, d->proj_V, d->n_proj));
@@ -557,6 +580,10 @@ extern "C" chfsi_status chfsi_operator_set_potential(chfsi_operator *op, const d
   CHFSI_HIP(launch_build_h(op->d_K, op->d_Nq, vJxW, nullptr, nullptr, op->C, op->ne, op->ne_pad,
                            op->nq, op->d_Ht64, op->d_Ht32, op->d_Ht16, as_stream(stream),
                            op->K_per_cell));
+  if (op->tn)
+    CHFSI_HIP(launch_tensor_potential(vJxW, op->C, op->tn, op->tq, op->d_vq64, op->d_vq32,
+                                      as_stream(stream)));
+  op->tensor_pot = op->tn > 0;
   op->has_H = true;
   op->h_sym = true;  // the build writes each off-diagonal pair block from one sum
   return rebuild_kpoint_matrices(op, as_stream(stream));
@@ -570,6 +597,7 @@ extern "C" chfsi_status chfsi_operator_set_potential_gga(chfsi_operator *op, con
   CHFSI_HIP(launch_build_h(op->d_K, op->d_Nq, vJxW, op->d_Gq, gJxW, op->C, op->ne, op->ne_pad,
                            op->nq, op->d_Ht64, op->d_Ht32, op->d_Ht16, as_stream(stream),
                            op->K_per_cell, op->d_invJ, op->jac));
+  op->tensor_pot = false;
   op->has_H = true;
   op->h_sym = true;
   return rebuild_kpoint_matrices(op, as_stream(stream));
@@ -582,6 +610,7 @@ extern "C" chfsi_status chfsi_operator_set_cell_matrices(chfsi_operator *op, con
                           as_stream(stream)));
   CHFSI_HIP(launch_f64_to_bf16(op->d_Ht64, int64_t(op->C) * op->ne_pad * op->ne_pad, op->d_Ht16,
                                as_stream(stream)));
+  op->tensor_pot = false;
   op->has_H = true;
   op->h_sym = false;  // caller's matrices: not assumed symmetric
   return rebuild_kpoint_matrices(op, as_stream(stream));
@@ -649,6 +678,9 @@ template <>
 struct OpData<double> {
   static const double *Ht(chfsi_operator *op) { return op->d_Ht64; }
   static const double *nlC(chfsi_operator *op) { return op->d_nlC64; }
+  static const double *ttab(chfsi_operator *op) { return op->d_ttab64; }
+  static const double *vq(chfsi_operator *op) { return op->d_vq64; }
+  static const double *nlCp(chfsi_operator *op) { return op->d_nlCp64; }
   static const double *nlCt(chfsi_operator *op) { return op->d_nlCt64; }
   static const double *nlCto(chfsi_operator *op) { return op->d_nlCto64; }
   static const double *s(chfsi_operator *op) { return op->d_inv_sqrt_mass; }
@@ -661,6 +693,9 @@ template <>
 struct OpData<float> {
   static const float *Ht(chfsi_operator *op) { return op->d_Ht32; }
   static const float *nlC(chfsi_operator *op) { return op->d_nlC32; }
+  static const float *ttab(chfsi_operator *op) { return op->d_ttab32; }
+  static const float *vq(chfsi_operator *op) { return op->d_vq32; }
+  static const float *nlCp(chfsi_operator *op) { return op->d_nlCp32; }
   static const float *nlCt(chfsi_operator *op) { return op->d_nlCt32; }
   static const float *nlCto(chfsi_operator *op) { return op->d_nlCto32; }
   static const float *s(chfsi_operator *op) { return op->d_inv_sqrt_mass32; }
@@ -759,13 +794,17 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
   a.beta_mode = beta_mode;
   a.B = B;
   a.variant = sizeof(T) == 8 ? op->hx_variant64 : (bf16 ? op->hx_variant16 : op->hx_variant32);
+  const bool tensor = a.variant < 0 && !bf16 && op->tensor_pot &&
+                      ld_src < (int64_t(1) << 29) && ld_dst < (int64_t(1) << 29) &&
+                      ldR < (int64_t(1) << 29) &&  // the kernels' row offsets are 32-bit bytes
+                      tensor_wins(op->tn, sizeof(T) == 8, op->max_color_cells, B);
   a.R = R;
   a.ldR = ldR;
   a.rcoef = rcoef;
   a.h_sym = op->h_sym ? 1 : 0;
   if (op->n_slots > 0) {
     a.nl_off = op->d_nl_off;
-    a.nl_C = OpData<T>::nlC(op);
+    a.nl_C = tensor ? OpData<T>::nlCp(op) : OpData<T>::nlC(op);
     a.slot_proj = op->d_slot_proj;
     a.W = W;
     a.ldW = B;
@@ -780,7 +819,10 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
         continue;
       }
     }
-    CHFSI_HIP(launch_hx<T>(a, s));
+    if (tensor)
+      CHFSI_HIP(launch_hx_tensor<T>(a, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq, s));
+    else
+      CHFSI_HIP(launch_hx<T>(a, s));
   }
   if (op->general_constraints) {
     // distribute_slave_to_master (kohnShamDFTOperatorDevice.cc:3832-3838):
@@ -930,8 +972,10 @@ chfsi_status time_variants(chfsi_operator *op, int B, int *best, float *times, h
   CHFSI_HIP(hipEventCreate(&e0));
   CHFSI_HIP(hipEventCreate(&e1));
   int &var = sizeof(T) == 8 ? op->hx_variant64 : op->hx_variant32;
-  float best_t = 1e30f;
-  for (int v = 0; v < nv; ++v) {
+  float best_t = 1e30f, tensor_t = 1e30f;
+  // v = -1: the tensor form, where the operator has it (kept when it is faster
+  // than every tile variant; *best and times report the tile variants)
+  for (int v = op->tensor_pot ? -1 : 0; v < nv; ++v) {
     var = v;
     const T *xs = static_cast<const T *>(x.ptr);
     T *ys = static_cast<T *>(y.ptr);
@@ -945,13 +989,17 @@ chfsi_status time_variants(chfsi_operator *op, int B, int *best, float *times, h
     }
     float ms = 1e30f;
     if (stt == CHFSI_OK) CHFSI_HIP(hipEventElapsedTime(&ms, e0, e1));
+    if (v < 0) {
+      tensor_t = ms;
+      continue;
+    }
     times[v] = stt == CHFSI_OK ? ms / 3 : -1.0f;
     if (stt == CHFSI_OK && ms < best_t) {
       best_t = ms;
       *best = v;
     }
   }
-  var = *best;
+  var = tensor_t < best_t ? -1 : *best;
   // projection variants with the chosen tile variant, timed as whole applies
   if (op->n_slots > 0) {
     int &pv = sizeof(T) == 8 ? op->proj_variant64 : op->proj_variant32;

@@ -59,6 +59,7 @@ struct chfsi_operator {
   static constexpr int kMaxColors = 128;
   int ncolors = 0;
   int color_off[kMaxColors + 1] = {0};
+  int max_color_cells = 0;
   // Loewdin scalings
   double *d_sqrt_mass = nullptr, *d_inv_sqrt_mass = nullptr;
   float *d_sqrt_mass32 = nullptr, *d_inv_sqrt_mass32 = nullptr;
@@ -89,8 +90,19 @@ struct chfsi_operator {
   double *d_nlCto64 = nullptr;
   float *d_nlCto32 = nullptr;
   chfsi::Scratch partial64, partial32, W64, W32, tmp;
-  // HX tile and projection variants per precision (chosen by chfsi_operator_autotune)
-  int hx_variant64 = 0, hx_variant32 = 0;
+  // tensor-product form of the cell operators (tensor.hpp): nodes and Gauss
+  // points per direction (0: the shape data is not of that form), the parity
+  // tables, the potential's weights in the kernels' order
+  // and the projector columns in their x-parity rows.  tensor_pot:
+  // the cell matrices are those of the weights held here (an LDA potential)
+  int tn = 0, tq = 0;
+  bool tensor_pot = false;
+  double *d_ttab64 = nullptr, *d_vq64 = nullptr, *d_nlCp64 = nullptr;
+  float *d_ttab32 = nullptr, *d_vq32 = nullptr, *d_nlCp32 = nullptr;
+  // HX tile and projection variants per precision (chosen by
+  // chfsi_operator_autotune); -1: the tensor form where the operator has it,
+  // tile variant 0 otherwise
+  int hx_variant64 = -1, hx_variant32 = -1;
   int hx_variant16 = 0;  // BF16 apply: 0 K = 32 ring, 1 register-staged K = 16
   int proj_variant64 = 0, proj_variant32 = 0;
   int max_srb = 1;  // largest slot count of any cell / 16

@@ -1,0 +1,1175 @@
+// Tensor-product cell operators (see tensor.hpp).
+//
+// A cell with n GLL nodes and q Gauss points per direction applies
+//   y = 1/2 K x + N^T diag(v JxW) N x,   N = I (x) I (x) I,
+//   K = a_x K1 (x) M1 (x) M1 + a_y M1 (x) K1 (x) M1 + a_z M1 (x) M1 (x) K1
+// direction by direction: at n = 7, q = 8 about 2.4e4 operations per column
+// against 2.4e5 of the dense 343 x 343 product.  All one-dimensional tables are
+// centro-symmetric, so a line is split into its even and odd part
+// (x_{+-i} = E_i +- O_i), which halves the products again and lets the even-x
+// and odd-x halves of a plane live in different waves.
+//
+// Scaling: the input carries a factor 1/8 (one half per direction, so that
+// E_i = x_i + x_{-i}, O_i = x_i - x_{-i} and a middle node enters alone), and
+// the weights at the quadrature points the same factor for the way back
+// (another half per direction whose quadrature index is the middle one).  All
+// of these are powers of two, so nothing is rounded by them.
+
+#include <algorithm>
+#include <cmath>
+
+#include "mfma.hpp"
+#include "scatter.hpp"
+#include "tensor.hpp"
+
+namespace chfsi {
+
+// ---------------------------------------------------------------------------
+// One-dimensional tables (host): taken from the operator's own arrays, so that
+// the apply agrees with its dense form to rounding
+// ---------------------------------------------------------------------------
+namespace {
+
+typedef long double ld;
+
+// Gauss weights on [0, 1] (Newton on the Legendre polynomial P_q)
+std::vector<ld> gauss_weights(int q) {
+  std::vector<ld> w(q);
+  for (int i = 0; i < q; ++i) {
+    ld t = cosl(acosl(-1.0L) * (q - i - 0.25L) / (q + 0.5L)), d = 1;
+    for (int it = 0; it < 50; ++it) {
+      ld p0 = 1, p1 = t;
+      for (int k = 2; k <= q; ++k) {
+        const ld p2 = ((2 * k - 1) * t * p1 - (k - 1) * p0) / k;
+        p0 = p1;
+        p1 = p2;
+      }
+      d = q * (t * p1 - p0) / (t * t - 1);
+      t -= p1 / d;
+    }
+    w[i] = 1 / ((1 - t * t) * d * d);
+  }
+  return w;
+}
+
+// Mean of a rows x cols table and its point reflection
+void symmetrise(std::vector<ld> &A) {
+  for (size_t i = 0, j = A.size() - 1; i < j; ++i, --j) A[i] = A[j] = (A[i] + A[j]) / 2;
+}
+
+// v[j] = A[j] on the grid of FP32 values below `big`, with the sum over a
+// constant (a middle value enters with one half) made `target` by entry `fix`
+void balance(const double *A, int n, bool middle, double big, double target, int fix,
+             double *out) {
+  const double g = std::ldexp(1.0, std::ilogb(big) + 1 - 24);
+  double sum = 0;
+  for (int j = 0; j < n; ++j) {
+    const double k = middle && j == n - 1 ? 0.5 : 1.0;
+    const double r = std::nearbyint(A[j] * k / g) * g;
+    out[j] = r / k;
+    sum += r;
+  }
+  out[fix] += (target - sum) / (middle && fix == n - 1 ? 0.5 : 1.0);
+}
+
+}  // namespace
+
+// FP64 tables: [parity][row][column] blocks over the first half of the rows and
+// columns, even part A[r][c] + A[r][-c], odd part A[r][c] - A[r][-c] (padded
+// with zeros to the size of the even one)
+template <int N, int Q>
+struct TensorTab {
+  static constexpr int NE = (N + 1) / 2, NO = N / 2;  // even / odd nodal values of a line
+  static constexpr int QE = (Q + 1) / 2, QO = Q / 2;  // even / odd quadrature values
+  static constexpr int oI = 0, oM = oI + 2 * QE * NE;
+  static constexpr int oKx = oM + 2 * NE * NE, oKy = oKx + 2 * NE * NE, oKz = oKy + 2 * NE * NE;
+  static constexpr int oW = oKz + 2 * NE * NE;        // 1/2 w, the middle one 1/4 w
+};
+
+// FP32 operand tables of the 4 x 4 products: [table][row][column], zero beyond
+// the blocks, then the weights
+enum {
+  kTabIe, kTabIo, kTabIeT, kTabIoT, kTabMe, kTabMo, kTabKx, kTabKxo, kTabKy, kTabKyo, kTabKz,
+  kTabKzo, kTabs
+};
+
+bool tensor_shape(int ne, int nqc, int *n, int *q) {
+  static const int shapes[3][2] = {{5, 5}, {6, 6}, {7, 8}};
+  for (auto &s : shapes)
+    if (ne == s[0] * s[0] * s[0] && nqc == s[1] * s[1] * s[1]) {
+      *n = s[0];
+      *q = s[1];
+      return true;
+    }
+  return false;
+}
+
+bool tensor_tables(const double *Nq, const double *K, int ne, int nqc, std::vector<double> *tab,
+                   std::vector<float> *tab32) {
+  int n = 0, q = 0;
+  if (!tensor_shape(ne, nqc, &n, &q)) return false;
+  const double tol = 1e-13;
+  const std::vector<ld> w = gauss_weights(q);
+  // I: sums of N over the nodes of the other two directions (which are one),
+  // mean over their quadrature points and over the directions; x is the
+  // fastest index of nodes and points
+  std::vector<ld> I(size_t(q) * n, 0), M(size_t(n) * n, 0), Kd[3];
+  for (int k = 0; k < nqc; ++k)
+    for (int i = 0; i < ne; ++i) {
+      const ld v = Nq[size_t(k) * ne + i] / ld(3 * q * q);
+      I[(k % q) * n + i % n] += v;
+      I[(k / q % q) * n + i / n % n] += v;
+      I[(k / q / q) * n + i / n / n] += v;
+    }
+  symmetrise(I);
+  for (int a = 0; a < n; ++a)
+    for (int b = 0; b < n; ++b)
+      for (int k = 0; k < q; ++k) M[a * n + b] += w[k] * I[k * n + a] * I[k * n + b];
+  // stiffness of each direction: the mass tables sum to one over the other
+  // two, the stiffness tables to zero
+  for (auto &A : Kd) A.assign(size_t(n) * n, 0);
+  ld kmax = 0;
+  for (int i = 0; i < ne; ++i)
+    for (int j = 0; j < ne; ++j) {
+      const ld v = K[size_t(i) * ne + j];
+      kmax = std::max(kmax, fabsl(v));
+      Kd[0][(i % n) * n + j % n] += v;
+      Kd[1][(i / n % n) * n + j / n % n] += v;
+      Kd[2][(i / n / n) * n + j / n / n] += v;
+    }
+  for (auto &A : Kd) symmetrise(A);
+  for (int k = 0; k < nqc; ++k)
+    for (int i = 0; i < ne; ++i) {
+      const ld v = I[(k % q) * n + i % n] * I[(k / q % q) * n + i / n % n] *
+                   I[(k / q / q) * n + i / n / n];
+      if (!(fabsl(Nq[size_t(k) * ne + i] - v) <= tol)) return false;
+    }
+  for (int i = 0; i < ne; ++i)
+    for (int j = 0; j < ne; ++j) {
+      const int ex = (i % n) * n + j % n, ey = (i / n % n) * n + j / n % n,
+                ez = (i / n / n) * n + j / n / n;
+      const ld v = Kd[0][ex] * M[ey] * M[ez] + M[ex] * Kd[1][ey] * M[ez] + M[ex] * M[ey] * Kd[2][ez];
+      if (!(fabsl(K[size_t(i) * ne + j] - v) <= tol * kmax)) return false;
+    }
+  // parity tables; the operator applies half the stiffness
+  const int NE = (n + 1) / 2, NO = n / 2, QE = (q + 1) / 2, QO = q / 2;
+  tab->clear();
+  tab32->assign(kTabs * 16 + QE, 0.f);
+  auto put = [&](const std::vector<ld> &A, int rows_e, int rows_o, ld f, int t32, int sums) {
+    const size_t at = tab->size();
+    for (int p = 0; p < 2; ++p)
+      for (int r = 0; r < rows_e; ++r)
+        for (int c = 0; c < NE; ++c) {
+          const ld v = A[r * n + c], m = A[r * n + n - 1 - c];
+          const bool in = p == 0 || (r < rows_o && c < NO);
+          tab->push_back(in ? (double)(f * (p == 0 ? v + m : v - m)) : 0.0);
+        }
+    // FP32: a rounding error of a table acts alike in every cell, so it shifts
+    // eigenvalues where the rounding of dense cell matrices averages out.  The
+    // even parts of I (sums = 1) and K (sums = 0) are therefore rounded to a
+    // common grid with their row sums kept exact: a constant is interpolated to
+    // itself and has no kinetic energy.  Smooth states at p = 6: shifts of
+    // 2.6e-6 Ha without, 1e-7 with it, 1e-7 in the dense FP32 product.
+    const double *e = tab->data() + at;
+    double big = 0;
+    for (int x = 0; x < rows_e * NE; ++x) big = std::max(big, std::fabs(e[x]));
+    for (int r = 0; r < rows_e; ++r) {
+      const double *er = e + r * NE;
+      std::vector<double> v(er, er + NE);
+      if (sums == 0) balance(er, NE, n & 1, big, 0.0, r, v.data());
+      if (sums == 1) {
+        const int fix = (int)(std::max_element(er, er + NE) - er);
+        balance(er, NE, n & 1, er[fix], 1.0, fix, v.data());
+      }
+      for (int c = 0; c < NE; ++c) {
+        float *d = tab32->data() + t32 * 16;
+        d[r * 4 + c] = (float)v[c];
+        d[16 + r * 4 + c] = (float)e[(rows_e + r) * NE + c];
+        if (t32 == kTabIe)
+          for (int p = 0; p < 2; ++p) d[32 + p * 16 + c * 4 + r] = d[p * 16 + r * 4 + c];
+      }
+    }
+  };
+  put(I, QE, QO, 1, kTabIe, 1);
+  put(M, NE, NO, 1, kTabMe, -1);
+  for (int d = 0; d < 3; ++d) put(Kd[d], NE, NO, 0.5L, kTabKx + 2 * d, 0);
+  for (int k = 0; k < QE; ++k) {
+    tab->push_back((double)(w[k] * (2 * k + 1 == q ? 0.25L : 0.5L)));
+    (*tab32)[kTabs * 16 + k] = (float)tab->back();
+  }
+  return true;
+}
+
+// ---------------------------------------------------------------------------
+// Potential weights in the order of the pencil threads: per cell
+// [group b * QE + a][mirror image s][z], s bit 0 mirroring x and bit 1 y, times
+// 1/8 and another 1/2 per direction whose index is the middle one (its mirror
+// image is the point itself and is counted twice; in z it enters once)
+// ---------------------------------------------------------------------------
+__global__ void tensor_potential_kernel(const double *v, int64_t total, int q, int qe, double *v64,
+                                        float *v32) {
+  const int per = qe * qe * 4 * q;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t c = e / per;
+    const int r = (int)(e % per);
+    const int z = r % q, s = r / q % 4, a = r / (4 * q) % qe, b = r / (4 * q * qe);
+    const int x = s & 1 ? q - 1 - a : a, y = s & 2 ? q - 1 - b : b;
+    double f = 0.125;
+    if (2 * a + 1 == q) f *= 0.5;
+    if (2 * b + 1 == q) f *= 0.5;
+    const double w = f * v[c * q * q * q + x + q * (y + q * z)];
+    v64[e] = w;
+    v32[e] = (float)w;
+  }
+}
+
+// Projector columns in the rows of the kernels' kinetic stage: (z, y, x) with
+// the even, then the odd values of y and x instead of the nodes
+__global__ void tensor_projector_kernel(const double *c, int64_t total, int n, int ne, int ne_pad,
+                                        double *c64, float *c32) {
+  const int nev = (n + 1) / 2;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    const int row = (int)(e / 16 % ne_pad);
+    double v = 0;
+    if (row < ne) {
+      const int kx = row % n, ky = row / n % n;
+      const int x = kx < nev ? kx : kx - nev, y = ky < nev ? ky : ky - nev;
+      const double *l = c + e - (int64_t)(row % (n * n)) * 16;  // the plane's first node
+      auto at = [&](int yy) {
+        const double p = l[(int64_t)(yy * n + x) * 16], m = l[(int64_t)(yy * n + n - 1 - x) * 16];
+        return kx < nev ? (2 * x + 1 == n ? p : 0.5 * (p + m)) : 0.5 * (p - m);
+      };
+      const double p = at(y), m = at(n - 1 - y);
+      v = ky < nev ? (2 * y + 1 == n ? p : 0.5 * (p + m)) : 0.5 * (p - m);
+    }
+    c64[e] = v;
+    c32[e] = (float)v;
+  }
+}
+
+hipError_t launch_tensor_projectors(const double *nlC, int64_t total, int n, int ne, int ne_pad,
+                                    double *c64, float *c32, hipStream_t s) {
+  const unsigned grid = (unsigned)std::min<int64_t>((total + 255) / 256, 1 << 16);
+  hipLaunchKernelGGL(tensor_projector_kernel, dim3(grid), dim3(256), 0, s, nlC, total, n, ne,
+                     ne_pad, c64, c32);
+  return hipGetLastError();
+}
+
+hipError_t launch_tensor_potential(const double *vJxW, int C, int n, int q, double *v64,
+                                   float *v32, hipStream_t s) {
+  (void)n;
+  const int qe = (q + 1) / 2;
+  const int64_t total = int64_t(C) * qe * qe * 4 * q;
+  const unsigned grid = (unsigned)std::min<int64_t>((total + 255) / 256, 1 << 16);
+  hipLaunchKernelGGL(tensor_potential_kernel, dim3(grid), dim3(256), 0, s, vJxW, total, q, qe, v64,
+                     v32);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Fused HX, tensor form
+// ---------------------------------------------------------------------------
+// One workgroup per (cell, TC columns).  A thread of the plane stages holds,
+// for one column, the even-x or odd-x half of one z plane (28 values at
+// n = 7), the parity uniform per wave so that all table entries are scalar
+// operands; a thread of the pencil stages holds the four z lines mirrored in x
+// and y.  The block goes through LDS between the stages:
+//   gather (scaled rows) -> planes: b = (K_x M_y + M_x K_y) x -> z lines: M_z b
+//   -> planes: u = I_x I_y x -> z lines: (I_z^T v I_z + w_x w_y K_z) u
+//   -> planes: I_x^T I_y^T, sum -> rows: scatter.
+// The nonlocal term C_e W (MFMA) joins M_z b.
+// K_z runs on the lines interpolated in x and y (weighted there), K_x and K_y on
+// nodal values: in FP32 the error is that of the dense product or below
+// (stiffness tables at quadrature points would double it).
+template <typename T, int N, int Q, int TC_, int VW>
+struct TensorShape : TensorTab<N, Q> {
+  static constexpr int TC = TC_, QE_ = (Q + 1) / 2;
+  static constexpr int G = 64 / TC;              // column groups of a wave
+  static constexpr int PW = (N + G - 1) / G;     // waves per x parity
+  static constexpr int NW = 2 * PW, NT = 64 * NW, GR = NT / TC;
+  static constexpr int ELEMS = (N * Q * Q > N * N * N ? N * Q * Q : N * N * N) * TC;
+  static constexpr int NE3 = N * N * N;
+  static constexpr int NRB = (NE3 + 15) / 16;
+  static constexpr int RBW = (NRB + NW - 1) / NW;
+  static constexpr int CBW = TC / 16;
+  // gather and scatter: a thread takes VW columns of whole x lines; lanes of a
+  // line, lines at once, lines per thread
+  static constexpr int NV = QE_ * QE_ * 4 * Q;   // weights of a cell
+  static constexpr int VT = (NV + NT - 1) / NT;
+  static constexpr int LR = TC / VW, LG = NT / LR, LT = (N * N + LG - 1) / LG;
+  // waves per SIMD the registers are limited for: two workgroups per CU at
+  // n = 7 (their LDS allows no more), else what fits without spills
+  static constexpr int WPE = sizeof(T) == 8 ? 2 : (N == 7 ? 4 : 3);
+};
+
+// FP64 tables are scalar operands
+typedef const __attribute__((address_space(4))) double *ctab;
+
+// (I_z^T diag(v) I_z + wk K_z) u on one line, in place
+template <typename T, int N, int Q>
+__device__ __forceinline__ void tensor_line(T (&u)[N], const T *v, T wk, ctab tab) {
+  using S = TensorTab<N, Q>;
+  constexpr int NE = S::NE, NO = S::NO, QE = S::QE, QO = S::QO;
+  T E[NE], O[NE], rE[NE], rO[NE];
+#pragma unroll
+  for (int i = 0; i < NO; ++i) {
+    E[i] = u[i] + u[N - 1 - i];
+    O[i] = u[i] - u[N - 1 - i];
+  }
+  if constexpr (N & 1) E[NO] = u[NO];
+#pragma unroll
+  for (int i = 0; i < NE; ++i) {
+    T t = tab[S::oKz + i * NE] * E[0];
+#pragma unroll
+    for (int j = 1; j < NE; ++j) t = fmadd(tab[S::oKz + i * NE + j], E[j], t);
+    rE[i] = wk * t;
+  }
+#pragma unroll
+  for (int i = 0; i < NO; ++i) {
+    T t = tab[S::oKz + (NE + i) * NE] * O[0];
+#pragma unroll
+    for (int j = 1; j < NO; ++j) t = fmadd(tab[S::oKz + (NE + i) * NE + j], O[j], t);
+    rO[i] = wk * t;
+  }
+#pragma unroll
+  for (int k = 0; k < QE; ++k) {
+    T e = tab[S::oI + k * NE] * E[0], o = T(0);
+#pragma unroll
+    for (int i = 1; i < NE; ++i) e = fmadd(tab[S::oI + k * NE + i], E[i], e);
+    if (k < QO) {
+      o = tab[S::oI + (QE + k) * NE] * O[0];
+#pragma unroll
+      for (int i = 1; i < NO; ++i) o = fmadd(tab[S::oI + (QE + k) * NE + i], O[i], o);
+      const T p = v[k] * (e + o), m = v[Q - 1 - k] * (e - o);
+      e = p + m;
+      o = p - m;
+    } else {
+      e = v[k] * e;
+    }
+#pragma unroll
+    for (int i = 0; i < NE; ++i) rE[i] = fmadd(tab[S::oI + k * NE + i], e, rE[i]);
+    if (k < QO) {
+#pragma unroll
+      for (int i = 0; i < NO; ++i) rO[i] = fmadd(tab[S::oI + (QE + k) * NE + i], o, rO[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NO; ++i) {
+    u[i] = rE[i] + rO[i];
+    u[N - 1 - i] = rE[i] - rO[i];
+  }
+  if constexpr (N & 1) u[NO] = rE[NO];
+}
+
+// Plane stages of x parity PX: the thread's values of plane k are NX x N nodal
+// ones, [x][y], y as even part (s = 0) and odd part (s = 1).
+template <typename T, int N, int Q, int TC, int PX>
+struct Planes {
+  using S = TensorTab<N, Q>;
+  static constexpr int NE = S::NE, NO = S::NO, QE = S::QE, QO = S::QO;
+  static constexpr int NX = PX ? NO : NE, QX = PX ? QO : QE;
+  typedef T Plane[2][NE][NE];  // [y parity][y][x]
+  typedef Plane Sums;
+  ctab tab;
+  __device__ __forceinline__ Planes(const double *t, const float *) : tab((ctab)t) {}
+  // entries of parity p
+  __device__ __forceinline__ double I(int p, int r, int c) const {
+    return tab[S::oI + (p * QE + r) * NE + c];
+  }
+  __device__ __forceinline__ double M(int p, int r, int c) const {
+    return tab[S::oM + (p * NE + r) * NE + c];
+  }
+  __device__ __forceinline__ double Kx(int r, int c) const {
+    return tab[S::oKx + (PX * NE + r) * NE + c];
+  }
+  __device__ __forceinline__ double Ky(int p, int r, int c) const {
+    return tab[S::oKy + (p * NE + r) * NE + c];
+  }
+
+  // x-parity values [z][y][x] (the plane's part of buf) -> parity values
+  static __device__ __forceinline__ void read(const T *b, Plane &x) {
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const T *c = b + ((PX ? NE : 0) + i) * TC;
+#pragma unroll
+      for (int j = 0; j < NO; ++j) {
+        const T p = c[j * N * TC], m = c[(N - 1 - j) * N * TC];
+        x[0][j][i] = p + m;
+        x[1][j][i] = p - m;
+      }
+      if constexpr (N & 1) x[0][NO][i] = c[NO * N * TC];
+    }
+  }
+
+  // b = (K_x M_y + M_x K_y) x -> nodal parity values [z][y][x] at b
+  __device__ __forceinline__ void kinetic(const Plane &x, bool act, T *b) const {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int ns = s ? NO : NE;
+#pragma unroll
+      for (int j = 0; j < ns; ++j) {
+        T m[NE], q[NE];
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+          m[i] = M(s, j, 0) * x[s][0][i];
+          q[i] = Ky(s, j, 0) * x[s][0][i];
+#pragma unroll
+          for (int jj = 1; jj < ns; ++jj) {
+            m[i] = fmadd(M(s, j, jj), x[s][jj][i], m[i]);
+            q[i] = fmadd(Ky(s, j, jj), x[s][jj][i], q[i]);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+          T r = Kx(i, 0) * m[0];
+#pragma unroll
+          for (int ii = 1; ii < NX; ++ii) r = fmadd(Kx(i, ii), m[ii], r);
+#pragma unroll
+          for (int ii = 0; ii < NX; ++ii) r = fmadd(M(PX, i, ii), q[ii], r);
+          if (act) b[((s ? NE + j : j) * N + (PX ? NE : 0) + i) * TC] = r;
+        }
+      }
+    }
+  }
+
+  static __device__ __forceinline__ void load(const T *b, Plane &o) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < (s ? NO : NE); ++j)
+#pragma unroll
+        for (int i = 0; i < NX; ++i)
+          o[s][j][i] = b[((s ? NE + j : j) * N + (PX ? NE : 0) + i) * TC];
+  }
+
+  // u = I_x I_y x -> quadrature parity values [z][y][x] at b
+  __device__ __forceinline__ void interpolate(const Plane &x, bool act, T *b) const {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int qs = s ? QO : QE, ns = s ? NO : NE;
+#pragma unroll
+      for (int j = 0; j < qs; ++j) {
+        T w[NE];
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+          w[i] = I(s, j, 0) * x[s][0][i];
+#pragma unroll
+          for (int jj = 1; jj < ns; ++jj) w[i] = fmadd(I(s, j, jj), x[s][jj][i], w[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < QX; ++i) {
+          T r = I(PX, i, 0) * w[0];
+#pragma unroll
+          for (int ii = 1; ii < NX; ++ii) r = fmadd(I(PX, i, ii), w[ii], r);
+          if (act) b[((s ? QE + j : j) * Q + (PX ? QE : 0) + i) * TC] = r;
+        }
+      }
+    }
+  }
+
+  // o += I_x^T I_y^T r
+  __device__ __forceinline__ void collect(const T *b, Plane &o) const {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int qs = s ? QO : QE, ns = s ? NO : NE;
+#pragma unroll
+      for (int j = 0; j < qs; ++j) {
+        T r[QE], w[NE];
+#pragma unroll
+        for (int i = 0; i < QX; ++i) r[i] = b[((s ? QE + j : j) * Q + (PX ? QE : 0) + i) * TC];
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+          w[i] = I(PX, 0, i) * r[0];
+#pragma unroll
+          for (int ii = 1; ii < QX; ++ii) w[i] = fmadd(I(PX, ii, i), r[ii], w[i]);
+        }
+#pragma unroll
+        for (int jj = 0; jj < ns; ++jj)
+#pragma unroll
+          for (int i = 0; i < NX; ++i)
+            o[s][jj][i] = fmadd(I(s, j, jj), w[i], o[s][jj][i]);
+      }
+    }
+  }
+
+  // x-parity values of the nodes, [z][y][x parity value] at b
+  static __device__ __forceinline__ void store(const Plane &o, bool act, T *b) {
+    if (!act) return;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      T *c = b + ((PX ? NE : 0) + i) * TC;
+#pragma unroll
+      for (int j = 0; j < NO; ++j) {
+        c[j * N * TC] = o[0][j][i] + o[1][j][i];
+        c[(N - 1 - j) * N * TC] = o[0][j][i] - o[1][j][i];
+      }
+      if constexpr (N & 1) c[NO * N * TC] = o[0][NO][i];
+    }
+  }
+};
+
+// z line stages
+template <typename T, int N, int Q>
+struct Lines {
+  using S = TensorTab<N, Q>;
+  static constexpr int NE = S::NE, NO = S::NO;
+  ctab tab;
+  __device__ __forceinline__ Lines(const double *t, const float *) : tab((ctab)t) {}
+  // M_z on one line of nodal values (stride st), in place
+  __device__ __forceinline__ void mass(T *b, int st) const {
+    T E[NE], O[NE];
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      const T p = b[i * st], m = b[(N - 1 - i) * st];
+      E[i] = p + m;
+      O[i] = p - m;
+    }
+    if constexpr (N & 1) E[NO] = b[NO * st];
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      T e = tab[S::oM + i * NE] * E[0];
+#pragma unroll
+      for (int j = 1; j < NE; ++j) e = fmadd(tab[S::oM + i * NE + j], E[j], e);
+      if (i < NO) {
+        T o = tab[S::oM + (NE + i) * NE] * O[0];
+#pragma unroll
+        for (int j = 1; j < NO; ++j) o = fmadd(tab[S::oM + (NE + i) * NE + j], O[j], o);
+        b[i * st] = e + o;
+        b[(N - 1 - i) * st] = e - o;
+      } else {
+        b[i * st] = e;
+      }
+    }
+  }
+  __device__ __forceinline__ T weight(int i) const { return tab[S::oW + i]; }
+  __device__ __forceinline__ void potential(T (&u)[N], const T *v, T wk) const {
+    tensor_line<T, N, Q>(u, v, wk, tab);
+  }
+};
+
+// ---------------------------------------------------------------------------
+// FP32 forms on v_mfma_f32_4x4x1: one instruction is 16 independent 4 x 4
+// outer products, lane l holding column l % 4 of block l / 4 and the four rows
+// of the result in four registers.  With the table entry A[l % 4][k] in the
+// first operand, four of them multiply each lane's own 4-vector by a 4 x 4
+// table: the parity blocks here, at twice the rate of 16 vector FMAs and beside
+// the vector pipe.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+}
+
+// c + A x over the first K entries of x (x(k): the k-th)
+template <int K, typename F>
+__device__ __forceinline__ f32x4 mat4(f32x4 a, F x, f32x4 c) {
+#pragma unroll
+  for (int k = 0; k < K; ++k) c = mfma4(a[k], x(k), c);
+  return c;
+}
+
+template <int N, int Q, int TC, int PX>
+struct Planes<float, N, Q, TC, PX> {
+  using S = TensorTab<N, Q>;
+  static constexpr int NE = S::NE, NO = S::NO, QE = S::QE, QO = S::QO;
+  static constexpr int NX = PX ? NO : NE, QX = PX ? QO : QE;
+  typedef float Plane[2][NE][NE];  // [y parity][y][x]
+  typedef f32x4 Sums[2][NE];       // [y parity][x] over y
+  const f32x4 *tab;                // this lane's rows of the operand tables
+  __device__ __forceinline__ Planes(const float *, const float *t)
+      : tab(reinterpret_cast<const f32x4 *>(t) + (threadIdx.x & 3)) {}
+  __device__ __forceinline__ f32x4 operand(int k) const { return tab[4 * k]; }
+
+  static __device__ __forceinline__ void read(const float *b, Plane &x) {
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const float *c = b + ((PX ? NE : 0) + i) * TC;
+#pragma unroll
+      for (int j = 0; j < NO; ++j) {
+        const float p = c[j * N * TC], m = c[(N - 1 - j) * N * TC];
+        x[0][j][i] = p + m;
+        x[1][j][i] = p - m;
+      }
+      if constexpr (N & 1) x[0][NO][i] = c[NO * N * TC];
+    }
+  }
+
+  template <int s>
+  __device__ __forceinline__ void kinetic_s(const Plane &x, bool act, float *b) const {
+    constexpr int ns = s ? NO : NE;
+    const f32x4 z = {0, 0, 0, 0};
+    const f32x4 my = operand(kTabMe + s), ky = operand(kTabKy + s);
+    const f32x4 mx = operand(kTabMe + PX), kx = operand(kTabKx + PX);
+    f32x4 m[NE], q[NE];
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      auto l = [&](int j) { return x[s][j][i]; };
+      m[i] = mat4<ns>(my, l, z);
+      q[i] = mat4<ns>(ky, l, z);
+    }
+#pragma unroll
+    for (int j = 0; j < ns; ++j) {
+      const f32x4 r = mat4<NX>(mx, [&](int i) { return q[i][j]; },
+                               mat4<NX>(kx, [&](int i) { return m[i][j]; }, z));
+#pragma unroll
+      for (int i = 0; i < NX; ++i)
+        if (act) b[((s ? NE + j : j) * N + (PX ? NE : 0) + i) * TC] = r[i];
+    }
+  }
+  __device__ __forceinline__ void kinetic(const Plane &x, bool act, float *b) const {
+    kinetic_s<0>(x, act, b);
+    kinetic_s<1>(x, act, b);
+  }
+
+  static __device__ __forceinline__ void load(const float *b, Sums &o) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < NX; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o[s][i][j] = j < (s ? NO : NE) ? b[((s ? NE + j : j) * N + (PX ? NE : 0) + i) * TC] : 0.f;
+  }
+
+  template <int s>
+  __device__ __forceinline__ void interpolate_s(const Plane &x, bool act, float *b) const {
+    constexpr int ns = s ? NO : NE, qs = s ? QO : QE;
+    const f32x4 z = {0, 0, 0, 0};
+    const f32x4 iy = operand(kTabIe + s), ix = operand(kTabIe + PX);
+    f32x4 w[NE];
+#pragma unroll
+    for (int i = 0; i < NX; ++i) w[i] = mat4<ns>(iy, [&](int j) { return x[s][j][i]; }, z);
+#pragma unroll
+    for (int j = 0; j < qs; ++j) {
+      const f32x4 r = mat4<NX>(ix, [&](int i) { return w[i][j]; }, z);
+#pragma unroll
+      for (int i = 0; i < QX; ++i)
+        if (act) b[((s ? QE + j : j) * Q + (PX ? QE : 0) + i) * TC] = r[i];
+    }
+  }
+  __device__ __forceinline__ void interpolate(const Plane &x, bool act, float *b) const {
+    interpolate_s<0>(x, act, b);
+    interpolate_s<1>(x, act, b);
+  }
+
+  template <int s>
+  __device__ __forceinline__ void collect_s(const float *b, Sums &o) const {
+    constexpr int qs = s ? QO : QE;
+    const f32x4 z = {0, 0, 0, 0};
+    const f32x4 iy = operand(kTabIeT + s), ix = operand(kTabIeT + PX);
+    f32x4 w[QE];
+#pragma unroll
+    for (int j = 0; j < qs; ++j)
+      w[j] = mat4<QX>(ix, [&](int i) { return b[((s ? QE + j : j) * Q + (PX ? QE : 0) + i) * TC]; },
+                      z);
+#pragma unroll
+    for (int i = 0; i < NX; ++i)
+      o[s][i] = mat4<qs>(iy, [&](int j) { return w[j][i]; }, o[s][i]);
+  }
+  __device__ __forceinline__ void collect(const float *b, Sums &o) const {
+    collect_s<0>(b, o);
+    collect_s<1>(b, o);
+  }
+
+  static __device__ __forceinline__ void store(const Sums &o, bool act, float *b) {
+    if (!act) return;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      float *c = b + ((PX ? NE : 0) + i) * TC;
+#pragma unroll
+      for (int j = 0; j < NO; ++j) {
+        c[j * N * TC] = o[0][i][j] + o[1][i][j];
+        c[(N - 1 - j) * N * TC] = o[0][i][j] - o[1][i][j];
+      }
+      if constexpr (N & 1) c[NO * N * TC] = o[0][i][NO];
+    }
+  }
+};
+
+template <int N, int Q>
+struct Lines<float, N, Q> {
+  using S = TensorTab<N, Q>;
+  static constexpr int NE = S::NE, NO = S::NO, QE = S::QE, QO = S::QO;
+  const f32x4 *tab;
+  const float *weights;
+  __device__ __forceinline__ Lines(const float *, const float *t)
+      : tab(reinterpret_cast<const f32x4 *>(t) + (threadIdx.x & 3)), weights(t + kTabs * 16) {}
+  __device__ __forceinline__ float weight(int i) const { return weights[i]; }
+  __device__ __forceinline__ f32x4 operand(int k) const { return tab[4 * k]; }
+
+  __device__ __forceinline__ void mass(float *b, int st) const {
+    const f32x4 z = {0, 0, 0, 0};
+    float E[NE], O[NE];
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      const float p = b[i * st], m = b[(N - 1 - i) * st];
+      E[i] = p + m;
+      O[i] = p - m;
+    }
+    if constexpr (N & 1) E[NO] = b[NO * st];
+    const f32x4 e = mat4<NE>(operand(kTabMe), [&](int k) { return E[k]; }, z);
+    const f32x4 o = mat4<NO>(operand(kTabMo), [&](int k) { return O[k]; }, z);
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      b[i * st] = e[i] + o[i];
+      b[(N - 1 - i) * st] = e[i] - o[i];
+    }
+    if constexpr (N & 1) b[NO * st] = e[NO];
+  }
+
+  __device__ __forceinline__ void potential(float (&u)[N], const float *v, float wk) const {
+    const f32x4 z = {0, 0, 0, 0};
+    float E[NE], O[NE];
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      E[i] = u[i] + u[N - 1 - i];
+      O[i] = u[i] - u[N - 1 - i];
+    }
+    if constexpr (N & 1) E[NO] = u[NO];
+    auto Ek = [&](int k) { return E[k]; };
+    auto Ok = [&](int k) { return O[k]; };
+    f32x4 rE = mat4<NE>(operand(kTabKz), Ek, z) * wk;
+    f32x4 rO = mat4<NO>(operand(kTabKzo), Ok, z) * wk;
+    f32x4 e = mat4<NE>(operand(kTabIe), Ek, z);
+    f32x4 o = mat4<NO>(operand(kTabIo), Ok, z);
+#pragma unroll
+    for (int k = 0; k < QE; ++k) {
+      if (k < QO) {
+        const float p = v[k] * (e[k] + o[k]), m = v[Q - 1 - k] * (e[k] - o[k]);
+        e[k] = p + m;
+        o[k] = p - m;
+      } else {
+        e[k] = v[k] * e[k];
+      }
+    }
+    rE = mat4<QE>(operand(kTabIeT), [&](int k) { return e[k]; }, rE);
+    rO = mat4<QO>(operand(kTabIoT), [&](int k) { return o[k]; }, rO);
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      u[i] = rE[i] + rO[i];
+      u[N - 1 - i] = rE[i] - rO[i];
+    }
+    if constexpr (N & 1) u[NO] = rE[NO];
+  }
+};
+
+// VW neighbouring columns of a row
+template <typename T, int VW>
+using tvec = T __attribute__((ext_vector_type(VW)));
+template <typename T, int VW>
+__device__ __forceinline__ tvec<T, VW> vload(const T *p) {
+  return *(const __attribute__((address_space(1))) tvec<T, VW> *)p;
+}
+template <typename T, int VW>
+__device__ __forceinline__ void vstore(T *p, tvec<T, VW> v) {
+  *(__attribute__((address_space(1))) tvec<T, VW> *)p = v;
+}
+// p + row g of a block whose rows are ldb bytes apart
+template <typename T>
+__device__ __forceinline__ T *row_ptr(T *p, uint32_t g, uint32_t ldb) {
+  return (T *)((char *)p + (uint64_t)g * ldb);
+}
+template <typename T, int N, int Q, int TC, int VW>
+__global__ __launch_bounds__((TensorShape<T, N, Q, TC, VW>::NT))
+__attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_tensor_kernel(
+    HxLaunch<T> a, const T *vq, const T *tabp) {
+  using S = TensorShape<T, N, Q, TC, VW>;
+  using vec = tvec<T, VW>;
+  const uint32_t lds_b = (uint32_t)(a.ld_src * sizeof(T)), ldd_b = (uint32_t)(a.ld_dst * sizeof(T)),
+                 ldr_b = (uint32_t)(a.ldR * sizeof(T));
+  constexpr int NE = S::NE, NO = S::NO, QE = S::QE, QO = S::QO, NE3 = S::NE3;
+  constexpr int GR = S::GR, NW = S::NW, PW = S::PW;
+  using v4 = typename V4<T>::t;
+  using P0 = Planes<T, N, Q, TC, 0>;
+  using P1 = Planes<T, N, Q, TC, 1>;
+  __shared__ __align__(16) T buf[S::ELEMS];
+  // per node: DOF and first-touch bit, input scale / 8, output scale; the
+  // weights at the cell's quadrature points take the input scales' place
+  __shared__ uint32_t smap[NE3];
+  __shared__ T sout[NE3];
+  __shared__ __align__(16) T svq[S::NV > NE3 ? S::NV : NE3];
+  T *const ssin = svq;
+  // the 4 x 4 operand tables of the FP32 form
+  __shared__ __align__(16) float tabs[sizeof(T) == 4 ? kTabs * 16 + QE : 4];
+
+  // consecutive items (the column tiles of a cell first) on one XCD
+  const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+  if (item >= a.ncells * a.ntiles) return;
+  const int cell = a.cells[item / a.ntiles];
+  const int v0 = (item % a.ntiles) * TC;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int col = t % TC, grp = t / TC;
+  // projector slots of the cell; the projectors of its first 16
+  const int s0 = a.nl_off ? a.nl_off[cell] : 0;
+  const int ns = a.nl_off ? a.nl_off[cell + 1] - s0 : 0;
+  int slot0[4];
+  if (ns > 0) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) slot0[r] = gload(a.slot_proj, s0 + 4 * (lane >> 4) + r);
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (t < kTabs * 16 + QE) tabs[t] = tabp[t];
+  }
+
+  // ---- gather: x lines of the cell's nodes, scaled, as x-parity values into
+  // buf[z][y][even, odd][col]
+  const int rl = t % S::LR, lg = t / S::LR;     // lane of a line, first line
+  const int vr = v0 + rl * VW;
+  const bool vin = vr < a.B;                    // VW > 1: B is a multiple of it
+  const int vc = vin ? vr : a.B - VW;
+  // W rows of 16 slots (four per lane), from the slots' projectors
+  auto projectors = [&](const int (&p)[4], T(&w)[4][S::CBW]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int cb = 0; cb < S::CBW; ++cb) {
+        const int v = v0 + cb * 16 + (lane & 15);
+        w[r][cb] = gload(a.W, (int64_t)(p[r] < 0 ? 0 : p[r]) * a.ldW + (v < a.B ? v : a.B - 1));
+      }
+  };
+  // projector columns of 16 slots: this wave's row blocks, four slots a lane
+  auto columns = [&](int kt, T(&c)[S::RBW][4]) {
+    const T *cm = a.nl_C + ((int64_t)s0 + kt) * a.ne_pad;
+#pragma unroll
+    for (int j = 0; j < S::RBW; ++j) {
+      const int rb = wave + NW * j < S::NRB ? wave + NW * j : 0;
+      const T *p = cm + (rb * 16 + (lane & 15)) * 16 + 4 * (lane >> 4);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) c[j][r] = gload(p, r);
+    }
+  };
+  T c0[S::RBW][4], w0[4][S::CBW];
+
+  // the cell's map and scales go through LDS: read by every lane of a line
+  // they cost more than the rows themselves (28 loads per thread at n = 7)
+  T vreg[S::VT];
+  {
+    constexpr int MT = (NE3 + S::NT - 1) / S::NT;
+    uint32_t w[MT];
+#pragma unroll
+    for (int e = 0; e < MT; ++e) {
+      const int i = t + e * S::NT;
+      w[e] = gload(a.map, (int64_t)cell * NE3 + (i < NE3 ? i : 0));
+      if (i < NE3) smap[i] = w[e];
+    }
+    __syncthreads();
+    vec x[S::LT][N];
+#pragma unroll
+    for (int l = 0; l < S::LT; ++l) {
+      const int line = lg + l * S::LG, lc = line < N * N ? line : N * N - 1;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        x[l][i] = vload<T, VW>(row_ptr(a.src + vc, smap[lc * N + i] & 0x7fffffffu, lds_b));
+    }
+    T si[MT], so[MT];
+#pragma unroll
+    for (int e = 0; e < MT; ++e) {
+      si[e] = a.s_in ? gload(a.s_in, w[e] & 0x7fffffffu) : T(1);
+      so[e] = a.s_out == a.s_in ? si[e] : (a.s_out ? gload(a.s_out, w[e] & 0x7fffffffu) : T(1));
+    }
+#pragma unroll
+    for (int e = 0; e < S::VT; ++e) {
+      const int i = t + e * S::NT;
+      vreg[e] = gload(vq, (int64_t)cell * S::NV + (i < S::NV ? i : 0));
+    }
+    if (ns > 0) {
+      projectors(slot0, w0);
+      columns(0, c0);
+    }
+#pragma unroll
+    for (int e = 0; e < MT; ++e) {
+      const int i = t + e * S::NT;
+      if (i < NE3) {
+        ssin[i] = T(0.125) * si[e];
+        sout[i] = so[e];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < S::LT; ++l) {
+      const int line = lg + l * S::LG;
+      if (line >= N * N) continue;
+      T *b = buf + line * N * TC + rl * VW;
+#pragma unroll
+      for (int i = 0; i < N; ++i) x[l][i] *= ssin[line * N + i];
+#pragma unroll
+      for (int i = 0; i < NO; ++i) {
+        *reinterpret_cast<vec *>(b + i * TC) = x[l][i] + x[l][N - 1 - i];
+        *reinterpret_cast<vec *>(b + (NE + i) * TC) = x[l][i] - x[l][N - 1 - i];
+      }
+      if constexpr (N & 1) *reinterpret_cast<vec *>(b + NO * TC) = x[l][NO];
+    }
+  }
+  __syncthreads();
+
+  // ---- plane stages: this wave's x parity and the thread's plane
+  const bool px = wave >= PW;
+  const int kk = (wave - (px ? PW : 0)) * S::G + lane / TC;
+  const bool act = kk < N;
+  const int k = act ? kk : N - 1;
+  T *const bn = buf + k * (N * N) * TC + col;   // the plane's nodal values
+  T *const bq = buf + k * (Q * Q) * TC + col;   // its quadrature values
+  const P0 p0(tabp, tabs);
+  const P1 p1(tabp, tabs);
+  const Lines<T, N, Q> lines(tabp, tabs);
+  typename P0::Plane x;
+  typename P0::Sums o;
+  if (px) P1::read(bn, x); else P0::read(bn, x);
+#pragma unroll
+  for (int e = 0; e < S::VT; ++e) {
+    const int i = t + e * S::NT;
+    if (i < S::NV) svq[i] = vreg[e];
+  }
+  __syncthreads();
+  if (px) p1.kinetic(x, act, bn); else p0.kinetic(x, act, bn);
+  __syncthreads();
+  // the nonlocal term C_e W runs on the matrix pipe beside the mass lines and
+  // joins the in-plane kinetic part in its rows
+  v4 acc[S::RBW][S::CBW];
+  if (ns > 0) {
+#pragma unroll
+    for (int j = 0; j < S::RBW; ++j)
+#pragma unroll
+      for (int cb = 0; cb < S::CBW; ++cb) acc[j][cb] = v4{T(0), T(0), T(0), T(0)};
+    for (int kt = 0; kt < ns; kt += 16) {
+      if (kt > 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) slot0[r] = gload(a.slot_proj, s0 + kt + 4 * (lane >> 4) + r);
+        projectors(slot0, w0);
+        columns(kt, c0);
+      }
+      // a slot without projector (padding) has a zero column; its row of W is
+      // another slot's, which need not be finite
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int cb = 0; cb < S::CBW; ++cb) w0[r][cb] = slot0[r] < 0 ? T(0) : w0[r][cb];
+#pragma unroll
+      for (int j = 0; j < S::RBW; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int cb = 0; cb < S::CBW; ++cb) acc[j][cb] = mfma16(c0[j][r], w0[r][cb], acc[j][cb]);
+    }
+  }
+  for (int id = grp; id < N * N; id += GR) lines.mass(buf + id * TC + col, N * N * TC);
+  __syncthreads();
+  if (ns > 0) {
+#pragma unroll
+    for (int j = 0; j < S::RBW; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = (wave + NW * j) * 16 + acc_row<T>(lane, r);
+        if (row < NE3)
+#pragma unroll
+          for (int cb = 0; cb < S::CBW; ++cb)
+            buf[row * TC + cb * 16 + (lane & 15)] += acc[j][cb][r];
+      }
+    __syncthreads();
+  }
+  if (px) P1::load(bn, o); else P0::load(bn, o);
+  __syncthreads();
+  if (px) p1.interpolate(x, act, bq); else p0.interpolate(x, act, bq);
+  __syncthreads();
+
+  // ---- z lines of u: four mirrored lines per thread
+  for (int id = grp; id < QE * QE; id += GR) {
+    const int ix = id % QE, iy = id / QE;
+    // the odd value of a middle index does not exist (and is zero)
+    const bool hx = ix < QO, hy = iy < QO;
+    T *b00 = buf + (iy * Q + ix) * TC + col;
+    T *b01 = b00 + (hx ? QE : 0) * TC, *b10 = b00 + (hy ? QE : 0) * Q * TC,
+      *b11 = b10 + (hx ? QE : 0) * TC;
+    T u[4][N];
+#pragma unroll
+    for (int z = 0; z < N; ++z) {
+      const int f = z * Q * Q * TC;
+      const T ee = b00[f];
+      const T oe = (Q & 1) && !hx ? T(0) : b01[f];
+      const T eo = (Q & 1) && !hy ? T(0) : b10[f];
+      const T oo = (Q & 1) && !(hx && hy) ? T(0) : b11[f];
+      const T s0 = ee + oe, d0 = ee - oe, s1 = eo + oo, d1 = eo - oo;
+      u[0][z] = s0 + s1;
+      u[1][z] = d0 + d1;
+      u[2][z] = s0 - s1;
+      u[3][z] = d0 - d1;
+    }
+    const T wk = lines.weight(ix) * lines.weight(iy);
+    const T *v = svq + id * (4 * Q);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      T vv[Q];
+#pragma unroll
+      for (int z = 0; z < Q; ++z) vv[z] = v[s * Q + z];
+      lines.potential(u[s], vv, wk);
+    }
+#pragma unroll
+    for (int z = 0; z < N; ++z) {
+      const int f = z * Q * Q * TC;
+      const T s0 = u[0][z] + u[1][z], d0 = u[0][z] - u[1][z], s1 = u[2][z] + u[3][z],
+              d1 = u[2][z] - u[3][z];
+      b00[f] = s0 + s1;
+      if (!(Q & 1) || hx) b01[f] = d0 + d1;
+      if (!(Q & 1) || hy) b10[f] = s0 - s1;
+      if (!(Q & 1) || (hx && hy)) b11[f] = d0 - d1;
+    }
+  }
+
+  // ---- the destination's rows and the first 16 projector rows: loaded here so
+  // that they arrive while the last plane stages run
+  vec dv[S::LT][N];
+#pragma unroll
+  for (int l = 0; l < S::LT; ++l) {
+    const int line = lg + l * S::LG, lc = line < N * N ? line : N * N - 1;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      dv[l][i] = vload<T, VW>(row_ptr(a.dst + vc, smap[lc * N + i] & 0x7fffffffu, ldd_b));
+  }
+  __syncthreads();
+  if (px) p1.collect(bq, o); else p0.collect(bq, o);
+  __syncthreads();
+  if (px) P1::store(o, act, bn); else P0::store(o, act, bn);
+  // what the combine adds on first touch: gamma times the source's row, and in
+  // the defect form rcoef times the row of R.  Other rows read the block's first
+  // row: one line for all of them
+  const bool any_src = a.gamma != T(0);
+  T gamma = a.gamma;
+  vec sv[S::LT][N];
+#pragma unroll
+  for (int l = 0; l < S::LT; ++l) {
+    const int line = lg + l * S::LG, lc = line < N * N ? line : N * N - 1;
+    if (any_src) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const uint32_t w = smap[lc * N + i];
+        sv[l][i] = vload<T, VW>(row_ptr(a.src + vc, w >> 31 ? w & 0x7fffffffu : 0, lds_b));
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) sv[l][i] = T(0);
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (a.R) {
+      const vec rc = vload<T, VW>(a.rcoef + vc);
+#pragma unroll
+      for (int l = 0; l < S::LT; ++l) {
+        const int line = lg + l * S::LG, lc = line < N * N ? line : N * N - 1;
+        vec rv[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const uint32_t w = smap[lc * N + i];
+          rv[i] = vload<T, VW>(row_ptr(a.R + vc, w >> 31 ? w & 0x7fffffffu : 0, ldr_b));
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+          for (int e = 0; e < VW; ++e)
+            sv[l][i][e] = fmadd(rc[e], rv[i][e], gamma * sv[l][i][e]);
+      }
+      gamma = T(1);
+    }
+  }
+
+  __syncthreads();
+
+  // ---- scatter (the combine of hx_scatter)
+#pragma unroll
+  for (int l = 0; l < S::LT; ++l) {
+    const int line = lg + l * S::LG;
+    if (line >= N * N) continue;
+    const T *b = buf + line * N * TC + rl * VW;
+    vec y[N];
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      const vec e = *reinterpret_cast<const vec *>(b + i * TC),
+                f = *reinterpret_cast<const vec *>(b + (NE + i) * TC);
+      y[i] = e + f;
+      y[N - 1 - i] = e - f;
+    }
+    if constexpr (N & 1) y[NO] = *reinterpret_cast<const vec *>(b + NO * TC);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const uint32_t w = smap[line * N + i], g = w & 0x7fffffffu;
+      const bool first = (w >> 31) != 0;
+      const T so = sout[line * N + i];
+      // a zero output scale marks a constrained row (hanging node): it takes
+      // the plain sums, nothing else on first touch
+      const bool cons = so == T(0);
+      const T sa = a.alpha * (cons ? T(1) : so);
+      const T kf = a.beta_mode == 2 ? a.beta * so : a.beta;
+      vec base;
+#pragma unroll
+      for (int e = 0; e < VW; ++e) {
+        const T d = dv[l][i][e];
+        T c = fmadd(gamma, sv[l][i][e], a.beta_mode == 1 ? T(0) : kf * d);
+        c = first ? (cons ? T(0) : c) : d;
+        base[e] = fmadd(sa, y[i][e], c);
+      }
+      if (vin) vstore<T, VW>(row_ptr(a.dst + vc, g, ldd_b), base);
+    }
+  }
+}
+
+template <typename T, int N, int Q, int TC, int VW>
+static hipError_t hx_tensor_go(HxLaunch<T> a, const T *vq, const T *tab, hipStream_t s) {
+  a.ntiles = (a.B + TC - 1) / TC;
+  const int items = a.ncells * a.ntiles;
+  if (items == 0) return hipSuccess;
+  a.per_xcd = (items + 7) / 8;
+  hipLaunchKernelGGL((hx_tensor_kernel<T, N, Q, TC, VW>), dim3(8 * a.per_xcd),
+                     dim3(TensorShape<T, N, Q, TC, VW>::NT), 0, s, a, vq, tab);
+  return hipGetLastError();
+}
+
+// 16 bytes per lane (FP32: four columns, FP64: two) need whole, aligned groups
+// of columns in every block; FP32 falls back to pairs, both to single columns.
+template <typename T, int N, int Q, int TC>
+static hipError_t hx_tensor_vec(const HxLaunch<T> &a, const T *vq, const T *tab,
+                                hipStream_t s) {
+  auto whole = [&](int w) {
+    auto ok = [w](const T *p, int64_t ld) {
+      return reinterpret_cast<uintptr_t>(p) % (w * sizeof(T)) == 0 && ld % w == 0;
+    };
+    return a.B % w == 0 && ok(a.src, a.ld_src) && ok(a.dst, a.ld_dst) && ok(a.R, a.ldR) &&
+           ok(a.rcoef, 0);
+  };
+  if constexpr (sizeof(T) == 4)
+    if (whole(4)) return hx_tensor_go<T, N, Q, TC, 4>(a, vq, tab, s);
+  return whole(2) ? hx_tensor_go<T, N, Q, TC, 2>(a, vq, tab, s)
+                  : hx_tensor_go<T, N, Q, TC, 1>(a, vq, tab, s);
+}
+
+// Where the tensor form is taken (cells: of the largest colour; one MI355X, ms per
+// apply, tensor / best tile variant or, for one column, the matrix-vector kernel):
+//   n = 7: 4096 cells x 1024 columns 5.8 / 11.0 FP32, 1728 x 1024 5.2 / 9.9 FP64,
+//          1728 x 16 0.27 / 0.86, x 1 0.26 / 0.48
+//   n = 6: 1728 cells x 256 columns 1.06 / 1.50 FP64, 0.58 / 0.80 FP32, x 1 0.24 / 0.29
+//   n = 5: the dense product is only 1.7 times the operations, on the matrix
+//          pipe; the tensor form has fewer bytes in flight behind its barriers
+//          and wins while a colour launch does not fill the chip: 512 cells x 64
+//          columns 0.15 / 0.19 FP64, 0.11 / 0.13 FP32, x 200 0.25 / 0.22 and 0.14 /
+//          0.21, 1728 x 256 0.77 / 0.62 and 0.44 / 0.38, 512 x 1 0.14 / 0.12
+bool tensor_wins(int n, bool fp64, int cells, int B) {
+  if (n > 5) return true;
+  const int64_t items = int64_t(cells) * ((B + 31) / 32);
+  return B > 1 && items <= (fp64 ? 320 : 1024);
+}
+
+template <typename T>
+hipError_t launch_hx_tensor(const HxLaunch<T> &a, const T *vq, const T *tab, int n, int q,
+                            hipStream_t s) {
+  constexpr int W7 = sizeof(T) == 8 ? 16 : 32;
+  if (n == 7 && q == 8) return hx_tensor_vec<T, 7, 8, W7>(a, vq, tab, s);
+  if (n == 6 && q == 6) return hx_tensor_vec<T, 6, 6, 32>(a, vq, tab, s);
+  if (n == 5 && q == 5) return hx_tensor_vec<T, 5, 5, 32>(a, vq, tab, s);
+  return hipErrorInvalidValue;
+}
+template hipError_t launch_hx_tensor<double>(const HxLaunch<double> &, const double *,
+                                             const double *, int, int, hipStream_t);
+template hipError_t launch_hx_tensor<float>(const HxLaunch<float> &, const float *, const float *,
+                                            int, int, hipStream_t);
+
+}  // namespace chfsi

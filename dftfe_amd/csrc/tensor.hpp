@@ -1,0 +1,44 @@
+// Tensor-product form of the cell operators: cells whose shape values and
+// stiffness are products of one-dimensional tables (GLL Lagrange basis, Gauss
+// quadrature, Cartesian cells) are applied direction by direction instead of
+// through the dense n_e x n_e cell matrix.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <vector>
+
+#include "kernels.hpp"
+
+namespace chfsi {
+
+// (nodes per direction, Gauss points per direction) with an instantiation
+bool tensor_shape(int ne, int nqc, int *n, int *q);
+
+// Whether the tensor form is the faster one on B columns, from the cells of the
+// largest colour
+bool tensor_wins(int n, bool fp64, int cells, int B);
+
+// Host check of an operator's shape values (nqc x ne) and stiffness (ne x ne):
+// true when every entry is the product of one-dimensional, centro-symmetric
+// tables (Gauss quadrature) to 1e-13 of the largest one.  Fills the kernels'
+// tables, FP64 and FP32.
+bool tensor_tables(const double *Nq, const double *K, int ne, int nqc, std::vector<double> *tab,
+                   std::vector<float> *tab32);
+
+// Weights vJxW (C x nqc) in the kernels' order (scaled by exact powers of two)
+hipError_t launch_tensor_potential(const double *vJxW, int C, int n, int q, double *v64,
+                                   float *v32, hipStream_t s);
+
+// Projector columns (layout of nl_C) in the x-parity rows of the kernels
+hipError_t launch_tensor_projectors(const double *nlC, int64_t total, int n, int ne, int ne_pad,
+                                    double *c64, float *c32, hipStream_t s);
+
+// One fused HX launch over a colour class (as launch_hx) on the tensor form;
+// a.nl_C: the columns of launch_tensor_projectors
+template <typename T>
+hipError_t launch_hx_tensor(const HxLaunch<T> &a, const T *vq, const T *tab, int n, int q,
+                            hipStream_t s);
+
+}  // namespace chfsi

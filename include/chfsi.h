@@ -264,8 +264,10 @@ chfsi_status chfsi_operator_get_cell_matrices(chfsi_operator *op, double *H_dev,
 
 /* Tile-shape selection of the fused HX kernel (no reference counterpart: the
  * reference calls hipBLAS gemmStridedBatched).  chfsi_operator_autotune times
- * every tile variant of both precisions on a B-column block, keeps the fastest,
- * then times the projection-kernel variants with it and keeps the fastest.
+ * every tile variant of both precisions on a B-column block, keeps the fastest
+ * (until a variant is set, and after autotuning where it is faster, operators
+ * whose cells are products of one-dimensional tables apply an LDA potential
+ * direction by direction instead of through the cell matrices), then times the projection-kernel variants with it and keeps the fastest.
  * times_ms (48 entries) [0..15]: FP64 tile variants, [16..23]: FP64 projection
  * variants, [24..39]: FP32 tile variants, [40..47]: FP32 projection variants
  * (ms per HX; -1 where a variant does not exist).  Projection variants 4
