@@ -1070,8 +1070,13 @@ chfsi_status quad_product(chfsi_operator *op, const T *a, int64_t lda, const T *
                                             op->d_c_vals, op->nc, sc, bw, ldb, B, st));
     if (scaled) s_in = op->d_s_gather64;
   }
-  CHFSI_HIP(launch_quad_product(op->d_map, op->C, op->ne, op->nq, op->d_Nq, jxw, a, lda, b, ldb,
-                                B, s_in, w, wscale, g, accumulate, st, wshift));
+  constexpr int64_t kLd = int64_t(1) << 29;  // row offsets are 32-bit bytes
+  if (op->tn && lda < kLd && ldb < kLd)
+    CHFSI_HIP(launch_quad_tensor<T>(op->d_map, op->C, op->tn, op->tq, jxw, a, lda, b, ldb, B, s_in,
+                                    w, wshift, wscale, g, accumulate, op->d_ttab64, st));
+  else
+    CHFSI_HIP(launch_quad_product(op->d_map, op->C, op->ne, op->nq, op->d_Nq, jxw, a, lda, b, ldb,
+                                  B, s_in, w, wscale, g, accumulate, st, wshift));
   if (op->general_constraints) {
     CHFSI_HIP(launch_zero_rows_t<T>(op->d_c_rows, op->nc, aw, lda, B, st));
     if (bw != aw) CHFSI_HIP(launch_zero_rows_t<T>(op->d_c_rows, op->nc, bw, ldb, B, st));

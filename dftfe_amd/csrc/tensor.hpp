@@ -41,4 +41,11 @@ template <typename T>
 hipError_t launch_hx_tensor(const HxLaunch<T> &a, const T *vq, const T *tab, int n, int q,
                             hipStream_t s);
 
+// launch_quad_product on the tensor form (tab: the FP64 tables)
+template <typename TIn>
+hipError_t launch_quad_tensor(const uint32_t *map, int C, int n, int q, const double *JxW,
+                              const TIn *a, int64_t lda, const TIn *b, int64_t ldb, int B,
+                              const double *s_in, const double *w, int wshift, double wscale,
+                              double *g, int accumulate, const double *tab, hipStream_t s);
+
 }  // namespace chfsi

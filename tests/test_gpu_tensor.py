@@ -122,3 +122,23 @@ def test_potential_changes(case):
     op.set_cell_matrices(H)
     assert torch.equal(op.apply(X), gga)
     op.set_potential(prob.vJxW)
+
+
+@pytest.mark.parametrize("B,ld,off", [(1, 1, 0), (2, 2, 0), (7, 9, 1), (16, 16, 0), (17, 20, 2),
+                                      (32, 32, 0), (50, 52, 0)])
+def test_quadrature_products(case, B, ld, off):
+    """Density (one block), V-adjoint (two blocks) and accumulation into them."""
+    prob, ref, op = case
+    rng = np.random.default_rng(B + 7 * ld)
+    full = rng.uniform(-1, 1, (2, prob.M, ld + off))
+    full[:, prob.constrained] = 0.0
+    a, b = (torch.tensor(f, device="cuda")[:, off:off + B] for f in full)
+    w = rng.uniform(0, 2, B)
+    rho = op.density(a, torch.tensor(w))
+    want = O.density_at_quadrature(prob, a.cpu().numpy(), w, spin_factor=1.0)
+    assert _rel(rho.cpu().numpy(), want) < 1e-12
+    g = op.hx_adjoint_v(a, b, 0.5)
+    adj = O.hx_adjoint_v(ref, a.cpu().numpy(), b.cpu().numpy())
+    assert _rel(g.cpu().numpy(), 0.5 * adj) < 1e-12
+    op.hx_adjoint_v(b, a, 1.0, g)
+    assert _rel(g.cpu().numpy(), 1.5 * adj) < 1e-12
