@@ -863,16 +863,16 @@ extern "C" chfsi_status chfsi_lanczos_bounds_complex(chfsi_operator *op, const v
                                                      double *lower, double *upper, void *stream) {
   CHFSI_ARG(op && v0 && lower && upper, "null argument");
   CHFSI_TRY(check_complex(op));
-  chfsi_solver tmp;
-  return zlanczos_impl(&tmp, op, static_cast<const double *>(v0), steps, reproducible, lower,
+  Workspace ws(op, as_stream(stream));
+  return zlanczos_impl(ws.get(), op, static_cast<const double *>(v0), steps, reproducible, lower,
                        upper, as_stream(stream));
 }
 
 extern "C" chfsi_status chfsi_cholgs_complex(chfsi_operator *op, void *X, int64_t M, int32_t N,
                                              void *stream) {
   CHFSI_ARG(op && X && M == op->M && N > 0, "bad argument");
-  chfsi_solver tmp;
-  return zcholgs_impl(&tmp, static_cast<zc *>(X), M, N, as_stream(stream));
+  Workspace ws(op, as_stream(stream));
+  return zcholgs_impl(ws.get(), static_cast<zc *>(X), M, N, as_stream(stream));
 }
 
 extern "C" chfsi_status chfsi_rayleigh_ritz_complex(chfsi_operator *op, void *X, int64_t M,
@@ -880,8 +880,8 @@ extern "C" chfsi_status chfsi_rayleigh_ritz_complex(chfsi_operator *op, void *X,
                                                     void *stream) {
   CHFSI_ARG(op && X && eig_host && M == op->M && N > 0 && block > 0, "bad argument");
   CHFSI_TRY(check_complex(op));
-  chfsi_solver tmp;
-  return zrr_impl(&tmp, op, static_cast<zc *>(X), M, N, std::min<int>(block, N), eig_host,
+  Workspace ws(op, as_stream(stream));
+  return zrr_impl(ws.get(), op, static_cast<zc *>(X), M, N, std::min<int>(block, N), eig_host,
                   as_stream(stream));
 }
 
@@ -891,8 +891,8 @@ extern "C" chfsi_status chfsi_residual_norms_complex(chfsi_operator *op, const v
                                                      void *stream) {
   CHFSI_ARG(op && X && eig_host && res_host && M == op->M && N > 0 && block > 0, "bad argument");
   CHFSI_TRY(check_complex(op));
-  chfsi_solver tmp;
-  return zresidual_impl(&tmp, op, static_cast<const zc *>(X), M, N, std::min<int>(block, N),
+  Workspace ws(op, as_stream(stream));
+  return zresidual_impl(ws.get(), op, static_cast<const zc *>(X), M, N, std::min<int>(block, N),
                         eig_host, res_host, as_stream(stream));
 }
 

@@ -73,6 +73,7 @@ void Scratch::release() {
 using namespace chfsi;
 
 chfsi_operator::~chfsi_operator() {
+  release_workspace(this);
   void *ptrs[] = {d_map, d_cells_by_color, d_sqrt_mass, d_inv_sqrt_mass, d_sqrt_mass32,
                   d_inv_sqrt_mass32, d_K, d_Nq, d_Gq, d_jxw, d_Ht64, d_Ht32, d_Ht16, d_nlC16, d_nl_off,
                   d_nlC64, d_nlC32,

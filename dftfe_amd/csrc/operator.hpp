@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -48,6 +49,8 @@ chfsi_status quad_product(chfsi_operator *op, const T *a, int64_t lda, const T *
                           double *g, int accumulate, hipStream_t st, int wshift);
 
 }  // namespace chfsi
+
+struct chfsi_solver;
 
 struct chfsi_operator {
   int device = 0;
@@ -139,12 +142,18 @@ struct chfsi_operator {
   float *d_nlCtko32 = nullptr;
   int zproj_variant = 1;
   int zhx_variant64 = 0, zhx_variant32 = 0;
+  // workspace of the entry points without a solver (see Workspace)
+  std::mutex work_mutex;
+  chfsi_solver *work = nullptr;
+  hipEvent_t work_done = nullptr;
   chfsi::Scratch ztab_dev, ztab_W, ztab_P;  // tables and scratch of single complex applies
 
   ~chfsi_operator();
 };
 
 namespace chfsi {
+// Frees the operator's kept workspace
+void release_workspace(chfsi_operator *op);
 // Rebuilds the complex cell matrices of every k-point from the real tiles.
 chfsi_status rebuild_kpoint_matrices(chfsi_operator *op, hipStream_t s);
 }  // namespace chfsi

@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <new>
 #include <vector>
 
 #include "common.hpp"
@@ -984,12 +985,47 @@ extern "C" chfsi_status chfsi_solver_set_lanczos_start(chfsi_solver *s, const do
   return CHFSI_OK;
 }
 
+namespace chfsi {
+Workspace::Workspace(chfsi_operator *op, hipStream_t st) : op_(op), st_(st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
+  if (!op->work_mutex.try_lock()) return;
+  if (!op->work_done && hipEventCreateWithFlags(&op->work_done, hipEventDisableTiming) != hipSuccess)
+    op->work_done = nullptr;
+  if (!op->work) op->work = new (std::nothrow) chfsi_solver();
+  if (!op->work_done || !op->work || hipStreamWaitEvent(st, op->work_done, 0) != hipSuccess) {
+    op->work_mutex.unlock();
+    return;
+  }
+  held_ = true;
+  s_ = op->work;
+}
+
+Workspace::~Workspace() {
+  if (!held_) return;
+  size_t bytes = 0;
+  for (Scratch *b : s_->scratch()) bytes += b->size;
+  if (bytes > kKeep || hipEventRecord(op_->work_done, st_) != hipSuccess) {
+    delete op_->work;  // hipFree waits for the work
+    op_->work = nullptr;
+  }
+  op_->work_mutex.unlock();
+}
+
+void release_workspace(chfsi_operator *op) {
+  delete op->work;
+  op->work = nullptr;
+  if (op->work_done) (void)hipEventDestroy(op->work_done);
+  op->work_done = nullptr;
+}
+}  // namespace chfsi
+
 extern "C" chfsi_status chfsi_chebyshev_filter(chfsi_operator *op, double *X, int64_t ld,
                                                int32_t B, int32_t m, double a, double b,
                                                double a0, int32_t precision, void *stream) {
   CHFSI_ARG(op && X && B > 0 && ld >= B && m >= 1, "bad argument");
-  chfsi_solver tmp;
-  return filter_block(&tmp, op, X, ld, B, m, a, b, a0, precision, 0, as_stream(stream));
+  Workspace ws(op, as_stream(stream));
+  return filter_block(ws.get(), op, X, ld, B, m, a, b, a0, precision, 0, as_stream(stream));
 }
 
 // Reverse pass of the scaled Chebyshev recurrence
@@ -1004,7 +1040,7 @@ extern "C" chfsi_status chfsi_chebyshev_filter(chfsi_operator *op, double *X, in
 // accumulated in FP64 from FP64 interpolations of the FP32 vectors.
 namespace {
 template <typename T>
-chfsi_status filter_backward_impl(chfsi_operator *op, const double *X0, int64_t ldx,
+chfsi_status filter_backward_impl(chfsi_solver *s, chfsi_operator *op, const double *X0, int64_t ldx,
                                   const double *Ybar, int64_t ldy, int B, int m, double a,
                                   double b, double a0, int every, double *Xbar, int64_t ldxb,
                                   double *g, hipStream_t st) {
@@ -1026,7 +1062,7 @@ chfsi_status filter_backward_impl(chfsi_operator *op, const double *X0, int64_t 
   const T c = T(cs.c);
   // storage: X_0 copy, checkpoint pairs, one segment of iterates, 3 adjoint buffers
   const int nseg = (m + every - 1) / every;
-  Scratch ck, seg, adj;
+  Scratch &ck = s->back_ck, &seg = s->back_seg, &adj = s->back_adj;
   CHFSI_TRY(ck.ensure(sizeof(T) * vec * (1 + 2 * nseg)));
   CHFSI_TRY(seg.ensure(sizeof(T) * vec * (every + 2)));
   CHFSI_TRY(adj.ensure(sizeof(T) * vec * 3));
@@ -1105,11 +1141,12 @@ extern "C" chfsi_status chfsi_chebyshev_filter_backward(
   CHFSI_ARG(ldx >= B && ldy >= B && ldxb >= B, "bad leading dimension");
   CHFSI_ARG(op->d_Nq && op->d_jxw, "operator was created without shape data / JxW");
   hipStream_t st = as_stream(stream);
+  Workspace ws(op, st);
   if (precision == CHFSI_FP64)
-    return filter_backward_impl<double>(op, X0, ldx, Ybar, ldy, B, m, a, b, a0, every, Xbar, ldxb,
+    return filter_backward_impl<double>(ws.get(), op, X0, ldx, Ybar, ldy, B, m, a, b, a0, every, Xbar, ldxb,
                                         g, st);
   CHFSI_ARG(precision == CHFSI_FP32, "filter backward precision must be CHFSI_FP64 or CHFSI_FP32");
-  return filter_backward_impl<float>(op, X0, ldx, Ybar, ldy, B, m, a, b, a0, every, Xbar, ldxb, g,
+  return filter_backward_impl<float>(ws.get(), op, X0, ldx, Ybar, ldy, B, m, a, b, a0, every, Xbar, ldxb, g,
                                      st);
 }
 
@@ -1117,22 +1154,22 @@ extern "C" chfsi_status chfsi_lanczos_bounds(chfsi_operator *op, const double *v
                                              int32_t reproducible, double *lower, double *upper,
                                              void *stream) {
   CHFSI_ARG(op && v0 && lower && upper, "null argument");
-  chfsi_solver tmp;
-  return lanczos_impl(&tmp, op, v0, steps, reproducible, lower, upper, as_stream(stream));
+  Workspace ws(op, as_stream(stream));
+  return lanczos_impl(ws.get(), op, v0, steps, reproducible, lower, upper, as_stream(stream));
 }
 
 extern "C" chfsi_status chfsi_cholgs(chfsi_operator *op, double *X, int64_t M, int32_t N,
                                      void *stream) {
   CHFSI_ARG(op && X && M == op->M && N > 0, "bad argument");
-  chfsi_solver tmp;
-  return cholgs_impl(&tmp, X, M, N, std::min<int>(N, 256), false, false, as_stream(stream));
+  Workspace ws(op, as_stream(stream));
+  return cholgs_impl(ws.get(), X, M, N, std::min<int>(N, 256), false, false, as_stream(stream));
 }
 
 extern "C" chfsi_status chfsi_rayleigh_ritz(chfsi_operator *op, double *X, int64_t M, int32_t N,
                                             int32_t block, double *eig_host, void *stream) {
   CHFSI_ARG(op && X && eig_host && M == op->M && N > 0 && block > 0, "bad argument");
-  chfsi_solver tmp;
-  return rr_impl(&tmp, op, X, M, N, std::min<int>(block, N), eig_host, false, false,
+  Workspace ws(op, as_stream(stream));
+  return rr_impl(ws.get(), op, X, M, N, std::min<int>(block, N), eig_host, false, false,
                  as_stream(stream));
 }
 
@@ -1140,8 +1177,8 @@ extern "C" chfsi_status chfsi_residual_norms(chfsi_operator *op, const double *X
                                              int32_t N, int32_t block, const double *eig_host,
                                              double *res_host, void *stream) {
   CHFSI_ARG(op && X && eig_host && res_host && M == op->M && N > 0 && block > 0, "bad argument");
-  chfsi_solver tmp;
-  return residual_impl(&tmp, op, X, N, M, N, std::min<int>(block, N), eig_host, res_host,
+  Workspace ws(op, as_stream(stream));
+  return residual_impl(ws.get(), op, X, N, M, N, std::min<int>(block, N), eig_host, res_host,
                        as_stream(stream));
 }
 
@@ -1153,10 +1190,10 @@ extern "C" chfsi_status chfsi_rayleigh_ritz_spectrum_split(chfsi_operator *op, d
   CHFSI_ARG(op && X && Xfrac && eig_host && M == op->M && N > 0 && block > 0, "bad argument");
   CHFSI_ARG(n_core >= 0 && n_core < N && ld_frac >= N - n_core, "need 0 <= n_core < N, ld_frac >= N - n_core");
   hipStream_t st = as_stream(stream);
-  chfsi_solver tmp;
+  Workspace ws(op, st);
   const int B = std::min<int>(block, N);
-  CHFSI_TRY(cholgs_impl(&tmp, X, M, N, B, false, false, st));
-  return rr_split_impl(&tmp, op, X, M, N, n_core, B, Xfrac, ld_frac, eig_host, mixed_xthx != 0, st);
+  CHFSI_TRY(cholgs_impl(ws.get(), X, M, N, B, false, false, st));
+  return rr_split_impl(ws.get(), op, X, M, N, n_core, B, Xfrac, ld_frac, eig_host, mixed_xthx != 0, st);
 }
 
 namespace {

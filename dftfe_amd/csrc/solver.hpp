@@ -43,11 +43,18 @@ struct chfsi_solver {
   hipStream_t filter_stream = nullptr;
   hipEvent_t filter_fork = nullptr, filter_join = nullptr;
   chfsi::Scratch top_hx;
+  // reverse pass of the filter: checkpoints, one segment of iterates, adjoints
+  chfsi::Scratch back_ck, back_seg, back_adj;
   bool have_v0 = false;
   // largest residual norm over the lowest 90% of states of the last pass that
   // computed residuals, and the filter precision the last pass used
   double last_res_lowest = 1e300;
   int last_precision = CHFSI_FP64;
+  std::vector<chfsi::Scratch *> scratch() {
+    return {&Y64, &X32, &Y32, &HXb, &Hp, &rot, &evals, &info, &part, &lam, &v0, &split, &Xf, &HXf,
+            &Qf, &split32, &rot32, &R32, &dcoef, &gep, &gtiles, &top_hx, &lz, &back_ck, &back_seg,
+            &back_adj};
+  }
   ~chfsi_solver() {
     if (blas) rocblas_destroy_handle(blas);
     for (hipEvent_t e : {rot_done[0], rot_done[1], copy_done[0], copy_done[1], filter_fork,
@@ -55,14 +62,35 @@ struct chfsi_solver {
       if (e) (void)hipEventDestroy(e);
     if (copy_stream) (void)hipStreamDestroy(copy_stream);
     if (filter_stream) (void)hipStreamDestroy(filter_stream);
-    for (chfsi::Scratch *s : {&Y64, &X32, &Y32, &HXb, &Hp, &rot, &evals, &info, &part, &lam, &v0,
-                              &split, &Xf, &HXf, &Qf, &split32, &rot32, &R32, &dcoef, &gep,
-                              &gtiles, &top_hx, &lz})
-      s->release();
+    for (chfsi::Scratch *s : scratch()) s->release();
   }
 };
 
 namespace chfsi {
+
+// Workspace of the entry points that take no solver (filter, Lanczos, CholGS,
+// Rayleigh-Ritz, residuals, their complex forms and the filter's reverse pass):
+// one kept with the operator, so that a call does not allocate and free its
+// blocks and BLAS handle (each hipFree waits for the device; freeing the 6.6 GB
+// of a 256-column reverse pass takes tens of ms).  Another thread's call in the
+// meantime, and calls on a stream under capture, get one of their own; a call on
+// another stream waits for the last one's work.  More than 8 GiB are given back
+// at the end of the call, the rest with the operator.
+class Workspace {
+ public:
+  Workspace(chfsi_operator *op, hipStream_t st);
+  ~Workspace();
+  Workspace(const Workspace &) = delete;
+  Workspace &operator=(const Workspace &) = delete;
+  chfsi_solver *get() { return s_; }
+
+ private:
+  static constexpr size_t kKeep = size_t(8) << 30;
+  chfsi_operator *op_;
+  hipStream_t st_;
+  chfsi_solver local_, *s_ = &local_;
+  bool held_ = false;
+};
 
 // Degree lookup on the upper bound (…SolverDevice.cc:29-46, :96-105).
 unsigned cheby_order_lookup(double upper);
