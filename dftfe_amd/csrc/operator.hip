@@ -82,7 +82,7 @@ chfsi_operator::~chfsi_operator() {
                   d_m_slaves, d_m_vals, d_Mc, d_Gd, d_Hk64, d_Hk32, d_nlCk64, d_nlCtk64,
                   d_nlCk32, d_nlCtk32, d_invJ, d_s_gather64, d_ones_cons64, d_s_gather32,
                   d_ones_cons32, d_own_map, d_own_n, d_nlCto64, d_nlCto32, d_nlCtko64,
-                  d_nlCtko32, d_ttab64, d_ttab32, d_vq64,
+                  d_nlCtko32, d_ttab64, d_ttab32, d_tprod, d_vq64,
                   d_vq32, d_nlCp64,
                   d_nlCp32};
   for (void *p : ptrs)
@@ -300,14 +300,18 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
     } else {
       CHFSI_TRY(dev_upload(&op->d_K, d->stiffness, size_t(ne) * ne));
     }
-    std::vector<double> tab;
+    std::vector<double> tab, products;
     std::vector<float> tab32;
     if (!d->cell_stiffness && Ctot == C &&
-        tensor_tables(d->shape_values, d->stiffness, ne, op->nq, &tab, &tab32)) {
+        tensor_tables(d->shape_values, d->stiffness,
+                      d->inverse_jacobians ? nullptr : d->shape_gradients, ne, op->nq, &tab,
+                      &tab32, &products)) {
       tensor_shape(ne, op->nq, &op->tn, &op->tq);
       const int qe = (op->tq + 1) / 2;
       const size_t nv = size_t(C) * qe * qe * 4 * op->tq;
       CHFSI_TRY(dev_upload(&op->d_ttab64, tab.data(), tab.size()));
+      op->tensor_gga = products.size() > size_t(op->tn) * op->tn * op->tq;
+      CHFSI_TRY(dev_upload(&op->d_tprod, products.data(), products.size()));
       CHFSI_TRY(dev_upload(&op->d_ttab32, tab32.data(), tab32.size()));
       CHFSI_TRY(dev_alloc(&op->d_vq64, nv));
       CHFSI_TRY(dev_alloc(&op->d_vq32, nv));
@@ -578,9 +582,14 @@ extern "C" chfsi_status chfsi_operator_set_potential(chfsi_operator *op, const d
                                                      void *stream) {
   CHFSI_ARG(op && vJxW, "null argument");
   CHFSI_ARG(op->d_Nq && op->d_K, "operator was created without shape data");
-  CHFSI_HIP(launch_build_h(op->d_K, op->d_Nq, vJxW, nullptr, nullptr, op->C, op->ne, op->ne_pad,
-                           op->nq, op->d_Ht64, op->d_Ht32, op->d_Ht16, as_stream(stream),
-                           op->K_per_cell));
+  if (op->tn)
+    CHFSI_HIP(launch_build_tensor(op->d_K, op->d_tprod, vJxW, nullptr, op->C, op->tn, op->tq,
+                                  op->ne_pad, op->d_Ht64, op->d_Ht32, op->d_Ht16,
+                                  as_stream(stream)));
+  else
+    CHFSI_HIP(launch_build_h(op->d_K, op->d_Nq, vJxW, nullptr, nullptr, op->C, op->ne, op->ne_pad,
+                             op->nq, op->d_Ht64, op->d_Ht32, op->d_Ht16, as_stream(stream),
+                             op->K_per_cell));
   if (op->tn)
     CHFSI_HIP(launch_tensor_potential(vJxW, op->C, op->tn, op->tq, op->d_vq64, op->d_vq32,
                                       as_stream(stream)));
@@ -595,9 +604,14 @@ extern "C" chfsi_status chfsi_operator_set_potential_gga(chfsi_operator *op, con
   CHFSI_ARG(op && vJxW && gJxW, "null argument");
   CHFSI_ARG(op->d_Nq && op->d_K, "operator was created without shape data");
   CHFSI_ARG(op->d_Gq, "operator was created without shape gradients");
-  CHFSI_HIP(launch_build_h(op->d_K, op->d_Nq, vJxW, op->d_Gq, gJxW, op->C, op->ne, op->ne_pad,
-                           op->nq, op->d_Ht64, op->d_Ht32, op->d_Ht16, as_stream(stream),
-                           op->K_per_cell, op->d_invJ, op->jac));
+  if (op->tn && op->tensor_gga)
+    CHFSI_HIP(launch_build_tensor(op->d_K, op->d_tprod, vJxW, gJxW, op->C, op->tn, op->tq,
+                                  op->ne_pad, op->d_Ht64, op->d_Ht32, op->d_Ht16,
+                                  as_stream(stream)));
+  else
+    CHFSI_HIP(launch_build_h(op->d_K, op->d_Nq, vJxW, op->d_Gq, gJxW, op->C, op->ne, op->ne_pad,
+                             op->nq, op->d_Ht64, op->d_Ht32, op->d_Ht16, as_stream(stream),
+                             op->K_per_cell, op->d_invJ, op->jac));
   op->tensor_pot = false;
   op->has_H = true;
   op->h_sym = true;

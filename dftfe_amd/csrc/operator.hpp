@@ -100,7 +100,8 @@ struct chfsi_operator {
   // the cell matrices are those of the weights held here (an LDA potential)
   int tn = 0, tq = 0;
   bool tensor_pot = false;
-  double *d_ttab64 = nullptr, *d_vq64 = nullptr, *d_nlCp64 = nullptr;
+  bool tensor_gga = false;  // the shape gradients are products too
+  double *d_ttab64 = nullptr, *d_tprod = nullptr, *d_vq64 = nullptr, *d_nlCp64 = nullptr;
   float *d_ttab32 = nullptr, *d_vq32 = nullptr, *d_nlCp32 = nullptr;
   // HX tile and projection variants per precision (chosen by
   // chfsi_operator_autotune); -1: the tensor form where the operator has it,

@@ -104,11 +104,68 @@ bool tensor_shape(int ne, int nqc, int *n, int *q) {
   return false;
 }
 
-bool tensor_tables(const double *Nq, const double *K, int ne, int nqc, std::vector<double> *tab,
-                   std::vector<float> *tab32) {
+namespace {
+// x, y, z index of each of n^3 nodes or points, x the fastest
+struct Index3 {
+  std::vector<int> x, y, z;
+  explicit Index3(int n) {
+    for (int c = 0; c < n; ++c)
+      for (int b = 0; b < n; ++b)
+        for (int a = 0; a < n; ++a) {
+          x.push_back(a);
+          y.push_back(b);
+          z.push_back(c);
+        }
+  }
+};
+
+// Appends 2 (D_d I + I D_d) of each direction when every shape gradient is a
+// product with one D_d to tol of the largest one
+bool gradient_products(const double *G, const std::vector<ld> &I, int n, int q, double tol,
+                       std::vector<double> *products) {
+  const int ne = n * n * n, nqc = q * q * q;
+  const Index3 in(n), iq(q);
+  std::vector<ld> D[3];
+  for (auto &d : D) d.assign(size_t(q) * n, 0);
+  double gmax = 0;
+  for (int k = 0; k < nqc; ++k)
+    for (int i = 0; i < ne; ++i) {
+      const double *g = G + (size_t(k) * ne + i) * 3;
+      for (int d = 0; d < 3; ++d) gmax = std::max(gmax, std::fabs(g[d]));
+      D[0][iq.x[k] * n + in.x[i]] += g[0] / ld(q * q);
+      D[1][iq.y[k] * n + in.y[i]] += g[1] / ld(q * q);
+      D[2][iq.z[k] * n + in.z[i]] += g[2] / ld(q * q);
+    }
+  const std::vector<double> Id(I.begin(), I.end());
+  std::vector<double> Dd[3];
+  for (int d = 0; d < 3; ++d) Dd[d].assign(D[d].begin(), D[d].end());
+  for (int k = 0; k < nqc; ++k)
+    for (int i = 0; i < ne; ++i) {
+      const int ex = iq.x[k] * n + in.x[i], ey = iq.y[k] * n + in.y[i],
+                ez = iq.z[k] * n + in.z[i];
+      const double *g = G + (size_t(k) * ne + i) * 3;
+      if (!(std::fabs(g[0] - Dd[0][ex] * Id[ey] * Id[ez]) <= tol * gmax &&
+            std::fabs(g[1] - Id[ex] * Dd[1][ey] * Id[ez]) <= tol * gmax &&
+            std::fabs(g[2] - Id[ex] * Id[ey] * Dd[2][ez]) <= tol * gmax))
+        return false;
+    }
+  for (const auto &d : D)
+    for (int a = 0; a < n; ++a)
+      for (int b = 0; b < n; ++b)
+        for (int k = 0; k < q; ++k)
+          products->push_back(
+              (double)(2 * (d[k * n + a] * I[k * n + b] + I[k * n + a] * d[k * n + b])));
+  return true;
+}
+}  // namespace
+
+bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, int nqc,
+                   std::vector<double> *tab, std::vector<float> *tab32,
+                   std::vector<double> *products) {
   int n = 0, q = 0;
   if (!tensor_shape(ne, nqc, &n, &q)) return false;
   const double tol = 1e-13;
+  const Index3 in(n), iq(q);
   const std::vector<ld> w = gauss_weights(q);
   // I: sums of N over the nodes of the other two directions (which are one),
   // mean over their quadrature points and over the directions; x is the
@@ -117,10 +174,18 @@ bool tensor_tables(const double *Nq, const double *K, int ne, int nqc, std::vect
   for (int k = 0; k < nqc; ++k)
     for (int i = 0; i < ne; ++i) {
       const ld v = Nq[size_t(k) * ne + i] / ld(3 * q * q);
-      I[(k % q) * n + i % n] += v;
-      I[(k / q % q) * n + i / n % n] += v;
-      I[(k / q / q) * n + i / n / n] += v;
+      I[iq.x[k] * n + in.x[i]] += v;
+      I[iq.y[k] * n + in.y[i]] += v;
+      I[iq.z[k] * n + in.z[i]] += v;
     }
+  // products of the cell matrix build: I I, and with shape gradients (nqc x ne x
+  // 3, of the same form) 2 (D_d I + I D_d), [a][b][q], symmetric in a and b
+  products->assign(size_t(n) * n * q, 0.0);
+  for (int a = 0; a < n; ++a)
+    for (int b = 0; b < n; ++b)
+      for (int k = 0; k < q; ++k)
+        (*products)[(size_t(a) * n + b) * q + k] = (double)(I[k * n + a] * I[k * n + b]);
+  if (G && !gradient_products(G, I, n, q, tol, products)) products->resize(size_t(n) * n * q);
   symmetrise(I);
   for (int a = 0; a < n; ++a)
     for (int b = 0; b < n; ++b)
@@ -128,28 +193,32 @@ bool tensor_tables(const double *Nq, const double *K, int ne, int nqc, std::vect
   // stiffness of each direction: the mass tables sum to one over the other
   // two, the stiffness tables to zero
   for (auto &A : Kd) A.assign(size_t(n) * n, 0);
-  ld kmax = 0;
+  double kmax = 0;
   for (int i = 0; i < ne; ++i)
     for (int j = 0; j < ne; ++j) {
       const ld v = K[size_t(i) * ne + j];
-      kmax = std::max(kmax, fabsl(v));
-      Kd[0][(i % n) * n + j % n] += v;
-      Kd[1][(i / n % n) * n + j / n % n] += v;
-      Kd[2][(i / n / n) * n + j / n / n] += v;
+      kmax = std::max(kmax, std::fabs((double)v));
+      Kd[0][in.x[i] * n + in.x[j]] += v;
+      Kd[1][in.y[i] * n + in.y[j]] += v;
+      Kd[2][in.z[i] * n + in.z[j]] += v;
     }
   for (auto &A : Kd) symmetrise(A);
+  const std::vector<double> Id(I.begin(), I.end()), Md(M.begin(), M.end());
+  const std::vector<double> Kd0(Kd[0].begin(), Kd[0].end()), Kd1(Kd[1].begin(), Kd[1].end()),
+      Kd2(Kd[2].begin(), Kd[2].end());
   for (int k = 0; k < nqc; ++k)
     for (int i = 0; i < ne; ++i) {
-      const ld v = I[(k % q) * n + i % n] * I[(k / q % q) * n + i / n % n] *
-                   I[(k / q / q) * n + i / n / n];
-      if (!(fabsl(Nq[size_t(k) * ne + i] - v) <= tol)) return false;
+      const double v = Id[iq.x[k] * n + in.x[i]] * Id[iq.y[k] * n + in.y[i]] *
+                       Id[iq.z[k] * n + in.z[i]];
+      if (!(std::fabs(Nq[size_t(k) * ne + i] - v) <= tol)) return false;
     }
   for (int i = 0; i < ne; ++i)
     for (int j = 0; j < ne; ++j) {
-      const int ex = (i % n) * n + j % n, ey = (i / n % n) * n + j / n % n,
-                ez = (i / n / n) * n + j / n / n;
-      const ld v = Kd[0][ex] * M[ey] * M[ez] + M[ex] * Kd[1][ey] * M[ez] + M[ex] * M[ey] * Kd[2][ez];
-      if (!(fabsl(K[size_t(i) * ne + j] - v) <= tol * kmax)) return false;
+      const int ex = in.x[i] * n + in.x[j], ey = in.y[i] * n + in.y[j],
+                ez = in.z[i] * n + in.z[j];
+      const double v =
+          Kd0[ex] * Md[ey] * Md[ez] + Md[ex] * Kd1[ey] * Md[ez] + Md[ex] * Md[ey] * Kd2[ez];
+      if (!(std::fabs(K[size_t(i) * ne + j] - v) <= tol * kmax)) return false;
     }
   // parity tables; the operator applies half the stiffness
   const int NE = (n + 1) / 2, NO = n / 2, QE = (q + 1) / 2, QO = q / 2;
@@ -1402,5 +1471,161 @@ template hipError_t launch_quad_tensor<float>(const uint32_t *, int, int, int, c
                                               const float *, int64_t, const float *, int64_t, int,
                                               const double *, const double *, int, double,
                                               double *, int, const double *, hipStream_t);
+
+// ---------------------------------------------------------------------------
+// Cell matrices, tensor form: H_e = 1/2 K + sum_q N_i N_j v_q (+ the GGA term), as
+// launch_build_h writes them.  A column (i', j', k') is contracted direction by
+// direction with the products P[a][b][q] of the tables: over z for its k', over
+// y for its (j', k') (shared by the n columns of a run), over x with 8 products
+// per entry, where the dense build took 512 (2048 with GGA).  A workgroup takes
+// one cell and a range of 16-column tiles; wave w writes the rows with i = w, two
+// columns per lane, so every 128-byte row of a tile is stored whole.  Entries
+// are sums over the same products in the same order for (i, j) and (j, i):
+// exactly symmetric.  Bound by the stores (7.1 GB of FP64, FP32 and BF16 copies
+// at 4096 cells, p = 6): LDA 5.5 -> 2.8 ms, GGA 20.1 -> 4.4 ms.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+  auto r = [](float x) {
+    uint32_t u = __float_as_uint(x);
+    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+  };
+  return r(a) | (r(b) << 16);
+}
+
+template <int N, int Q, bool GGA>
+__global__ __launch_bounds__(64 * N) void build_tensor_kernel(const double *K, const double *P,
+                                                             const double *vJxW,
+                                                             const double *gJxW, int ne_pad,
+                                                             int tiles, double *Ht64, float *Ht32,
+                                                             uint16_t *Ht16) {
+  constexpr int NT = 64 * N, NN = N * N, NE3 = NN * N, QQ = Q * Q, RUNS = 4;
+  constexpr int F = GGA ? 3 : 1, G2 = GGA ? 2 : 1, NP = GGA ? 4 : 1;
+  constexpr int SB = Q == 8 ? 10 : 6;  // row of y-contracted values, 16-byte aligned
+  static_assert(16 <= (RUNS - 1) * N + 1, "runs of a tile");
+  __shared__ double sP[NP][NN][Q];               // products
+  __shared__ double sV[GGA ? 4 : 1][Q * QQ];     // weights (V, then g of each direction)
+  __shared__ double sA[2][F][N][QQ];             // z-contracted, for k' and the next
+  __shared__ __align__(16) double sB[RUNS][G2][NN][SB];
+  const int64_t cell = blockIdx.x;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  for (int e = t; e < NP * NN * Q; e += NT) (&sP[0][0][0])[e] = P[e];
+  for (int e = t; e < Q * QQ; e += NT) {
+    sV[0][e] = vJxW[cell * (Q * QQ) + e];
+    if constexpr (GGA) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) sV[GGA ? 1 + d : 0][e] = gJxW[(cell * (Q * QQ) + e) * 3 + d];
+    }
+  }
+  __syncthreads();
+  int have[2] = {-1, -1};
+  const int kt1 = min((int)(blockIdx.y + 1) * tiles, ne_pad / 16);
+  for (int kt = blockIdx.y * tiles; kt < kt1; ++kt) {
+    const int c0 = kt * 16, r0 = c0 / N;
+    const int cl = min(c0 + 15, NE3 - 1), nrun = cl / N - r0 + 1;
+    for (int kp = r0 / N; kp <= cl / NN; ++kp) {
+      if (have[kp & 1] == kp) continue;
+      have[kp & 1] = kp;
+      for (int e = t; e < N * QQ; e += NT) {
+        const int k = e / QQ, yx = e % QQ;
+        const double *p = sP[0][k * N + kp];
+        double v = 0.0, x = 0.0, y = 0.0;
+#pragma unroll
+        for (int z = 0; z < Q; ++z) {
+          v = fmadd(p[z], sV[0][z * QQ + yx], v);
+          if constexpr (GGA) {
+            v = fmadd(sP[GGA ? 3 : 0][k * N + kp][z], sV[GGA ? 3 : 0][z * QQ + yx], v);
+            x = fmadd(p[z], sV[GGA ? 1 : 0][z * QQ + yx], x);
+            y = fmadd(p[z], sV[GGA ? 2 : 0][z * QQ + yx], y);
+          }
+        }
+        sA[kp & 1][0][k][yx] = v;
+        if constexpr (GGA) {
+          sA[kp & 1][GGA ? 1 : 0][k][yx] = x;
+          sA[kp & 1][GGA ? 2 : 0][k][yx] = y;
+        }
+      }
+    }
+    __syncthreads();
+    for (int e = t; e < nrun * NN * Q; e += NT) {
+      const int x = e % Q, jk = e / Q % NN, rr = e / (Q * NN);
+      const int jp = (r0 + rr) % N, kp = (r0 + rr) / N, j = jk % N, k = jk / N;
+      const double *p = sP[0][j * N + jp], *a = sA[kp & 1][0][k];
+      double v = 0.0, w = 0.0;
+#pragma unroll
+      for (int y = 0; y < Q; ++y) {
+        v = fmadd(p[y], a[y * Q + x], v);
+        if constexpr (GGA) {
+          v = fmadd(sP[GGA ? 2 : 0][j * N + jp][y], sA[kp & 1][GGA ? 2 : 0][k][y * Q + x], v);
+          w = fmadd(p[y], sA[kp & 1][GGA ? 1 : 0][k][y * Q + x], w);
+        }
+      }
+      sB[rr][0][jk][x] = v;
+      if constexpr (GGA) sB[rr][GGA ? 1 : 0][jk][x] = w;
+    }
+    __syncthreads();
+    // rows of i = wave: lane = (row group, column pair)
+    const int c = c0 + 2 * (lane & 7);
+    const int ca = min(c, NE3 - 1), cb = min(c + 1, NE3 - 1);
+    const int ra = ca / N - r0, rb = cb / N - r0;
+    double pa[G2][Q], pb[G2][Q];
+#pragma unroll
+    for (int s = 0; s < G2; ++s)
+#pragma unroll
+      for (int x = 0; x < Q; ++x) {
+        pa[s][x] = sP[s][wave * N + ca % N][x];
+        pb[s][x] = sP[s][wave * N + cb % N][x];
+      }
+    const int64_t base = (cell * (ne_pad / 16) + kt) * (int64_t)ne_pad * 16 + 2 * (lane & 7);
+    for (int jk = lane >> 3; jk < NN; jk += 8) {
+      const int row = wave + N * jk;
+      double va = 0.0, vb = 0.0;
+#pragma unroll
+      for (int s = 0; s < G2; ++s)
+#pragma unroll
+        for (int x = 0; x < Q; ++x) {
+          va = fmadd(pa[s][x], sB[ra][s][jk][x], va);
+          vb = fmadd(pb[s][x], sB[rb][s][jk][x], vb);
+        }
+      va = c < NE3 ? fmadd(0.5, K[row * NE3 + ca], va) : 0.0;
+      vb = c + 1 < NE3 ? fmadd(0.5, K[row * NE3 + cb], vb) : 0.0;
+      const int64_t o = base + (int64_t)row * 16;
+      *reinterpret_cast<double2 *>(Ht64 + o) = make_double2(va, vb);
+      *reinterpret_cast<float2 *>(Ht32 + o) = make_float2((float)va, (float)vb);
+      *reinterpret_cast<uint32_t *>(Ht16 + o) = bf16_pair((float)va, (float)vb);
+    }
+    for (int e = t; e < (ne_pad - NE3) * 16; e += NT) {  // padded rows
+      const int64_t o = (cell * (ne_pad / 16) + kt) * (int64_t)ne_pad * 16 + NE3 * 16 + e;
+      Ht64[o] = 0.0;
+      Ht32[o] = 0.f;
+      Ht16[o] = 0;
+    }
+    __syncthreads();
+  }
+}
+
+hipError_t launch_build_tensor(const double *K, const double *P, const double *vJxW,
+                               const double *gJxW, int C, int n, int q, int ne_pad, double *Ht64,
+                               float *Ht32, uint16_t *Ht16, hipStream_t s) {
+  // at least about four workgroups per CU
+  const int nt = ne_pad / 16, split = std::min(nt, std::max(1, 1024 / C));
+  const int tiles = (nt + split - 1) / split;
+  const dim3 grid(C, (nt + tiles - 1) / tiles);
+#define CHFSI_BUILD(N, Q)                                                                       \
+  if (n == N && q == Q) {                                                                       \
+    if (gJxW)                                                                                   \
+      hipLaunchKernelGGL((build_tensor_kernel<N, Q, true>), grid, dim3(64 * N), 0, s, K, P,     \
+                         vJxW, gJxW, ne_pad, tiles, Ht64, Ht32, Ht16);                          \
+    else                                                                                        \
+      hipLaunchKernelGGL((build_tensor_kernel<N, Q, false>), grid, dim3(64 * N), 0, s, K, P,    \
+                         vJxW, gJxW, ne_pad, tiles, Ht64, Ht32, Ht16);                          \
+    return hipGetLastError();                                                                   \
+  }
+  CHFSI_BUILD(7, 8)
+  CHFSI_BUILD(6, 6)
+  CHFSI_BUILD(5, 5)
+#undef CHFSI_BUILD
+  return hipErrorInvalidValue;
+}
 
 }  // namespace chfsi

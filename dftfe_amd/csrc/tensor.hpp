@@ -23,9 +23,11 @@ bool tensor_wins(int n, bool fp64, int cells, int B);
 // Host check of an operator's shape values (nqc x ne) and stiffness (ne x ne):
 // true when every entry is the product of one-dimensional, centro-symmetric
 // tables (Gauss quadrature) to 1e-13 of the largest one.  Fills the kernels'
-// tables, FP64 and FP32.
-bool tensor_tables(const double *Nq, const double *K, int ne, int nqc, std::vector<double> *tab,
-                   std::vector<float> *tab32);
+// tables, FP64 and FP32, and the products of the cell matrix build (n^2 q, or
+// 4 n^2 q when the shape gradients G (nqc x ne x 3, nullable) have that form too).
+bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, int nqc,
+                   std::vector<double> *tab, std::vector<float> *tab32,
+                   std::vector<double> *products);
 
 // Weights vJxW (C x nqc) in the kernels' order (scaled by exact powers of two)
 hipError_t launch_tensor_potential(const double *vJxW, int C, int n, int q, double *v64,
@@ -47,5 +49,10 @@ hipError_t launch_quad_tensor(const uint32_t *map, int C, int n, int q, const do
                               const TIn *a, int64_t lda, const TIn *b, int64_t ldb, int B,
                               const double *s_in, const double *w, int wshift, double wscale,
                               double *g, int accumulate, const double *tab, hipStream_t s);
+
+// launch_build_h for one stiffness and geometry, from the products
+hipError_t launch_build_tensor(const double *K, const double *P, const double *vJxW,
+                               const double *gJxW, int C, int n, int q, int ne_pad, double *Ht64,
+                               float *Ht32, uint16_t *Ht16, hipStream_t s);
 
 }  // namespace chfsi

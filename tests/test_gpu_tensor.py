@@ -142,3 +142,25 @@ def test_quadrature_products(case, B, ld, off):
     assert _rel(g.cpu().numpy(), 0.5 * adj) < 1e-12
     op.hx_adjoint_v(b, a, 1.0, g)
     assert _rel(g.cpu().numpy(), 1.5 * adj) < 1e-12
+
+
+@pytest.mark.parametrize("gga", [False, True])
+def test_cell_matrices(case, gga):
+    """LDA and GGA cell matrices, and what the FP32 and BF16 applies read of them."""
+    prob, _, op = case
+    rng = np.random.default_rng(9)
+    g = 0.1 * rng.uniform(-1, 1, (prob.C, prob.nqc, 3)) * prob.jxw_cells[..., None]
+    if gga:
+        op.set_potential_gga(prob.vJxW, g)
+    else:
+        op.set_potential(prob.vJxW)
+    want = O.cell_hamiltonians(prob, gJxW=g) if gga else O.cell_hamiltonians(prob)
+    assert _rel(op.cell_matrices().cpu().numpy(), want) < 1e-13
+    X = torch.tensor(prob.initial_guess(N=16, seed_offset=2), device="cuda")
+    ref = op.apply(X)
+    X32, Y16 = X.float(), torch.zeros_like(X, dtype=torch.float32)
+    op.set_hx_variant(L.FP32, 0)   # the FP32 copy of the matrices
+    assert _rel(op.apply(X32).double().cpu().numpy(), ref.cpu().numpy()) < 2e-6
+    op.HX(X32, False, 1.0, Y16, bf16=True)
+    assert _rel(Y16.double().cpu().numpy(), ref.cpu().numpy()) < 3e-2
+    op.set_potential(prob.vJxW)
