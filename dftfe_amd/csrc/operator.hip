@@ -82,7 +82,7 @@ chfsi_operator::~chfsi_operator() {
                   d_m_slaves, d_m_vals, d_Mc, d_Gd, d_Hk64, d_Hk32, d_nlCk64, d_nlCtk64,
                   d_nlCk32, d_nlCtk32, d_invJ, d_s_gather64, d_ones_cons64, d_s_gather32,
                   d_ones_cons32, d_own_map, d_own_n, d_nlCto64, d_nlCto32, d_nlCtko64,
-                  d_nlCtko32, d_ttab64, d_ttab32, d_tprod, d_vq64,
+                  d_nlCtko32, d_ttab64, d_ttab32, d_tprod, d_touch_ptr, d_touch_idx, d_vq64,
                   d_vq32, d_nlCp64,
                   d_nlCp32};
   for (void *p : ptrs)
@@ -95,6 +95,7 @@ chfsi_operator::~chfsi_operator() {
   W64.release();
   W32.release();
   tmp.release();
+  cells_out.release();
 }
 
 extern "C" const char *chfsi_last_error(void) { return g_last_error.c_str(); }
@@ -313,6 +314,18 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
       op->tensor_gga = products.size() > size_t(op->tn) * op->tn * op->tq;
       CHFSI_TRY(dev_upload(&op->d_tprod, products.data(), products.size()));
       CHFSI_TRY(dev_upload(&op->d_ttab32, tab32.data(), tab32.size()));
+      if (op->max_color_cells <= kAllCellsItems) {
+        std::vector<uint32_t> tptr(M + 1, 0), tidx(size_t(C) * ne);
+        for (int c = 0; c < C; ++c)
+          for (int i = 0; i < ne; ++i) ++tptr[(map[size_t(c) * ne + i] & 0x7fffffffu) + 1];
+        for (int64_t g = 0; g < M; ++g) tptr[g + 1] += tptr[g];
+        std::vector<uint32_t> fill(tptr.begin(), tptr.end() - 1);
+        for (int k = 0; k < C; ++k)
+          for (int i = 0; i < ne; ++i)
+            tidx[fill[map[size_t(cells_sorted[k]) * ne + i] & 0x7fffffffu]++] = uint32_t(k * ne + i);
+        CHFSI_TRY(dev_upload(&op->d_touch_ptr, tptr.data(), tptr.size()));
+        CHFSI_TRY(dev_upload(&op->d_touch_idx, tidx.data(), tidx.size()));
+      }
       CHFSI_TRY(dev_alloc(&op->d_vq64, nv));
       CHFSI_TRY(dev_alloc(&op->d_vq32, nv));
     }
@@ -809,6 +822,7 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
   a.beta_mode = beta_mode;
   a.B = B;
   a.variant = sizeof(T) == 8 ? op->hx_variant64 : (bf16 ? op->hx_variant16 : op->hx_variant32);
+  bool all_cells = false;
   const bool tensor = a.variant < 0 && !bf16 && op->tensor_pot &&
                       ld_src < (int64_t(1) << 29) && ld_dst < (int64_t(1) << 29) &&
                       ldR < (int64_t(1) << 29) &&  // the kernels' row offsets are 32-bit bytes
@@ -824,7 +838,29 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
     a.W = W;
     a.ldW = B;
   }
-  for (int k = 0; k < op->ncolors; ++k) {
+  if (tensor && !ext_scratch) {
+    // small blocks: one launch over all cells and a sum, where the operator
+    // already owns scratch (its projections') and need not grow it in a capture
+    TensorTouch touch{op->d_touch_ptr, op->d_touch_idx, op->M};
+    Scratch &co = op->cells_out;
+    const size_t bytes = sizeof(T) * size_t(op->C) * op->ne * B;
+    bool all = op->d_touch_ptr && op->n_slots > 0 &&
+               tensor_all_cells(op->tn, sizeof(T) == 8, op->max_color_cells, B);
+    if (all && bytes > co.size) {
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      CHFSI_HIP(hipStreamIsCapturing(s, &cap));
+      all = cap == hipStreamCaptureStatusNone;
+    }
+    if (all) {
+      CHFSI_TRY(co.ensure(bytes));
+      a.cells = op->d_cells_by_color;
+      a.ncells = op->C;
+      CHFSI_HIP(launch_hx_tensor<T>(a, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq,
+                                    &touch, static_cast<T *>(co.ptr), s));
+    }
+    all_cells = all;
+  }
+  for (int k = 0; k < (all_cells ? 0 : op->ncolors); ++k) {
     a.cells = op->d_cells_by_color + op->color_off[k];
     a.ncells = op->color_off[k + 1] - op->color_off[k];
     if (a.ncells == 0) continue;
@@ -835,7 +871,8 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
       }
     }
     if (tensor)
-      CHFSI_HIP(launch_hx_tensor<T>(a, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq, s));
+      CHFSI_HIP(launch_hx_tensor<T>(a, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq,
+                                    nullptr, nullptr, s));
     else
       CHFSI_HIP(launch_hx<T>(a, s));
   }

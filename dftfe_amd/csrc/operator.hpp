@@ -100,6 +100,10 @@ struct chfsi_operator {
   // the cell matrices are those of the weights held here (an LDA potential)
   int tn = 0, tq = 0;
   bool tensor_pot = false;
+  // touches of every DOF in colour order and the cells' sums of one apply, for
+  // small blocks (nullable)
+  uint32_t *d_touch_ptr = nullptr, *d_touch_idx = nullptr;
+  chfsi::Scratch cells_out;
   bool tensor_gga = false;  // the shape gradients are products too
   double *d_ttab64 = nullptr, *d_tprod = nullptr, *d_vq64 = nullptr, *d_nlCp64 = nullptr;
   float *d_ttab32 = nullptr, *d_vq32 = nullptr, *d_nlCp32 = nullptr;

@@ -22,6 +22,10 @@
 #include "scatter.hpp"
 #include "tensor.hpp"
 
+// Fused multiply-adds are written out: an instantiation for other widths must
+// not contract other sums, a column has the same bits in every block
+#pragma clang fp contract(off)
+
 namespace chfsi {
 
 // ---------------------------------------------------------------------------
@@ -839,10 +843,12 @@ template <typename T>
 __device__ __forceinline__ T *row_ptr(T *p, uint32_t g, uint32_t ldb) {
   return (T *)((char *)p + (uint64_t)g * ldb);
 }
-template <typename T, int N, int Q, int TC, int VW>
+// CELLS: all cells in one launch, each writing its own sums to cells_out
+// [cell position in a.cells][node][column]; hx_assemble_kernel adds them up
+template <typename T, int N, int Q, int TC, int VW, bool CELLS>
 __global__ __launch_bounds__((TensorShape<T, N, Q, TC, VW>::NT))
 __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_tensor_kernel(
-    HxLaunch<T> a, const T *vq, const T *tabp) {
+    HxLaunch<T> a, const T *vq, const T *tabp, T *cells_out) {
   using S = TensorShape<T, N, Q, TC, VW>;
   using vec = tvec<T, VW>;
   const uint32_t lds_b = (uint32_t)(a.ld_src * sizeof(T)), ldd_b = (uint32_t)(a.ld_dst * sizeof(T)),
@@ -1086,16 +1092,18 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
     }
   }
 
-  // ---- the destination's rows and the first 16 projector rows: loaded here so
+  // ---- the destination's rows: loaded here so
   // that they arrive while the last plane stages run
   vec dv[S::LT][N];
+  if constexpr (!CELLS) {
 #pragma unroll
-  for (int l = 0; l < S::LT; ++l) {
-    const int line = lg + l * S::LG, lc = line < N * N ? line : N * N - 1;
+    for (int l = 0; l < S::LT; ++l) {
+      const int line = lg + l * S::LG, lc = line < N * N ? line : N * N - 1;
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-      dv[l][i] = vload<T, VW>(row_ptr(a.dst + vc, smap[lc * N + i] & 0x7fffffffu, ldd_b));
-  }
+      for (int i = 0; i < N; ++i)
+        dv[l][i] = vload<T, VW>(row_ptr(a.dst + vc, smap[lc * N + i] & 0x7fffffffu, ldd_b));
+    }
+}
   __syncthreads();
   if (px) p1.collect(bq, o); else p0.collect(bq, o);
   __syncthreads();
@@ -1103,11 +1111,12 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
   // what the combine adds on first touch: gamma times the source's row, and in
   // the defect form rcoef times the row of R.  Other rows read the block's first
   // row: one line for all of them
-  const bool any_src = a.gamma != T(0);
   T gamma = a.gamma;
   vec sv[S::LT][N];
 #pragma unroll
   for (int l = 0; l < S::LT; ++l) {
+    if constexpr (CELLS) continue;
+    const bool any_src = a.gamma != T(0);
     const int line = lg + l * S::LG, lc = line < N * N ? line : N * N - 1;
     if (any_src) {
 #pragma unroll
@@ -1120,7 +1129,7 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
       for (int i = 0; i < N; ++i) sv[l][i] = T(0);
     }
   }
-  if constexpr (sizeof(T) == 4) {
+  if constexpr (sizeof(T) == 4 && !CELLS) {
     if (a.R) {
       const vec rc = vload<T, VW>(a.rcoef + vc);
 #pragma unroll
@@ -1159,6 +1168,13 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
       y[N - 1 - i] = e - f;
     }
     if constexpr (N & 1) y[NO] = *reinterpret_cast<const vec *>(b + NO * TC);
+    if constexpr (CELLS) {
+      T *out = cells_out + ((int64_t)(item / a.ntiles) * NE3 + line * N) * a.B + vc;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (vin) vstore<T, VW>(out + (int64_t)i * a.B, y[i]);
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const uint32_t w = smap[line * N + i], g = w & 0x7fffffffu;
@@ -1182,14 +1198,71 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
   }
 }
 
+// ---------------------------------------------------------------------------
+// Sum of the cells' contributions, row by row in colour order: the same
+// multiply-adds in the same order as the colour launches, so the same bits.
+// ---------------------------------------------------------------------------
+template <typename T, int VW>
+__global__ __launch_bounds__(256) void hx_assemble_kernel(HxLaunch<T> a, const uint32_t *ptr,
+                                                          const uint32_t *idx, int64_t M,
+                                                          const T *cells_out) {
+  using vec = tvec<T, VW>;
+  const int per = a.B / VW;
+  const int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x;
+  const int64_t g = e / per;
+  if (g >= M) return;
+  const int v = (int)(e % per) * VW;
+  const uint32_t k0 = ptr[g], k1 = ptr[g + 1];
+  if (k0 == k1) return;  // a folded row: no cell writes it
+  const vec d = vload<T, VW>(a.dst + g * a.ld_dst + v);
+  vec x, r;
+#pragma unroll
+  for (int i = 0; i < VW; ++i) x[i] = r[i] = T(0);
+  if (a.gamma != T(0)) x = vload<T, VW>(a.src + g * a.ld_src + v);
+  T gamma = a.gamma;
+  if constexpr (sizeof(T) == 4) {
+    if (a.R) {
+      r = vload<T, VW>(a.R + g * a.ldR + v);
+      const vec rc = vload<T, VW>(a.rcoef + v);
+#pragma unroll
+      for (int i = 0; i < VW; ++i) x[i] = fmadd(rc[i], r[i], gamma * x[i]);
+      gamma = T(1);
+    }
+  }
+  const T so = a.s_out ? a.s_out[g] : T(1);
+  const bool cons = so == T(0);
+  const T sa = a.alpha * (cons ? T(1) : so);
+  const T kf = a.beta_mode == 2 ? a.beta * so : a.beta;
+  vec y;
+#pragma unroll
+  for (int i = 0; i < VW; ++i)
+    y[i] = cons ? T(0) : fmadd(gamma, x[i], a.beta_mode == 1 ? T(0) : kf * d[i]);
+  for (uint32_t k = k0; k < k1; ++k) {
+    const vec c = vload<T, VW>(cells_out + (int64_t)idx[k] * a.B + v);
+#pragma unroll
+    for (int i = 0; i < VW; ++i) y[i] = fmadd(sa, c[i], y[i]);
+  }
+  vstore<T, VW>(a.dst + g * a.ld_dst + v, y);
+}
+
 template <typename T, int N, int Q, int TC, int VW>
-static hipError_t hx_tensor_go(HxLaunch<T> a, const T *vq, const T *tab, hipStream_t s) {
+static hipError_t hx_tensor_go(HxLaunch<T> a, const T *vq, const T *tab, const TensorTouch *touch,
+                               T *cells_out, hipStream_t s) {
+  using S = TensorShape<T, N, Q, TC, VW>;
   a.ntiles = (a.B + TC - 1) / TC;
   const int items = a.ncells * a.ntiles;
   if (items == 0) return hipSuccess;
   a.per_xcd = (items + 7) / 8;
-  hipLaunchKernelGGL((hx_tensor_kernel<T, N, Q, TC, VW>), dim3(8 * a.per_xcd),
-                     dim3(TensorShape<T, N, Q, TC, VW>::NT), 0, s, a, vq, tab);
+  if (!touch) {
+    hipLaunchKernelGGL((hx_tensor_kernel<T, N, Q, TC, VW, false>), dim3(8 * a.per_xcd),
+                       dim3(S::NT), 0, s, a, vq, tab, nullptr);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((hx_tensor_kernel<T, N, Q, TC, VW, true>), dim3(8 * a.per_xcd), dim3(S::NT),
+                     0, s, a, vq, tab, cells_out);
+  const int64_t n = touch->M * (a.B / VW);
+  hipLaunchKernelGGL((hx_assemble_kernel<T, VW>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                     s, a, touch->ptr, touch->idx, touch->M, cells_out);
   return hipGetLastError();
 }
 
@@ -1197,7 +1270,7 @@ static hipError_t hx_tensor_go(HxLaunch<T> a, const T *vq, const T *tab, hipStre
 // of columns in every block; FP32 falls back to pairs, both to single columns.
 template <typename T, int N, int Q, int TC>
 static hipError_t hx_tensor_vec(const HxLaunch<T> &a, const T *vq, const T *tab,
-                                hipStream_t s) {
+                                const TensorTouch *touch, T *cells_out, hipStream_t s) {
   auto whole = [&](int w) {
     auto ok = [w](const T *p, int64_t ld) {
       return reinterpret_cast<uintptr_t>(p) % (w * sizeof(T)) == 0 && ld % w == 0;
@@ -1206,40 +1279,57 @@ static hipError_t hx_tensor_vec(const HxLaunch<T> &a, const T *vq, const T *tab,
            ok(a.rcoef, 0);
   };
   if constexpr (sizeof(T) == 4)
-    if (whole(4)) return hx_tensor_go<T, N, Q, TC, 4>(a, vq, tab, s);
-  return whole(2) ? hx_tensor_go<T, N, Q, TC, 2>(a, vq, tab, s)
-                  : hx_tensor_go<T, N, Q, TC, 1>(a, vq, tab, s);
+    if (whole(4)) return hx_tensor_go<T, N, Q, TC, 4>(a, vq, tab, touch, cells_out, s);
+  return whole(2) ? hx_tensor_go<T, N, Q, TC, 2>(a, vq, tab, touch, cells_out, s)
+                  : hx_tensor_go<T, N, Q, TC, 1>(a, vq, tab, touch, cells_out, s);
 }
 
 // Where the tensor form is taken (cells: of the largest colour; one MI355X, ms per
 // apply, tensor / best tile variant or, for one column, the matrix-vector kernel):
 //   n = 7: 4096 cells x 1024 columns 5.8 / 11.0 FP32, 1728 x 1024 5.2 / 9.9 FP64,
-//          1728 x 16 0.27 / 0.86, x 1 0.26 / 0.48
-//   n = 6: 1728 cells x 256 columns 1.06 / 1.50 FP64, 0.58 / 0.80 FP32, x 1 0.24 / 0.29
+//          1728 x 16 0.21 / 0.86, x 1 0.16 / 0.48
+//   n = 6: 1728 cells x 256 columns 1.06 / 1.50 FP64, 0.58 / 0.80 FP32, x 1 0.16 / 0.29
 //   n = 5: the dense product is only 1.7 times the operations, on the matrix
 //          pipe; the tensor form has fewer bytes in flight behind its barriers
-//          and wins while a colour launch does not fill the chip: 512 cells x 64
-//          columns 0.15 / 0.19 FP64, 0.11 / 0.13 FP32, x 200 0.25 / 0.22 and 0.14 /
-//          0.21, 1728 x 256 0.77 / 0.62 and 0.44 / 0.38, 512 x 1 0.14 / 0.12
+//          and wins while a colour does not fill the chip: 512 cells x 64 columns
+//          0.09 / 0.19 FP64, 0.06 / 0.13 FP32, x 200 0.216 / 0.218 and 0.13 / 0.21,
+//          x 1 0.05 / 0.12; 1728 x 256 0.77 / 0.62 and 0.44 / 0.38
+static int64_t colour_items(int n, bool fp64, int cells, int B) {
+  const int tc = n == 7 && fp64 ? 16 : 32;
+  return int64_t(cells) * ((B + tc - 1) / tc);
+}
+
 bool tensor_wins(int n, bool fp64, int cells, int B) {
   if (n > 5) return true;
-  const int64_t items = int64_t(cells) * ((B + 31) / 32);
-  return B > 1 && items <= (fp64 ? 320 : 1024);
+  const int64_t items = colour_items(n, fp64, cells, B);
+  return items <= (fp64 || B == 1 ? kAllCellsItems : 1024);
+}
+
+// One launch over all cells and a sum (all) against the colour launches: a launch
+// lasts as long as one workgroup (12-20 us) however few it has, and eight of
+// them in turn leave a small apply waiting; beyond about 450 workgroups a colour
+// the extra pass over the cells' sums costs what the waiting did.  ms per apply,
+// colours / all, FP64: n = 5, 512 cells x 1 column 0.140 / 0.051, x 64 0.146 / 0.092,
+// x 128 0.154 / 0.142, x 400 0.416 / 0.408; n = 7, 512 cells x 1 0.215 / 0.070,
+// x 64 0.228 / 0.177, x 128 0.304 / 0.306; 1728 x 16 0.264 / 0.213
+bool tensor_all_cells(int n, bool fp64, int cells, int B) {
+  return colour_items(n, fp64, cells, B) <= kAllCellsItems;
 }
 
 template <typename T>
 hipError_t launch_hx_tensor(const HxLaunch<T> &a, const T *vq, const T *tab, int n, int q,
-                            hipStream_t s) {
+                            const TensorTouch *touch, T *cells_out, hipStream_t s) {
   constexpr int W7 = sizeof(T) == 8 ? 16 : 32;
-  if (n == 7 && q == 8) return hx_tensor_vec<T, 7, 8, W7>(a, vq, tab, s);
-  if (n == 6 && q == 6) return hx_tensor_vec<T, 6, 6, 32>(a, vq, tab, s);
-  if (n == 5 && q == 5) return hx_tensor_vec<T, 5, 5, 32>(a, vq, tab, s);
+  if (n == 7 && q == 8) return hx_tensor_vec<T, 7, 8, W7>(a, vq, tab, touch, cells_out, s);
+  if (n == 6 && q == 6) return hx_tensor_vec<T, 6, 6, 32>(a, vq, tab, touch, cells_out, s);
+  if (n == 5 && q == 5) return hx_tensor_vec<T, 5, 5, 32>(a, vq, tab, touch, cells_out, s);
   return hipErrorInvalidValue;
 }
 template hipError_t launch_hx_tensor<double>(const HxLaunch<double> &, const double *,
-                                             const double *, int, int, hipStream_t);
+                                             const double *, int, int, const TensorTouch *,
+                                             double *, hipStream_t);
 template hipError_t launch_hx_tensor<float>(const HxLaunch<float> &, const float *, const float *,
-                                            int, int, hipStream_t);
+                                            int, int, const TensorTouch *, float *, hipStream_t);
 
 // ---------------------------------------------------------------------------
 // Products of two blocks at the quadrature points, tensor form (see

@@ -20,6 +20,11 @@ bool tensor_shape(int ne, int nqc, int *n, int *q);
 // largest colour
 bool tensor_wins(int n, bool fp64, int cells, int B);
 
+// workgroups of a colour up to which one launch over all cells is the faster apply
+constexpr int kAllCellsItems = 448;
+// Whether all cells at once beat the colour launches on B columns
+bool tensor_all_cells(int n, bool fp64, int cells, int B);
+
 // Host check of an operator's shape values (nqc x ne) and stiffness (ne x ne):
 // true when every entry is the product of one-dimensional, centro-symmetric
 // tables (Gauss quadrature) to 1e-13 of the largest one.  Fills the kernels'
@@ -37,11 +42,20 @@ hipError_t launch_tensor_potential(const double *vJxW, int C, int n, int q, doub
 hipError_t launch_tensor_projectors(const double *nlC, int64_t total, int n, int ne, int ne_pad,
                                     double *c64, float *c32, hipStream_t s);
 
+// Touches of every DOF row by the cells' nodes in colour order: rows ptr[g] ..
+// ptr[g + 1] of idx, each (position of the cell in the colour order) * n_e + node
+struct TensorTouch {
+  const uint32_t *ptr, *idx;
+  int64_t M;
+};
+
 // One fused HX launch over a colour class (as launch_hx) on the tensor form;
-// a.nl_C: the columns of launch_tensor_projectors
+// a.nl_C: the columns of launch_tensor_projectors.  With touch, all cells at once
+// (a.cells: every colour's) through cells_out (cells x n_e x B) and a sum over
+// the touches: the same result bit for bit
 template <typename T>
 hipError_t launch_hx_tensor(const HxLaunch<T> &a, const T *vq, const T *tab, int n, int q,
-                            hipStream_t s);
+                            const TensorTouch *touch, T *cells_out, hipStream_t s);
 
 // launch_quad_product on the tensor form (tab: the FP64 tables)
 template <typename TIn>

@@ -147,7 +147,10 @@ def test_quadrature_products(case, B, ld, off):
 @pytest.mark.parametrize("gga", [False, True])
 def test_cell_matrices(case, gga):
     """LDA and GGA cell matrices, and what the FP32 and BF16 applies read of them."""
-    prob, _, op = case
+    from dftfe_amd.chfsi import KohnShamOperatorDevice
+
+    prob = case[0]
+    op = KohnShamOperatorDevice(prob)   # of its own: a variant, once set, stays
     rng = np.random.default_rng(9)
     g = 0.1 * rng.uniform(-1, 1, (prob.C, prob.nqc, 3)) * prob.jxw_cells[..., None]
     if gga:
@@ -163,4 +166,33 @@ def test_cell_matrices(case, gga):
     assert _rel(op.apply(X32).double().cpu().numpy(), ref.cpu().numpy()) < 2e-6
     op.HX(X32, False, 1.0, Y16, bf16=True)
     assert _rel(Y16.double().cpu().numpy(), ref.cpu().numpy()) < 3e-2
-    op.set_potential(prob.vJxW)
+
+
+@pytest.mark.parametrize("B", [1, 6, 32])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_all_cells_at_once_equals_colour_launches(case, B, dtype):
+    """Small blocks run all cells in one launch and add up per row in colour order;
+    the same columns inside a block wide enough for the colour launches have the
+    same bits, through the Chebyshev combine too."""
+    from dftfe_amd.chfsi import chebyshev_filter
+
+    prob, ref, op = case
+    wide = 2048                 # 8 cells a colour: 512 (64-bit p = 6: 1024) workgroups
+    rng = np.random.default_rng(B)
+    X = torch.zeros(prob.M, wide, device="cuda", dtype=dtype)
+    X[:, :B] = torch.tensor(rng.uniform(-1, 1, (prob.M, B)), device="cuda", dtype=dtype)
+    X[torch.tensor(prob.constrained, device="cuda")] = 0
+    Y, y = torch.ones_like(X), torch.ones(prob.M, B, device="cuda", dtype=dtype)
+    op.HX(X, False, 0.5, Y)
+    op.HX(X[:, :B].contiguous(), False, 0.5, y)
+    if prob.wl.p > 4:           # wide p = 4 blocks take the dense form
+        assert torch.equal(Y[:, :B], y)
+    else:
+        assert _rel(Y[:, :B].double().cpu().numpy(), y.double().cpu().numpy()) < (
+            1e-13 if dtype == torch.float64 else 2e-6)
+    if dtype == torch.float64:
+        F, f = X.clone(), X[:, :B].contiguous()
+        for Z in (F, f):
+            chebyshev_filter(op, Z, 5, 1.0, 120.0, -3.0)
+        if prob.wl.p > 4:
+            assert torch.equal(F[:, :B], f)
