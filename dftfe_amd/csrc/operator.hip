@@ -733,6 +733,15 @@ struct OpData<float> {
   static const float *ones_cons(chfsi_operator *op) { return op->d_ones_cons32; }
 };
 
+// Projection of an operator whose variant was not set: owned rows on wide tiles
+// (variant 4) where their workgroups fill the chip, the cell form on 64 columns
+// (0) for less.  ms per apply, 0 / 4: p = 6, 4096 cells x 1024 columns FP32 6.07 / 5.79,
+// 1728 cells x 333 FP64 2.29 / 2.14, x 1 0.27 / 0.26; p = 5, 1728 x 250 1.15 / 1.07;
+// p = 6, 216 cells x 16 0.175 / 0.189; p = 4, 512 x 64 0.141 / 0.147
+static int proj_default(int cells, int B) {
+  return int64_t(cells) * ((B + 127) / 128) >= 768 ? 4 : 0;
+}
+
 template <typename T>
 chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, int64_t ld_dst,
                       int B, T alpha, T beta, T gamma, int beta_mode, bool scaled,
@@ -796,6 +805,7 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
     pl.B = B;
     pl.max_srb = op->max_srb;
     pl.variant = sizeof(T) == 8 ? op->proj_variant64 : op->proj_variant32;
+    if (pl.variant < 0) pl.variant = bf16 ? 0 : proj_default(op->n_nl_cells, B);
     if (pl.variant >= 4) {
       pl.nl_Ct = OpData<T>::nlCto(op);
       pl.own_map = op->d_own_map;

@@ -112,7 +112,7 @@ struct chfsi_operator {
   // tile variant 0 otherwise
   int hx_variant64 = -1, hx_variant32 = -1;
   int hx_variant16 = 0;  // BF16 apply: 0 K = 32 ring, 1 register-staged K = 16
-  int proj_variant64 = 0, proj_variant32 = 0;
+  int proj_variant64 = -1, proj_variant32 = -1;  // -1: by size (proj_default)
   int max_srb = 1;  // largest slot count of any cell / 16
   // extra cell ids C .. C + n_extra_cells - 1: further projector groups of
   // cells with more than 128 slots (zero cell matrix, own colours, the nodes
