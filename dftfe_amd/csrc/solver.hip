@@ -476,8 +476,10 @@ chfsi_status gram_fp64(chfsi_solver *s, const double *A, int64_t lda, const doub
 // its own panel of X).  Before panel p + 2 reuses the buffer, st waits for
 // panel p's copy; at the end st waits for every copy.  upper: R is upper
 // triangular with its lower part stored as zeros; the panel is rotated by
-// column blocks of 256, block [c0, c0 + 256) over the inner extent
-// c0 + 256 only, so every launch has work items of one length.
+// column blocks of 128, block [c0, c0 + 128) over the inner extent
+// c0 + 128 only, so every launch has work items of one length (CholGS of 500 columns
+// on 216k rows 5.52 ms; blocks of 256: 5.66, which compute 15% more zeros; one launch
+// over all lengths: 6.28).
 chfsi_status rotate_fp64(chfsi_solver *s, double *X, int64_t M, int N, const double *Rm,
                          int64_t ldr, int trans, int upper, hipStream_t st) {
   const int64_t chunk = panel_rows(M, N);
@@ -499,7 +501,7 @@ chfsi_status rotate_fp64(chfsi_solver *s, double *X, int64_t M, int N, const dou
     double *tmp = sptr<double>(s->rot) + (int64_t)b * chunk * N;
     if (p >= 2) CHFSI_HIP(hipStreamWaitEvent(st, s->copy_done[b], 0));
     if (upper) {
-      constexpr int CB = 256;
+      constexpr int CB = 128;
       for (int c0 = 0; c0 < N; c0 += CB) {
         const int bw = std::min(CB, N - c0);
         // R(i, c0 + j): Rm[c0 + j + i ldr] (trans) or Rm[i + (c0 + j) ldr]
