@@ -1450,6 +1450,15 @@ __global__ void slave_to_master_kernel(const int64_t *m_rows, const int64_t *m_p
   const int64_t m = m_rows[r];
   X[m * ld + v] += (so ? so[m] : T(1)) * s;
 }
+// X[rows[r], v] *= a
+template <typename T>
+__global__ void scale_listed_rows_kernel(const int64_t *rows, int64_t nrows, T a, T *X, int64_t ld,
+                                         int B) {
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= nrows * B) return;
+  X[rows[idx / B] * ld + idx % B] *= a;
+}
+
 template <typename T>
 __global__ void zero_rows_kernel(const int64_t *rows, int64_t nrows, T *X, int64_t ld, int B) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2752,8 +2761,6 @@ hipError_t launch_axpby(int64_t n, T a, const T *x, T b, T *y, hipStream_t st) {
 }
 template hipError_t launch_axpby<double>(int64_t, double, const double *, double, double *,
                                          hipStream_t);
-template hipError_t launch_axpby<float>(int64_t, float, const float *, float, float *,
-                                        hipStream_t);
 
 hipError_t launch_residual_partial(const double *HX, int64_t ldH, const double *X, int64_t ldX,
                                    const double *lam, int64_t M, int B, double *partial,
@@ -2890,6 +2897,18 @@ template hipError_t launch_slave_to_master_scaled<float>(const int64_t *, const 
                                                          int64_t, const float *, float *,
                                                          int64_t, int, hipStream_t);
 
+template <typename T>
+hipError_t launch_scale_listed_rows(const int64_t *rows, int64_t nrows, T a, T *X, int64_t ld,
+                                    int B, hipStream_t st) {
+  if (nrows == 0) return hipSuccess;
+  hipLaunchKernelGGL(scale_listed_rows_kernel<T>, dim3(grid_for(nrows * B, 256, 1u << 30)),
+                     dim3(256), 0, st, rows, nrows, a, X, ld, B);
+  return hipGetLastError();
+}
+template hipError_t launch_scale_listed_rows<double>(const int64_t *, int64_t, double, double *,
+                                                     int64_t, int, hipStream_t);
+template hipError_t launch_scale_listed_rows<float>(const int64_t *, int64_t, float, float *,
+                                                    int64_t, int, hipStream_t);
 template <typename T>
 hipError_t launch_zero_rows_t(const int64_t *rows, int64_t nrows, T *X, int64_t ld, int B,
                               hipStream_t st) {

@@ -204,6 +204,10 @@ hipError_t launch_slave_to_master_scaled(const int64_t *m_rows, const int64_t *m
                                          const int64_t *m_slaves, const double *m_vals,
                                          int64_t nm, const T *so, T *X, int64_t ld, int B,
                                          hipStream_t st);
+// X[rows[r], v] *= a
+template <typename T>
+hipError_t launch_scale_listed_rows(const int64_t *rows, int64_t nrows, T a, T *X, int64_t ld,
+                                    int B, hipStream_t st);
 template <typename T>
 hipError_t launch_zero_rows_t(const int64_t *rows, int64_t nrows, T *X, int64_t ld, int B,
                               hipStream_t st);

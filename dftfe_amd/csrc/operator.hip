@@ -78,7 +78,7 @@ chfsi_operator::~chfsi_operator() {
                   d_inv_sqrt_mass32, d_K, d_Nq, d_Gq, d_jxw, d_Ht64, d_Ht32, d_Ht16, d_nlC16, d_nl_off,
                   d_nlC64, d_nlC32,
                   d_nlCt64, d_nlCt32, d_slot_proj, d_proj_ptr, d_proj_slots, d_proj_V,
-                  d_nl_cells, d_c_rows, d_c_ptr, d_c_cols, d_c_vals, d_m_rows, d_m_ptr,
+                  d_nl_cells, d_idle_rows, d_c_rows, d_c_ptr, d_c_cols, d_c_vals, d_m_rows, d_m_ptr,
                   d_m_slaves, d_m_vals, d_Mc, d_Gd, d_Hk64, d_Hk32, d_nlCk64, d_nlCtk64,
                   d_nlCk32, d_nlCtk32, d_invJ, d_s_gather64, d_ones_cons64, d_s_gather32,
                   d_ones_cons32, d_own_map, d_own_n, d_nlCto64, d_nlCto32, d_nlCtko64,
@@ -281,6 +281,11 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
     }
   }
   CHFSI_TRY(dev_upload(&op->d_map, map.data(), map.size()));
+  std::vector<int64_t> idle;
+  for (int64_t g = 0; g < M; ++g)
+    if (touched_color[g] < 0) idle.push_back(g);
+  op->n_idle = (int64_t)idle.size();
+  if (op->n_idle > 0) CHFSI_TRY(dev_upload(&op->d_idle_rows, idle.data(), idle.size()));
   CHFSI_TRY(dev_upload(&op->d_cells_by_color, cells_sorted.data(), cells_sorted.size()));
 
   // ---- mass vectors

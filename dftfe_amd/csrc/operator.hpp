@@ -120,6 +120,8 @@ struct chfsi_operator {
   int n_extra_cells = 0;
   // constraints (slave-major and master-major CSR)
   int64_t nc = 0, nm = 0;
+  int64_t *d_idle_rows = nullptr;  // rows no cell writes (folded constraints)
+  int64_t n_idle = 0;
   int64_t *d_c_rows = nullptr, *d_c_ptr = nullptr, *d_c_cols = nullptr;
   double *d_c_vals = nullptr;
   int64_t *d_m_rows = nullptr, *d_m_ptr = nullptr, *d_m_slaves = nullptr;

@@ -1034,8 +1034,7 @@ extern "C" chfsi_status chfsi_chebyshev_filter(chfsi_operator *op, double *X, in
 //   X_1 = k1 (H~ - c) X_0,   X_k = a1_k (H~ - c) X_{k-1} + a2_k X_{k-2}  (k = 2..m),  Y = X_m.
 // With L_k = dL/dX_k, going from k = m down to 1:
 //   g     += a1_k * adjV(L_k, X_{k-1})           (dL/dV through the HX of step k)
-//   L_{k-1} += a1_k (H~ - c) L_k                  (one fused HX, beta = 1)
-//   L_{k-2} += a2_k L_k
+//   L_{k-1} = a1_k (H~ - c) L_k + a2_{k+1} L_{k+1}   (one fused HX in place of L_{k+1})
 // and X0bar = L_0.  Forward iterates come from checkpoints (pairs X_{k-1}, X_k
 // every `every` degrees) re-run one segment at a time.  T is the arithmetic of
 // the iterates and adjoints (FP64, or FP32 on the FP32 apply); g is always
@@ -1062,12 +1061,12 @@ chfsi_status filter_backward_impl(chfsi_solver *s, chfsi_operator *op, const dou
     }
   }
   const T c = T(cs.c);
-  // storage: X_0 copy, checkpoint pairs, one segment of iterates, 3 adjoint buffers
+  // storage: X_0 copy, checkpoint pairs, one segment of iterates, 2 adjoint buffers
   const int nseg = (m + every - 1) / every;
   Scratch &ck = s->back_ck, &seg = s->back_seg, &adj = s->back_adj;
   CHFSI_TRY(ck.ensure(sizeof(T) * vec * (1 + 2 * nseg)));
   CHFSI_TRY(seg.ensure(sizeof(T) * vec * (every + 2)));
-  CHFSI_TRY(adj.ensure(sizeof(T) * vec * 3));
+  CHFSI_TRY(adj.ensure(sizeof(T) * vec * 2));
   T *ckp = sptr<T>(ck), *segp = sptr<T>(seg), *adjp = sptr<T>(adj);
   auto ckv = [&](int i) { return ckp + vec * i; };
   CHFSI_HIP(launch_copy_block<double, T>(X0, ldx, ckv(0), B, M, B, st));
@@ -1091,10 +1090,10 @@ chfsi_status filter_backward_impl(chfsi_solver *s, chfsi_operator *op, const dou
       std::swap(ldc, ldp);
     }
   }
-  // adjoint sweep: Lk = L_k, Lm1 = L_{k-1}, Lm2 = L_{k-2}
-  T *Lk = adjp, *Lm1 = adjp + vec, *Lm2 = adjp + 2 * vec;
+  // adjoint sweep: Lk = L_k, Lp = L_{k+1}
+  T *Lk = adjp, *Lp = adjp + vec;
   CHFSI_HIP(launch_copy_block<double, T>(Ybar, ldy, Lk, B, M, B, st));
-  CHFSI_HIP(hipMemsetAsync(Lm1, 0, sizeof(T) * vec * 2, st));
+  CHFSI_HIP(hipMemsetAsync(Lp, 0, sizeof(T) * vec, st));
   for (int sg = nseg - 1; sg >= 0; --sg) {
     const int k0 = sg * every, k1 = std::min(m, k0 + every);
     // iterates X_{k0-1 .. k1-1} into seg[0 .. ]: seg[i] = X_{k0 - 1 + i}
@@ -1118,14 +1117,12 @@ chfsi_status filter_backward_impl(chfsi_solver *s, chfsi_operator *op, const dou
     for (int k = k1; k >= k0 + 1; --k) {
       CHFSI_TRY(quad_product<T>(op, Lk, B, X(k - 1), B, B, true, op->d_jxw, nullptr, a1[k], g, 1,
                                 st, 0));
-      CHFSI_TRY(hx_fused<T>(op, Lk, B, Lm1, B, B, T(a1[k]), T(1), T(-c * a1[k]), 0, true, st));
-      if (k >= 2) CHFSI_HIP(launch_axpby<T>((int64_t)vec, T(a2[k]), Lk, T(1), Lm2, st));
-      // shift: (L_k, L_{k-1}, L_{k-2}) <- (L_{k-1}, L_{k-2}, 0)
-      T *t = Lk;
-      Lk = Lm1;
-      Lm1 = Lm2;
-      Lm2 = t;
-      CHFSI_HIP(hipMemsetAsync(Lm2, 0, sizeof(T) * vec, st));
+      if (k < m)  // rows that no cell writes
+        CHFSI_HIP(launch_scale_listed_rows<T>(op->d_idle_rows, op->n_idle, T(a2[k + 1]), Lp, B, B,
+                                              st));
+      CHFSI_TRY(hx_fused<T>(op, Lk, B, Lp, B, B, T(a1[k]), k < m ? T(a2[k + 1]) : T(0),
+                            T(-c * a1[k]), k < m ? 0 : 1, true, st));
+      std::swap(Lk, Lp);
     }
   }
   CHFSI_HIP(launch_copy_block<T, double>(Lk, B, Xbar, ldxb, M, B, st));

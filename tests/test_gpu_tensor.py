@@ -79,6 +79,35 @@ def test_filter_and_defect_combine(case, N):
         assert _rel(Y.cpu().numpy(), want) < tol, prec
 
 
+@pytest.mark.parametrize("m,every", [(1, 1), (2, 1), (4, 3), (5, 8)])
+@pytest.mark.parametrize("prec,tol", [(L.FP64, 1e-11), (L.FP32, 2e-4)])
+def test_filter_backward_in_place(case, m, every, prec, tol):
+    """The reverse pass keeps two adjoint blocks and writes each step over the older
+    one; rows that no cell writes take the recurrence's a2 alone."""
+    prob, ref, op = case
+    X = prob.sqrt_mass[:, None] * prob.initial_guess(N=10, seed_offset=m)
+    Y = np.random.default_rng(m).uniform(-1, 1, X.shape)
+    _, up, _, _ = O.lanczos_bounds(ref, prob.lanczos_start, 10)
+    a, b, a0 = 1.0, up + 10.0, -3.0
+    got, g = op.filter_backward(torch.tensor(X, device="cuda"), torch.tensor(Y, device="cuda"), m,
+                                a, b, a0, checkpoint_every=every, precision=prec)
+    ok = ~prob.constrained
+    free = np.where(ok[:, None], Y, 0.0)
+    want, gw = O.filter_backward(ref, X, free, m, a, b, a0)
+    got = got.cpu().numpy()
+    assert _rel(got[ok], want[ok]) < tol
+    assert _rel(g.cpu().numpy(), gw) < tol
+    if prob.constrained.any():
+        e, c = (b - a) / 2, (b + a) / 2
+        s1 = s = e / (a0 - c)
+        f = 0.0 if m % 2 else 1.0
+        for k in range(2, m + 1):
+            s2 = 1.0 / (2.0 / s1 - s)
+            f *= -(s * s2) if k % 2 == 0 else 1.0
+            s = s2
+        assert np.abs(got[~ok] - f * Y[~ok]).max() < tol * max(abs(f), 1e-30)
+
+
 def test_other_tables_take_the_dense_form():
     """A stiffness that is no sum of products, and cells of another quadrature,
     give the oracle's apply (through the cell matrices)."""
