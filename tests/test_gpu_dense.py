@@ -74,3 +74,25 @@ def test_pass_library_kernels_and_rocblas(small):
         print(f"dense_rocblas={rb}: max|dlambda| {err:.2e} Ha")
         assert err <= 1e-10
         assert np.abs(res - res_o).max() <= 1e-8
+
+
+@pytest.mark.parametrize("N", [1, 2, 15, 16, 17, 31, 97, 127, 128, 129, 130, 161, 257])
+@pytest.mark.parametrize("off", [0, 1])
+def test_dense_tile_edges(small, N, off):
+    """Widths around the 16-wide blocks and 128-wide tiles; off 1: X starts on an odd
+    double, so that rows cannot be read in pairs."""
+    from dftfe_amd.chfsi import cholgs, rayleigh_ritz
+
+    prob, ref, op = small
+    X = prob.sqrt_mass[:, None] * prob.initial_guess(N=N, seed_offset=N + 1)
+    buf = torch.empty(prob.M * N + 1, device="cuda", dtype=torch.float64)
+    Xd = buf[off:off + prob.M * N].view(prob.M, N)
+    Xd.copy_(torch.tensor(X))
+    cholgs(op, Xd)
+    Xo = O.cholgs(X)
+    assert _rel(Xd.cpu().numpy(), Xo) < 1e-10
+    lam = rayleigh_ritz(op, Xd, 64)
+    lam_o, _ = O.rayleigh_ritz(ref, Xo, 64)
+    assert np.abs(lam - lam_o).max() < 1e-10
+    G = (Xd.T @ Xd).cpu().numpy()
+    assert np.abs(G - np.eye(N)).max() < 1e-12
