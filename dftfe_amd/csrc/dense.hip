@@ -17,6 +17,9 @@
 
 #include <stdint.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "dense.hpp"
 #include "mfma.hpp"
 
@@ -26,7 +29,7 @@ namespace {
 
 constexpr int TT = 128;   // output tile edge
 constexpr int KS = 16;    // K rows per LDS slab
-constexpr int NT = 256;   // 4 waves, each a 64 x 64 quarter of the tile
+constexpr int NT = 256;   // 4 waves (wi, wj): blocks of 16 (2a + wi, 2b + wj), a, b < 4
 constexpr int PADW = 16;  // LDS row padding of [k][128] slabs (doubles)
 
 // Work items are spread over the 8 XCDs so that consecutive items (the tiles
@@ -35,6 +38,40 @@ constexpr int PADW = 16;  // LDS row padding of [k][128] slabs (doubles)
 __device__ __forceinline__ int xcd_item(int per_xcd) {
   const int wid = blockIdx.x;
   return (wid & 7) * per_xcd + (wid >> 3);
+}
+
+// acc[a][b] += A block a x B block b over one slab, for the blocks in MASK (bit 4 a + b).
+// A[k][row] is at as[k AK + row AR], B[k][column] at bs[k BK + column BR], from the lane's
+// own k, row and column on.
+template <unsigned MASK, int AK, int AR, int BK, int BR>
+__device__ __forceinline__ void blocks(const double *as, const double *bs, f64x4 (&acc)[4][4]) {
+#pragma unroll
+  for (int kk = 0; kk < KS / 4; ++kk) {
+    double av[4], bv[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (MASK >> (4 * q) & 15) av[q] = as[kk * 4 * AK + q * 32 * AR];
+      if (MASK >> q & 0x1111) bv[q] = bs[kk * 4 * BK + q * 32 * BR];
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        if (MASK >> (4 * a + b) & 1) acc[a][b] = mfma16(av[a], bv[b], acc[a][b]);
+  }
+}
+
+// Sets of blocks (bit 4 a + b) that the kernels are compiled for.  One set serves the
+// four waves of a workgroup: branches around single MFMAs made the compiler copy
+// accumulators (190 spilled registers).  gram: all; on and below the diagonal; tiles
+// with 96 / 64 rows and their diagonal forms.  rotate: all columns, 96, 64, 32.
+constexpr int kGramForms = 6;
+constexpr unsigned kGramForm[kGramForms] = {0xffff, 0xf731, 0x0fff, 0x0731, 0x00ff, 0x0031};
+constexpr unsigned kColumnForm[4] = {0x1111, 0x3333, 0x7777, 0xffff};
+
+__host__ __device__ inline int gram_form(int I, int J, int m, int diag_off) {
+  const int na = m - I > 96 ? 0 : (m - I > 64 ? 2 : 4);
+  return na + (diag_off >= 0 && J + diag_off >= I ? 1 : 0);
 }
 
 // Entries c .. c + 7 of a row of n into r, those past its end read from entry 0.
@@ -56,25 +93,26 @@ __device__ __forceinline__ void load8(const double *row, int c, int n, double2 (
 
 // Bound by the FP64 matrix cores.  The loads of slab s + 1 are issued before the MFMAs
 // of slab s and first used when they are stored behind them; with the masks applied
-// at the load every slab waited for them (500 columns on 216k rows: 1.77 ms, now 1.39).
+// at the load every slab waited for them (500 columns on 216k rows: 1.77 ms, then 1.39;
+// 1.33 with the blocks below).
 //
 // C_tile(I, J) = sum_{k in chunk} A[k, I + i] B[k, J + j], written to
-// P[item][i + 128 j] (item = chunk * ntiles + tile)
+// P[part][i + 128 j].  Blocks of 16 past the edge or above the diagonal are left out
+// (zero in P); dealing the blocks to the waves alternately leaves each of them 10 of 16
+// in a diagonal tile.
 template <bool VEC>
 __global__ __launch_bounds__(NT, 2) void gram_kernel(const double *A, int64_t lda, const double *B,
                                                      int64_t ldb, int m, int n, int64_t K,
-                                                     int64_t kchunk, const int2 *tiles,
-                                                     int ntiles, int per_xcd, int nitems,
-                                                     double *P) {
+                                                     int diag_off, const GramItem *items,
+                                                     int per_xcd, int nitems, double *P) {
   __shared__ __align__(16) double As[2][KS][TT + PADW];
   __shared__ __align__(16) double Bs[2][KS][TT + PADW];
   const int item = xcd_item(per_xcd);
   if ((blockIdx.x >> 3) >= per_xcd || item >= nitems) return;
-  const int chunk = item / ntiles;
-  const int2 tl = tiles[item % ntiles];
-  const int I = tl.x * TT, J = tl.y * TT;
-  const int64_t kb = (int64_t)chunk * kchunk;
-  const int64_t ke = kb + kchunk < K ? kb + kchunk : K;
+  const GramItem it = items[item];
+  const int I = it.I * TT, J = it.J * TT;
+  const int64_t kb = (int64_t)it.slab * KS;
+  const int64_t ke = kb + (int64_t)it.nslab * KS < K ? kb + (int64_t)it.nslab * KS : K;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wi = w & 1, wj = w >> 1;
 
@@ -101,65 +139,65 @@ __global__ __launch_bounds__(NT, 2) void gram_kernel(const double *A, int64_t ld
     }
   };
 
-  f64x4 acc[4][4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = f64x4{0, 0, 0, 0};
-
   const int nslab = (int)((ke - kb + KS - 1) / KS);
-  if (nslab > 0) {
-    load(kb);
-    store(0, kb);
-  }
-  __syncthreads();
-  for (int s = 0; s < nslab; ++s) {
-    const int buf = s & 1;
-    if (s + 1 < nslab) load(kb + (int64_t)(s + 1) * KS);
+  auto run = [&](auto form) {
+    constexpr unsigned MASK = decltype(form)::value;
+    f64x4 acc[4][4];
 #pragma unroll
-    for (int kk = 0; kk < KS / 4; ++kk) {
-      const int k = kk * 4 + (lane >> 4);
-      double av[4], bv[4];
+    for (int a = 0; a < 4; ++a)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        av[q] = As[buf][k][wi * 64 + q * 16 + (lane & 15)];
-        bv[q] = Bs[buf][k][wj * 64 + q * 16 + (lane & 15)];
-      }
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = mfma16(av[a], bv[b], acc[a][b]);
+      for (int b = 0; b < 4; ++b) acc[a][b] = f64x4{0, 0, 0, 0};
+    if (nslab > 0) {
+      load(kb);
+      store(0, kb);
     }
-    if (s + 1 < nslab) store(buf ^ 1, kb + (int64_t)(s + 1) * KS);
     __syncthreads();
+    for (int s = 0; s < nslab; ++s) {
+      const int buf = s & 1;
+      if (s + 1 < nslab) load(kb + (int64_t)(s + 1) * KS);
+      blocks<MASK, TT + PADW, 1, TT + PADW, 1>(&As[buf][lane >> 4][wi * 16 + (lane & 15)],
+                                               &Bs[buf][lane >> 4][wj * 16 + (lane & 15)], acc);
+      if (s + 1 < nslab) store(buf ^ 1, kb + (int64_t)(s + 1) * KS);
+      __syncthreads();
+    }
+    double *Pt = P + (int64_t)it.part * TT * TT;
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = (2 * a + wi) * 16 + acc_row<double>(lane, r);
+          const int j = (2 * b + wj) * 16 + (lane & 15);
+          Pt[i + (int64_t)j * TT] = acc[a][b][r];
+        }
+  };
+  switch (gram_form(I, J, m, diag_off)) {
+    case 0: run(std::integral_constant<unsigned, kGramForm[0]>{}); break;
+    case 1: run(std::integral_constant<unsigned, kGramForm[1]>{}); break;
+    case 2: run(std::integral_constant<unsigned, kGramForm[2]>{}); break;
+    case 3: run(std::integral_constant<unsigned, kGramForm[3]>{}); break;
+    case 4: run(std::integral_constant<unsigned, kGramForm[4]>{}); break;
+    default: run(std::integral_constant<unsigned, kGramForm[5]>{}); break;
   }
-  double *Pt = P + (int64_t)item * TT * TT;
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = wi * 64 + a * 16 + acc_row<double>(lane, r);
-        const int j = wj * 64 + b * 16 + (lane & 15);
-        Pt[i + (int64_t)j * TT] = acc[a][b][r];
-      }
 }
 
 // C[I + i + (J + j) ldc] = sum over chunks of the partial tiles (chunk order)
-__global__ void gram_reduce_kernel(const double *P, const int2 *tiles, int ntiles, int nchunks,
-                                   int m, int n, double *C, int64_t ldc) {
-  const int t = blockIdx.y;
+__global__ void gram_reduce_kernel(const double *P, const GramItem *tiles, int m, int n, double *C,
+                                   int64_t ldc) {
+  const GramItem t = tiles[blockIdx.y];
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= TT * TT) return;
   const int i = e % TT, j = e / TT;
-  const int gi = tiles[t].x * TT + i, gj = tiles[t].y * TT + j;
+  const int gi = t.I * TT + i, gj = t.J * TT + j;
   if (gi >= m || gj >= n) return;
   double s = 0.0;
-  for (int c = 0; c < nchunks; ++c) s += P[((int64_t)c * ntiles + t) * TT * TT + e];
+  for (int c = 0; c < t.nslab; ++c) s += P[(int64_t)(t.part + c) * TT * TT + e];
   C[gi + (int64_t)gj * ldc] = s;
 }
 
+// Rows of R past diag + 16 (column / 16) + 15 hold zeros: those blocks are left out.
+//
 // Y[k, J + j] = sum_{i < K} X[k, i] R[i, J + j] for the rows [r0, r0 + rows)
 // of the panel and J + j < N; R[i][j] = Rm[i + j ldr] (TR = 0) or
 // Rm[j + i ldr] (TR = 1).  LDS slabs: X as [128 rows][KS + 1] (odd stride:
@@ -169,7 +207,7 @@ __global__ void gram_reduce_kernel(const double *P, const int2 *tiles, int ntile
 template <int TR, bool VEC>
 __global__ __launch_bounds__(NT, 2) void rotate_kernel(const double *X, int64_t ldx,
                                                        const double *Rm, int64_t ldr, int K,
-                                                       int N, int64_t rows, double *Y,
+                                                       int diag, int N, int64_t rows, double *Y,
                                                        int64_t ldy, int ntj, int per_xcd,
                                                        int nitems) {
   constexpr int XS = KS + 1;
@@ -221,47 +259,58 @@ __global__ __launch_bounds__(NT, 2) void rotate_kernel(const double *X, int64_t 
     }
   };
 
-  f64x4 acc[4][4];
+  // slabs whose rows of R reach column block c end at (diag + J) / 16 + c + 1
+  constexpr int RK = TR ? TT + PADW : 1, RB = TR ? 1 : XS;
+  const int dslab = diag >= K ? nslab : (diag + J + KS - 1) / KS;
+  auto run = [&](auto form) {
+    constexpr unsigned MASK = decltype(form)::value;
+    f64x4 acc[4][4];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < 4; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = f64x4{0, 0, 0, 0};
-  load(0);
-  store(0, 0);
-  __syncthreads();
-  for (int s = 0; s < nslab; ++s) {
-    const int buf = s & 1;
-    if (s + 1 < nslab) load((s + 1) * KS);
-#pragma unroll
-    for (int kk = 0; kk < KS / 4; ++kk) {
-      const int k = kk * 4 + (lane >> 4);
-      double av[4], bv[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int c = q * 16 + (lane & 15);
-        av[q] = Xs[buf][(wi * 64 + c) * XS + k];
-        bv[q] = TR ? Rs[buf][k * (TT + PADW) + wj * 64 + c] : Rs[buf][(wj * 64 + c) * XS + k];
-      }
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = mfma16(av[a], bv[b], acc[a][b]);
-    }
-    if (s + 1 < nslab) store(buf ^ 1, (s + 1) * KS);
+      for (int b = 0; b < 4; ++b) acc[a][b] = f64x4{0, 0, 0, 0};
+    load(0);
+    store(0, 0);
     __syncthreads();
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t k = R0 + wi * 64 + a * 16 + acc_row<double>(lane, r);
-      if (k >= rows) continue;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int j = J + wj * 64 + b * 16 + (lane & 15);
-        if (j < N) Y[k * ldy + j] = acc[a][b][r];
+    auto upto = [&](auto part, int s, int end) {
+      end = end < nslab ? end : nslab;
+      for (; s < end; ++s) {
+        const int buf = s & 1;
+        if (s + 1 < nslab) load((s + 1) * KS);
+        blocks<MASK & decltype(part)::value, 1, XS, RK, RB>(
+            &Xs[buf][(wi * 16 + (lane & 15)) * XS + (lane >> 4)],
+            TR ? &Rs[buf][(lane >> 4) * (TT + PADW) + wj * 16 + (lane & 15)]
+               : &Rs[buf][(wj * 16 + (lane & 15)) * XS + (lane >> 4)],
+            acc);
+        if (s + 1 < nslab) store(buf ^ 1, (s + 1) * KS);
+        __syncthreads();
       }
+    };
+    upto(std::integral_constant<unsigned, 0xffff>{}, 0, diag >= K ? nslab : dslab + 2);
+    if (diag < K) {
+      upto(std::integral_constant<unsigned, 0xeeee>{}, dslab + 2, dslab + 4);
+      upto(std::integral_constant<unsigned, 0xcccc>{}, dslab + 4, dslab + 6);
+      upto(std::integral_constant<unsigned, 0x8888>{}, dslab + 6, dslab + 8);
     }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t k = R0 + (2 * a + wi) * 16 + acc_row<double>(lane, r);
+        if (k >= rows) continue;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int j = J + (2 * b + wj) * 16 + (lane & 15);
+          if (j < N) Y[k * ldy + j] = acc[a][b][r];
+        }
+      }
+  };
+  switch (N - J > 96 ? 3 : (N - J - 1) / 32) {
+    case 0: run(std::integral_constant<unsigned, kColumnForm[0]>{}); break;
+    case 1: run(std::integral_constant<unsigned, kColumnForm[1]>{}); break;
+    case 2: run(std::integral_constant<unsigned, kColumnForm[2]>{}); break;
+    default: run(std::integral_constant<unsigned, kColumnForm[3]>{}); break;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -273,54 +322,84 @@ static bool pairs(const double *p, int64_t ld, int n) {
   return ld % 2 == 0 && ((uintptr_t)p & 15) == 0 && n % 2 == 0;
 }
 
-static int64_t gram_chunk_rows(int64_t K, int ntiles) {
-  // at most one wave of work items over the chip's 512 workgroup slots (256
-  // CUs, two workgroups each): a second, partial wave would double the time.
-  // Chunks of at least 4096 rows, at most 256 chunks.
-  int64_t nch = 512 / ntiles;
-  nch = nch < 1 ? 1 : (nch > 256 ? 256 : nch);
-  int64_t kc = (K + nch - 1) / nch;
-  if (kc < 4096) kc = 4096;
-  return (kc + KS - 1) / KS * KS;
-}
-
-static std::vector<int2> gram_tiles(int m, int n, int diag_off) {
-  std::vector<int2> t;
+// Work items of a gram call and, per tile, its partial sums.  At most one wave of
+// items over the chip's 512 workgroup slots (256 CUs, two workgroups each): a second,
+// partial wave would double the time.  A tile whose waves multiply fewer blocks (diagonal,
+// edge) gets longer chunks, so that the items end together; chunks of at least 4096
+// rows, at most 256 of them.  (216k rows, whole CholGS in ms, every block of every tile
+// on equal chunks / so: 500 columns 4.94 / 4.73, 333 columns 3.60 / 3.35.)
+static void gram_plan(int64_t K, int m, int n, int diag_off, std::vector<GramItem> *items,
+                      std::vector<GramItem> *tiles) {
   const int tm = (m + TT - 1) / TT, tn = (n + TT - 1) / TT;
+  items->clear();
+  tiles->clear();
+  std::vector<int> load;  // blocks of a wave, and 2 for the staging
+  int sum = 0;
   for (int J = 0; J < tn; ++J)
     for (int I = 0; I < tm; ++I)
-      if (diag_off < 0 || (I + 1) * TT - 1 >= J * TT + diag_off) t.push_back(int2{I, J});
-  return t;
+      if (diag_off < 0 || (I + 1) * TT - 1 >= J * TT + diag_off) {
+        const int most = __builtin_popcount(kGramForm[gram_form(I * TT, J * TT, m, diag_off)]);
+        tiles->push_back(GramItem{I, J, 0, 0, 0});
+        load.push_back(most + 2);
+        sum += most + 2;
+      }
+  const int nt = (int)tiles->size();
+  if (nt == 0 || K <= 0) return;
+  // slabs of a chunk of load 18, grown until the items fit
+  const int64_t slabs = (K + KS - 1) / KS;
+  auto chunk = [&](int t, int64_t full) {
+    return std::max<int64_t>({full * 18 / load[t], (slabs + 255) / 256, 4096 / KS});
+  };
+  int64_t full = std::max<int64_t>(1, slabs * sum / (18 * 512));
+  for (;; full += std::max<int64_t>(1, full / 256)) {
+    int64_t count = 0;
+    for (int t = 0; t < nt; ++t) {
+      const int64_t c = chunk(t, full);
+      count += (slabs + c - 1) / c;
+    }
+    if (count <= std::max(512, nt)) break;
+  }
+  for (int t = 0; t < nt; ++t) {
+    const int64_t c = chunk(t, full);
+    const int nch = (int)((slabs + c - 1) / c);
+    GramItem &tl = (*tiles)[t];
+    tl.part = (int)items->size();
+    tl.nslab = nch;
+    for (int j = 0; j < nch; ++j)
+      items->push_back(GramItem{tl.I, tl.J, (int)(j * c), (int)std::min(c, slabs - j * c),
+                                tl.part + j});
+  }
+  // items that start on the same rows next to each other: they share an XCD's L2
+  std::stable_sort(items->begin(), items->end(),
+                   [](const GramItem &x, const GramItem &y) { return x.slab < y.slab; });
 }
 
 size_t gram_partial_bytes(int64_t K, int m, int n, int diag_off) {
-  const int nt = (int)gram_tiles(m, n, diag_off).size();
-  if (nt == 0) return 0;
-  const int64_t kc = gram_chunk_rows(K, nt);
-  const int64_t nch = (K + kc - 1) / kc;
-  return sizeof(double) * (size_t)nch * nt * TT * TT;
+  std::vector<GramItem> items, tiles;
+  gram_plan(K, m, n, diag_off, &items, &tiles);
+  return sizeof(double) * items.size() * TT * TT;
 }
 
 hipError_t launch_gram(const double *A, int64_t lda, const double *B, int64_t ldb, int m, int n,
                        int64_t K, int diag_off, double *C, int64_t ldc, double *P,
-                       int2 *tiles_dev, hipStream_t s) {
-  const std::vector<int2> t = gram_tiles(m, n, diag_off);
-  const int nt = (int)t.size();
-  if (nt == 0 || K <= 0) return hipSuccess;
-  if (nt > kGramMaxTiles) return hipErrorInvalidValue;
-  hipError_t e = hipMemcpyAsync(tiles_dev, t.data(), sizeof(int2) * nt, hipMemcpyHostToDevice, s);
+                       GramItem *table_dev, hipStream_t s) {
+  std::vector<GramItem> items, tiles;
+  gram_plan(K, m, n, diag_off, &items, &tiles);
+  const int nt = (int)tiles.size(), nitems = (int)items.size();
+  if (nitems == 0) return hipSuccess;
+  if (nt > kGramMaxTiles || nt + nitems > kGramMaxTable) return hipErrorInvalidValue;
+  tiles.insert(tiles.end(), items.begin(), items.end());
+  hipError_t e = hipMemcpyAsync(table_dev, tiles.data(), sizeof(GramItem) * tiles.size(),
+                                hipMemcpyHostToDevice, s);
   if (e != hipSuccess) return e;
-  const int64_t kc = gram_chunk_rows(K, nt);
-  const int nch = (int)((K + kc - 1) / kc);
-  const int nitems = nch * nt;
   const int per_xcd = (nitems + 7) / 8;
   const bool vec = pairs(A, lda, m) && pairs(B, ldb, n);
   hipLaunchKernelGGL((vec ? gram_kernel<true> : gram_kernel<false>), dim3(8 * per_xcd), dim3(NT),
-                     0, s, A, lda, B, ldb, m, n, K, kc, tiles_dev, nt, per_xcd, nitems, P);
+                     0, s, A, lda, B, ldb, m, n, K, diag_off, table_dev + nt, per_xcd, nitems, P);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(gram_reduce_kernel, dim3(TT * TT / 256, nt), dim3(256), 0, s, P, tiles_dev, nt,
-                     nch, m, n, C, ldc);
+  hipLaunchKernelGGL(gram_reduce_kernel, dim3(TT * TT / 256, nt), dim3(256), 0, s, P, table_dev, m,
+                     n, C, ldc);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   // the host table is read by the copy above before this call returns
@@ -328,7 +407,7 @@ hipError_t launch_gram(const double *A, int64_t lda, const double *B, int64_t ld
 }
 
 hipError_t launch_rotate(const double *X, int64_t ldx, const double *Rm, int64_t ldr, int trans,
-                         int K, int N, int64_t rows, double *Y, int64_t ldy, hipStream_t s) {
+                         int K, int diag, int N, int64_t rows, double *Y, int64_t ldy, hipStream_t s) {
   if (rows <= 0 || N <= 0 || K <= 0) return hipSuccess;
   const int ntj = (N + TT - 1) / TT;
   const int64_t nti = (rows + TT - 1) / TT;
@@ -339,7 +418,7 @@ hipError_t launch_rotate(const double *X, int64_t ldx, const double *Rm, int64_t
   const bool vec = pairs(X, ldx, K) && pairs(Rm, ldr, trans ? N : K);
   hipLaunchKernelGGL((trans ? (vec ? rotate_kernel<1, true> : rotate_kernel<1, false>)
                             : (vec ? rotate_kernel<0, true> : rotate_kernel<0, false>)),
-                     dim3(8 * per_xcd), dim3(NT), 0, s, X, ldx, Rm, ldr, K, N, rows, Y, ldy, ntj,
+                     dim3(8 * per_xcd), dim3(NT), 0, s, X, ldx, Rm, ldr, K, diag, N, rows, Y, ldy, ntj,
                      per_xcd, nitems);
   return hipGetLastError();
 }

@@ -463,9 +463,9 @@ chfsi_status gram_fp64(chfsi_solver *s, const double *A, int64_t lda, const doub
   const size_t pb = gram_partial_bytes(M, m, n, diag_off);
   if (pb == 0) return CHFSI_OK;
   CHFSI_TRY(s->split.ensure(pb));
-  CHFSI_TRY(s->gtiles.ensure(sizeof(int2) * kGramMaxTiles));
+  CHFSI_TRY(s->gtiles.ensure(sizeof(GramItem) * kGramMaxTable));
   CHFSI_HIP(launch_gram(A, lda, B, ldb, m, n, M, diag_off, C, ldc, sptr<double>(s->split),
-                        static_cast<int2 *>(s->gtiles.ptr), st));
+                        static_cast<GramItem *>(s->gtiles.ptr), st));
   return CHFSI_OK;
 }
 
@@ -506,10 +506,11 @@ chfsi_status rotate_fp64(chfsi_solver *s, double *X, int64_t M, int N, const dou
         const int bw = std::min(CB, N - c0);
         // R(i, c0 + j): Rm[c0 + j + i ldr] (trans) or Rm[i + (c0 + j) ldr]
         const double *Rc = trans ? Rm + c0 : Rm + (int64_t)c0 * ldr;
-        CHFSI_HIP(launch_rotate(X + n0 * N, N, Rc, ldr, trans, c0 + bw, bw, nc, tmp + c0, N, st));
+        CHFSI_HIP(launch_rotate(X + n0 * N, N, Rc, ldr, trans, c0 + bw, c0, bw, nc, tmp + c0, N,
+                                st));
       }
     } else {
-      CHFSI_HIP(launch_rotate(X + n0 * N, N, Rm, ldr, trans, N, N, nc, tmp, N, st));
+      CHFSI_HIP(launch_rotate(X + n0 * N, N, Rm, ldr, trans, N, N, N, nc, tmp, N, st));
     }
     CHFSI_HIP(hipEventRecord(s->rot_done[b], st));
     CHFSI_HIP(hipStreamWaitEvent(s->copy_stream, s->rot_done[b], 0));
