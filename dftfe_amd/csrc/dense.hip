@@ -30,6 +30,7 @@ namespace {
 constexpr int TT = 128;   // output tile edge
 constexpr int KS = 16;    // K rows per LDS slab
 constexpr int NT = 256;   // 4 waves (wi, wj): blocks of 16 (2a + wi, 2b + wj), a, b < 4
+constexpr int kMinRows = 1024;  // of a gram chunk
 constexpr int PADW = 16;  // LDS row padding of [k][128] slabs (doubles)
 
 // Work items are spread over the 8 XCDs so that consecutive items (the tiles
@@ -74,14 +75,14 @@ __host__ __device__ inline int gram_form(int I, int J, int m, int diag_off) {
   return na + (diag_off >= 0 && J + diag_off >= I ? 1 : 0);
 }
 
-// Entries c .. c + 7 of a row of n into r, those past its end read from entry 0.
+// Pairs c + STEP e of a row of n into r, entries past its end read from entry 0.
 // VEC: 16-byte loads (rows 16-byte aligned, c and n even, so that a pair lies
 // inside or outside the row).
-template <bool VEC>
+template <bool VEC, int STEP>
 __device__ __forceinline__ void load8(const double *row, int c, int n, double2 (&r)[4]) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int i = c + 2 * e;
+    const int i = c + STEP * e;
     if (VEC)
       r[e] = *reinterpret_cast<const double2 *>(row + (i < n ? i : 0));
     else
@@ -116,25 +117,25 @@ __global__ __launch_bounds__(NT, 2) void gram_kernel(const double *A, int64_t ld
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wi = w & 1, wj = w >> 1;
 
-  // staging: thread t loads row t/16 of the slab, 8 consecutive columns.  Indices
-  // past the block are clamped and the values dropped when they are stored, so
+  // staging: thread t loads row t/16 of the slab, the column pairs 2 (t%16) + 32 e (16
+  // lanes a line of memory and all banks of LDS).  Indices past the block are clamped and the values dropped when they are stored, so
   // nothing waits for a load before the MFMAs of the slab in between.
-  const int lr = tid >> 4, lc = (tid & 15) * 8;
+  const int lr = tid >> 4, lc = (tid & 15) * 2;
   double2 ra[4], rb[4];
   auto load = [&](int64_t k0) {
     const int64_t k = k0 + lr < ke ? k0 + lr : ke - 1;
     const double *ap = A + k * lda, *bp = B + k * ldb;
-    load8<VEC>(ap, I + lc, m, ra);
-    load8<VEC>(bp, J + lc, n, rb);
+    load8<VEC, 32>(ap, I + lc, m, ra);
+    load8<VEC, 32>(bp, J + lc, n, rb);
   };
   auto store = [&](int buf, int64_t k0) {
     const bool kok = k0 + lr < ke;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int i = I + lc + 2 * e, j = J + lc + 2 * e;
-      *reinterpret_cast<double2 *>(&As[buf][lr][lc + 2 * e]) =
+      const int i = I + lc + 32 * e, j = J + lc + 32 * e;
+      *reinterpret_cast<double2 *>(&As[buf][lr][lc + 32 * e]) =
           double2{kok & (i < m) ? ra[e].x : 0.0, kok & (i + 1 < m) ? ra[e].y : 0.0};
-      *reinterpret_cast<double2 *>(&Bs[buf][lr][lc + 2 * e]) =
+      *reinterpret_cast<double2 *>(&Bs[buf][lr][lc + 32 * e]) =
           double2{kok & (j < n) ? rb[e].x : 0.0, kok & (j + 1 < n) ? rb[e].y : 0.0};
     }
   };
@@ -226,17 +227,17 @@ __global__ __launch_bounds__(NT, 2) void rotate_kernel(const double *X, int64_t 
   // X slab: thread t takes row t/2, HK consecutive columns from HK*(t%2)
   const int xr = tid >> 1, xc = (tid & 1) * HK;
   double2 rx[HK / 2], rr[HK / 2];
-  // row of X; row (TR = 1: i0 + t/16, 8 consecutive columns) or column (TR = 0: J + t/2,
+  // row of X; row (TR = 1: i0 + t/16, the pairs 2 (t%16) + 32 e) or column (TR = 0: J + t/2,
   // HK consecutive rows) of R.  As in gram_kernel, clamped and dropped at the store.
   const double *xp = X + (R0 + xr < rows ? R0 + xr : 0) * ldx;
   const int rm = TR ? tid >> 4 : J + (tid >> 1);
-  const int rc = TR ? J + (tid & 15) * 8 : xc;
+  const int rc = TR ? J + (tid & 15) * 2 : xc;
   auto load = [&](int i0) {
-    load8<VEC>(xp, i0 + xc, K, rx);
+    load8<VEC, 2>(xp, i0 + xc, K, rx);
     if (TR)
-      load8<VEC>(Rm + (int64_t)(i0 + rm < K ? i0 + rm : 0) * ldr, rc, N, rr);
+      load8<VEC, 32>(Rm + (int64_t)(i0 + rm < K ? i0 + rm : 0) * ldr, rc, N, rr);
     else
-      load8<VEC>(Rm + (int64_t)(rm < N ? rm : 0) * ldr, i0 + rc, K, rr);
+      load8<VEC, 2>(Rm + (int64_t)(rm < N ? rm : 0) * ldr, i0 + rc, K, rr);
   };
   auto store = [&](int buf, int i0) {
     const bool kok = R0 + xr < rows;
@@ -248,7 +249,7 @@ __global__ __launch_bounds__(NT, 2) void rotate_kernel(const double *X, int64_t 
       x[1] = kok & (i + 1 < K) ? rx[e].y : 0.0;
       if (TR) {
         const bool iok = i0 + rm < K;
-        const int j = rc + 2 * e;
+        const int j = rc + 32 * e;
         *reinterpret_cast<double2 *>(&Rs[buf][rm * (TT + PADW) + j - J]) =
             double2{iok & (j < N) ? rr[e].x : 0.0, iok & (j + 1 < N) ? rr[e].y : 0.0};
       } else {
@@ -348,7 +349,7 @@ static void gram_plan(int64_t K, int m, int n, int diag_off, std::vector<GramIte
   // slabs of a chunk of load 18, grown until the items fit
   const int64_t slabs = (K + KS - 1) / KS;
   auto chunk = [&](int t, int64_t full) {
-    return std::max<int64_t>({full * 18 / load[t], (slabs + 255) / 256, 4096 / KS});
+    return std::max<int64_t>({full * 18 / load[t], (slabs + 255) / 256, kMinRows / KS});
   };
   int64_t full = std::max<int64_t>(1, slabs * sum / (18 * 512));
   for (;; full += std::max<int64_t>(1, full / 256)) {
