@@ -30,7 +30,7 @@ namespace {
 constexpr int TT = 128;   // output tile edge
 constexpr int KS = 16;    // K rows per LDS slab
 constexpr int NT = 256;   // 4 waves (wi, wj): blocks of 16 (2a + wi, 2b + wj), a, b < 4
-constexpr int kMinRows = 1024;  // of a gram chunk
+constexpr int kMinRows = 512;  // of a gram chunk
 constexpr int PADW = 16;  // LDS row padding of [k][128] slabs (doubles)
 
 // Work items are spread over the 8 XCDs so that consecutive items (the tiles
@@ -75,18 +75,32 @@ __host__ __device__ inline int gram_form(int I, int J, int m, int diag_off) {
   return na + (diag_off >= 0 && J + diag_off >= I ? 1 : 0);
 }
 
-// Pairs c + STEP e of a row of n into r, entries past its end read from entry 0.
+// Pairs c + 32 e of a row of n into r, entries past its end read from entry 0.
 // VEC: 16-byte loads (rows 16-byte aligned, c and n even, so that a pair lies
 // inside or outside the row).
-template <bool VEC, int STEP>
+template <bool VEC>
 __device__ __forceinline__ void load8(const double *row, int c, int n, double2 (&r)[4]) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int i = c + STEP * e;
+    const int i = c + 32 * e;
     if (VEC)
       r[e] = *reinterpret_cast<const double2 *>(row + (i < n ? i : 0));
     else
       r[e] = double2{row[i < n ? i : 0], row[i + 1 < n ? i + 1 : 0]};
+  }
+}
+
+// Pair c of the rows r0 + 32 e of n entries, those past the last row read from row 0.
+template <bool VEC>
+__device__ __forceinline__ void load_rows(const double *M, int64_t ld, int64_t r0, int64_t rows,
+                                          int c, int n, double2 (&r)[4]) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const double *row = M + (r0 + 32 * e < rows ? r0 + 32 * e : 0) * ld;
+    if (VEC)
+      r[e] = *reinterpret_cast<const double2 *>(row + (c < n ? c : 0));
+    else
+      r[e] = double2{row[c < n ? c : 0], row[c + 1 < n ? c + 1 : 0]};
   }
 }
 
@@ -125,8 +139,8 @@ __global__ __launch_bounds__(NT, 2) void gram_kernel(const double *A, int64_t ld
   auto load = [&](int64_t k0) {
     const int64_t k = k0 + lr < ke ? k0 + lr : ke - 1;
     const double *ap = A + k * lda, *bp = B + k * ldb;
-    load8<VEC, 32>(ap, I + lc, m, ra);
-    load8<VEC, 32>(bp, J + lc, n, rb);
+    load8<VEC>(ap, I + lc, m, ra);
+    load8<VEC>(bp, J + lc, n, rb);
   };
   auto store = [&](int buf, int64_t k0) {
     const bool kok = k0 + lr < ke;
@@ -213,7 +227,6 @@ __global__ __launch_bounds__(NT, 2) void rotate_kernel(const double *X, int64_t 
                                                        int nitems) {
   constexpr int XS = KS + 1;
   constexpr int RSZ = TR ? KS * (TT + PADW) : TT * XS;
-  constexpr int HK = KS / 2;  // doubles per thread and row of a slab
   __shared__ __align__(16) double Xs[2][TT * XS];
   __shared__ __align__(16) double Rs[2][RSZ];
   const int item = xcd_item(per_xcd);
@@ -224,38 +237,37 @@ __global__ __launch_bounds__(NT, 2) void rotate_kernel(const double *X, int64_t 
   const int wi = w & 1, wj = w >> 1;
   const int nslab = (K + KS - 1) / KS;
 
-  // X slab: thread t takes row t/2, HK consecutive columns from HK*(t%2)
-  const int xr = tid >> 1, xc = (tid & 1) * HK;
-  double2 rx[HK / 2], rr[HK / 2];
-  // row of X; row (TR = 1: i0 + t/16, the pairs 2 (t%16) + 32 e) or column (TR = 0: J + t/2,
-  // HK consecutive rows) of R.  As in gram_kernel, clamped and dropped at the store.
-  const double *xp = X + (R0 + xr < rows ? R0 + xr : 0) * ldx;
-  const int rm = TR ? tid >> 4 : J + (tid >> 1);
-  const int rc = TR ? J + (tid & 15) * 2 : xc;
+  // X slab: thread t takes the rows t/8 + 32 e and one column pair (8 lanes a line); R
+  // slab: TR = 1 row t/16 and the column pairs 2 (t%16) + 32 e, TR = 0 columns t/8 + 32 e
+  // and one row pair.  As in gram_kernel, clamped and dropped at the store.
+  const int xr = tid >> 3, xc = (tid & 7) * 2;
+  const int rm = TR ? tid >> 4 : xr, rc = TR ? (tid & 15) * 2 : xc;
+  double2 rx[4], rr[4];
   auto load = [&](int i0) {
-    load8<VEC, 2>(xp, i0 + xc, K, rx);
+    load_rows<VEC>(X, ldx, R0 + xr, rows, i0 + xc, K, rx);
     if (TR)
-      load8<VEC, 32>(Rm + (int64_t)(i0 + rm < K ? i0 + rm : 0) * ldr, rc, N, rr);
+      load8<VEC>(Rm + (int64_t)(i0 + rm < K ? i0 + rm : 0) * ldr, J + rc, N, rr);
     else
-      load8<VEC, 2>(Rm + (int64_t)(rm < N ? rm : 0) * ldr, i0 + rc, K, rr);
+      load_rows<VEC>(Rm, ldr, J + rm, N, i0 + rc, K, rr);
   };
   auto store = [&](int buf, int i0) {
-    const bool kok = R0 + xr < rows;
+    const bool i0ok = i0 + xc < K, i1ok = i0 + xc + 1 < K;
 #pragma unroll
-    for (int e = 0; e < HK / 2; ++e) {
-      const int i = i0 + xc + 2 * e;
-      double *x = &Xs[buf][xr * XS + xc + 2 * e];
-      x[0] = kok & (i < K) ? rx[e].x : 0.0;
-      x[1] = kok & (i + 1 < K) ? rx[e].y : 0.0;
+    for (int e = 0; e < 4; ++e) {
+      const bool kok = R0 + xr + 32 * e < rows;
+      double *x = &Xs[buf][(xr + 32 * e) * XS + xc];
+      x[0] = kok & i0ok ? rx[e].x : 0.0;
+      x[1] = kok & i1ok ? rx[e].y : 0.0;
       if (TR) {
         const bool iok = i0 + rm < K;
-        const int j = rc + 32 * e;
-        *reinterpret_cast<double2 *>(&Rs[buf][rm * (TT + PADW) + j - J]) =
+        const int j = J + rc + 32 * e;
+        *reinterpret_cast<double2 *>(&Rs[buf][rm * (TT + PADW) + rc + 32 * e]) =
             double2{iok & (j < N) ? rr[e].x : 0.0, iok & (j + 1 < N) ? rr[e].y : 0.0};
       } else {
-        double *r = &Rs[buf][(rm - J) * XS + xc + 2 * e];
-        r[0] = (rm < N) & (i < K) ? rr[e].x : 0.0;
-        r[1] = (rm < N) & (i + 1 < K) ? rr[e].y : 0.0;
+        const bool jok = J + rm + 32 * e < N;
+        double *r = &Rs[buf][(rm + 32 * e) * XS + xc];
+        r[0] = jok & i0ok ? rr[e].x : 0.0;
+        r[1] = jok & i1ok ? rr[e].y : 0.0;
       }
     }
   };
