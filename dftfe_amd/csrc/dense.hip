@@ -27,10 +27,12 @@ namespace chfsi {
 
 namespace {
 
-constexpr int TT = 128;   // output tile edge
+constexpr int TT = kRotateTile;  // output tile edge
 constexpr int KS = 16;    // K rows per LDS slab
 constexpr int NT = 256;   // 4 waves (wi, wj): blocks of 16 (2a + wi, 2b + wj), a, b < 4
-constexpr int kMinRows = 512;  // of a gram chunk
+// rows of a gram chunk at least: gram of 64 columns on 110k rows 0.49 ms with 4096, 0.20
+// with 1024, 0.13 with 512, 0.14 with 256
+constexpr int kMinRows = 512;
 constexpr int PADW = 16;  // LDS row padding of [k][128] slabs (doubles)
 
 // Work items are spread over the 8 XCDs so that consecutive items (the tiles
@@ -90,17 +92,17 @@ __device__ __forceinline__ void load8(const double *row, int c, int n, double2 (
   }
 }
 
-// Pair c of the rows r0 + 32 e of n entries, those past the last row read from row 0.
+// Pair c of the rows r0 + r + 32 e of n entries, those past the last row read from row r0.
 template <bool VEC>
-__device__ __forceinline__ void load_rows(const double *M, int64_t ld, int64_t r0, int64_t rows,
-                                          int c, int n, double2 (&r)[4]) {
+__device__ __forceinline__ void load_rows(const double *M, int64_t ld, int64_t r0, int r,
+                                          int64_t rows, int c, int n, double2 (&v)[4]) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const double *row = M + (r0 + 32 * e < rows ? r0 + 32 * e : 0) * ld;
+    const double *row = M + (r0 + r + 32 * e < rows ? r0 + r + 32 * e : r0) * ld;
     if (VEC)
-      r[e] = *reinterpret_cast<const double2 *>(row + (c < n ? c : 0));
+      v[e] = *reinterpret_cast<const double2 *>(row + (c < n ? c : 0));
     else
-      r[e] = double2{row[c < n ? c : 0], row[c + 1 < n ? c + 1 : 0]};
+      v[e] = double2{row[c < n ? c : 0], row[c + 1 < n ? c + 1 : 0]};
   }
 }
 
@@ -109,7 +111,7 @@ __device__ __forceinline__ void load_rows(const double *M, int64_t ld, int64_t r
 // Bound by the FP64 matrix cores.  The loads of slab s + 1 are issued before the MFMAs
 // of slab s and first used when they are stored behind them; with the masks applied
 // at the load every slab waited for them (500 columns on 216k rows: 1.77 ms, then 1.39;
-// 1.33 with the blocks below).
+// 1.33 with the blocks below, 1.19 with whole lines staged and shorter chunks).
 //
 // C_tile(I, J) = sum_{k in chunk} A[k, I + i] B[k, J + j], written to
 // P[part][i + 128 j].  Blocks of 16 past the edge or above the diagonal are left out
@@ -244,11 +246,11 @@ __global__ __launch_bounds__(NT, 2) void rotate_kernel(const double *X, int64_t 
   const int rm = TR ? tid >> 4 : xr, rc = TR ? (tid & 15) * 2 : xc;
   double2 rx[4], rr[4];
   auto load = [&](int i0) {
-    load_rows<VEC>(X, ldx, R0 + xr, rows, i0 + xc, K, rx);
+    load_rows<VEC>(X, ldx, R0, xr, rows, i0 + xc, K, rx);
     if (TR)
       load8<VEC>(Rm + (int64_t)(i0 + rm < K ? i0 + rm : 0) * ldr, J + rc, N, rr);
     else
-      load_rows<VEC>(Rm, ldr, J + rm, N, i0 + rc, K, rr);
+      load_rows<VEC>(Rm, ldr, J, rm, N, i0 + rc, K, rr);
   };
   auto store = [&](int buf, int i0) {
     const bool i0ok = i0 + xc < K, i1ok = i0 + xc + 1 < K;
@@ -338,7 +340,7 @@ static bool pairs(const double *p, int64_t ld, int n) {
 // Work items of a gram call and, per tile, its partial sums.  At most one wave of
 // items over the chip's 512 workgroup slots (256 CUs, two workgroups each): a second,
 // partial wave would double the time.  A tile whose waves multiply fewer blocks (diagonal,
-// edge) gets longer chunks, so that the items end together; chunks of at least 4096
+// edge) gets longer chunks, so that the items end together; chunks of at least kMinRows
 // rows, at most 256 of them.  (216k rows, whole CholGS in ms, every block of every tile
 // on equal chunks / so: 500 columns 4.94 / 4.73, 333 columns 3.60 / 3.35.)
 static void gram_plan(int64_t K, int m, int n, int diag_off, std::vector<GramItem> *items,

@@ -32,9 +32,13 @@ hipError_t launch_gram(const double *A, int64_t lda, const double *B, int64_t ld
                        GramItem *table_dev, hipStream_t s);
 size_t gram_partial_bytes(int64_t K, int m, int n, int diag_off);
 
+// column tile of the rotation kernel
+constexpr int kRotateTile = 128;
+
 // Y[k ldy + j] = sum_{i < K} X[k ldx + i] R(i, j) for k < rows, j < N, with
 // R(i, j) = Rm[i + j ldr] (trans = 0) or Rm[j + i ldr] (trans = 1).  R(i, j) is zero
-// for i > diag + j (diag >= K: none need be).  Y must not overlap X.
+// for i > diag + j (diag >= K: none need be).  Y must not overlap X unless N <= kRotateTile
+// and Y's columns are among the K of X (row for row: in place).
 hipError_t launch_rotate(const double *X, int64_t ldx, const double *Rm, int64_t ldr, int trans,
                          int K, int diag, int N, int64_t rows, double *Y, int64_t ldy, hipStream_t s);
 

@@ -469,19 +469,30 @@ chfsi_status gram_fp64(chfsi_solver *s, const double *A, int64_t lda, const doub
   return CHFSI_OK;
 }
 
-// X <- X R in row panels with the library's FP64 MFMA kernel; R(i, j) =
-// Rm[i + j ldr] (trans 0) or Rm[j + i ldr] (trans 1), upper triangular when upper
-// Panel p is rotated into buffer p % 2 on st; its copy back into X runs on the
-// solver's copy stream while panel p + 1 is rotated (the rotation reads only
-// its own panel of X).  Before panel p + 2 reuses the buffer, st waits for
-// panel p's copy; at the end st waits for every copy.  upper: R is upper
-// triangular with its lower part stored as zeros; the panel is rotated by
-// column blocks of 128, block [c0, c0 + 128) over the inner extent
-// c0 + 128 only, so every launch has work items of one length (CholGS of 500 columns
-// on 216k rows 5.52 ms; blocks of 256: 5.66, which compute 15% more zeros; one launch
-// over all lengths: 6.28).
+// X <- X R with the library's FP64 MFMA kernel; R(i, j) = Rm[i + j ldr] (trans 0) or
+// Rm[j + i ldr] (trans 1), upper triangular when upper.
+// A launch whose output is one column tile is in place: a workgroup reads only its own
+// rows and writes them last.  upper: R's lower part is stored as zeros; X is rotated by
+// column blocks of kRotateTile from the last one down, block [c0, c0 + tile) over the
+// inner extent c0 + tile only: the columns it reads are still unrotated, and every launch
+// has work items of one length.  CholGS of 500 columns on 216k rows, ms: in place 3.95;
+// into a panel buffer and copied back 4.45 (the copy alone 0.55); blocks of 256 and one
+// launch over all lengths were slower by 2% and 13%.
+// Otherwise by row panels: panel p is rotated into buffer p % 2 on st; its copy back
+// into X runs on the solver's copy stream while panel p + 1 is rotated (the rotation
+// reads only its own panel of X).  Before panel p + 2 reuses the buffer, st waits for
+// panel p's copy; at the end st waits for every copy.
 chfsi_status rotate_fp64(chfsi_solver *s, double *X, int64_t M, int N, const double *Rm,
                          int64_t ldr, int trans, int upper, hipStream_t st) {
+  if (upper || N <= kRotateTile) {
+    for (int c0 = (N - 1) / kRotateTile * kRotateTile; c0 >= 0; c0 -= kRotateTile) {
+      const int bw = std::min(kRotateTile, N - c0), K = upper ? c0 + bw : N;
+      // R(i, c0 + j): Rm[c0 + j + i ldr] (trans) or Rm[i + (c0 + j) ldr]
+      const double *Rc = trans ? Rm + c0 : Rm + (int64_t)c0 * ldr;
+      CHFSI_HIP(launch_rotate(X, N, Rc, ldr, trans, K, upper ? c0 : K, bw, M, X + c0, N, st));
+    }
+    return CHFSI_OK;
+  }
   const int64_t chunk = panel_rows(M, N);
   const int64_t npanel = (M + chunk - 1) / chunk;
   const int nbuf = npanel > 1 ? 2 : 1;
@@ -500,18 +511,7 @@ chfsi_status rotate_fp64(chfsi_solver *s, double *X, int64_t M, int N, const dou
     const int64_t n0 = p * chunk, nc = std::min(chunk, M - n0);
     double *tmp = sptr<double>(s->rot) + (int64_t)b * chunk * N;
     if (p >= 2) CHFSI_HIP(hipStreamWaitEvent(st, s->copy_done[b], 0));
-    if (upper) {
-      constexpr int CB = 128;
-      for (int c0 = 0; c0 < N; c0 += CB) {
-        const int bw = std::min(CB, N - c0);
-        // R(i, c0 + j): Rm[c0 + j + i ldr] (trans) or Rm[i + (c0 + j) ldr]
-        const double *Rc = trans ? Rm + c0 : Rm + (int64_t)c0 * ldr;
-        CHFSI_HIP(launch_rotate(X + n0 * N, N, Rc, ldr, trans, c0 + bw, c0, bw, nc, tmp + c0, N,
-                                st));
-      }
-    } else {
-      CHFSI_HIP(launch_rotate(X + n0 * N, N, Rm, ldr, trans, N, N, N, nc, tmp, N, st));
-    }
+    CHFSI_HIP(launch_rotate(X + n0 * N, N, Rm, ldr, trans, N, N, N, nc, tmp, N, st));
     CHFSI_HIP(hipEventRecord(s->rot_done[b], st));
     CHFSI_HIP(hipStreamWaitEvent(s->copy_stream, s->rot_done[b], 0));
     CHFSI_HIP(hipMemcpyAsync(X + n0 * N, tmp, sizeof(double) * nc * N, hipMemcpyDeviceToDevice,
