@@ -206,6 +206,8 @@ def test_all_cells_at_once_equals_colour_launches(case, B, dtype):
     from dftfe_amd.chfsi import chebyshev_filter
 
     prob, ref, op = case
+    for prec in (L.FP64, L.FP32):
+        op.set_proj_variant(prec, 0)  # unset, its tile goes by the width
     wide = 2048                 # 8 cells a colour: 512 (64-bit p = 6: 1024) workgroups
     rng = np.random.default_rng(B)
     X = torch.zeros(prob.M, wide, device="cuda", dtype=dtype)
