@@ -47,14 +47,17 @@ METRIC = "ChFSI pass time + HX GFLOP/s, mixed vs FP64 GPU at 1e-8 Ha eigval erro
 
 
 def hx_flops(prob, B):
-    """Algorithmic flops of one block HX: dense cell GEMMs + C^T X and C (V C^T X)."""
+    """Flops of one block HX with dense cell matrices: cell GEMMs + C^T X and
+    C (V C^T X).  The unit of the reported GFLOP/s whichever form the apply takes
+    (the tensor-product form does about a seventh of them)."""
     return 2.0 * prob.C * prob.ne ** 2 * B + 16.0 * len(prob.pair_cell) * prob.ne * B
 
 
 def hx_bytes(prob, B, s):
-    """Algorithmic HBM bytes of one fused block HX with element size s: read X,
-    read the cell matrices, read+write Y, read the index map."""
-    return prob.M * B * s + prob.C * prob.ne ** 2 * s + 2 * prob.M * B * s + prob.C * prob.ne * 4
+    """Algorithmic HBM bytes of one fused block HX with element size s in the
+    tensor-product form: read X, read the potential at the quadrature points,
+    read+write Y, read the index map."""
+    return prob.M * B * s + prob.C * prob.nqc * s + 2 * prob.M * B * s + prob.C * prob.ne * 4
 
 
 def measured_hx_traffic(workload, width, variant, proj_variant, precision="fp32"):
@@ -445,23 +448,35 @@ def main():
     # BF16 apply: FP32 multivectors (read, read + write Y), BF16 cell matrices
     bf16_bytes = 3 * prob.M * W * 4 + prob.C * prob.ne ** 2 * 2 + prob.C * prob.ne * 4
     bf16_traffic = measured_hx_traffic(args.workload, W, vb, proj32, "bf16")
+    # degrees and quadratures the tensor-product form is built for; it is slower
+    # than every tile form only on wide p = 4 blocks
+    shaped = (prob.wl.p, prob.nqc) in ((5, 6 ** 3), (6, 8 ** 3))
+    tensor = {"fp32": shaped, "fp64": shaped}
+    tile = {k: "tensor" if tensor[k] else tune[k] for k in ("fp32", "fp64")}
+
+    def hx_rate(ms, s, prec):
+        got = hx_bytes(prob, W, s) / ms / 1e6 if tensor[prec] else F / ms / 1e9
+        peak = PEAK_HBM_GBPS if tensor[prec] else PEAK_TFLOPS[prec]
+        return {"achieved": round(got, 2), "peak": peak, "frac": round(got / peak, 4)}
+
     out["roofline"] = {
-        "kernel": f"fused FP32 HX on {W} columns (8 colour launches of tile variant "
-                  f"{tune['fp32']} + projection variant {proj32} + reduction)",
-        "bound": "mfma",
-        "achieved": round(F / hx32_ms / 1e9, 2),
-        "peak": PEAK_TFLOPS["fp32"],
-        "unit": "TFLOP/s",
-        "frac": round(F / hx32_ms / 1e9 / PEAK_TFLOPS["fp32"], 4),
-        "traffic": measured_hx_traffic(args.workload, W, tune["fp32"], proj32),
+        "kernel": f"fused FP32 HX on {W} columns (8 colour launches, "
+                  f"{'tensor-product form' if tensor['fp32'] else 'tile variant %d' % tune['fp32']}"
+                  f" + projection variant {proj32} + reduction)",
+        "bound": "hbm" if tensor["fp32"] else "mfma",
+        **hx_rate(hx32_ms, 4, "fp32"),
+        "unit": "GB/s" if tensor["fp32"] else "TFLOP/s",
+        "traffic": measured_hx_traffic(args.workload, W, tile["fp32"], proj32),
         "traffic_source": f"profiles/hx_traffic_{args.workload}_w{W}.json, FP32 tile variant "
-                          f"{tune['fp32']}, projection variant {proj32} "
+                          f"{tile['fp32']}, projection variant {proj32} "
                           f"(rocprofv3 FETCH_SIZE x2.0 + WRITE_SIZE x1.0)",
         "algorithmic_bytes": hx_bytes(prob, W, 4),
-        "fp64": {"achieved": round(F / hx64_ms / 1e9, 2), "peak": PEAK_TFLOPS["fp64"],
-                 "frac": round(F / hx64_ms / 1e9 / PEAK_TFLOPS["fp64"], 4),
-                 "tile_variant": tune["fp64"], "projection_variant": proj64,
-                 "traffic": measured_hx_traffic(args.workload, W, tune["fp64"], proj64, "fp64")},
+        "dense_tflops": round(F / hx32_ms / 1e9, 2),
+        "fp64": {"bound": "hbm" if tensor["fp64"] else "mfma", **hx_rate(hx64_ms, 8, "fp64"),
+                 "unit": "GB/s" if tensor["fp64"] else "TFLOP/s",
+                 "tile_variant": tile["fp64"], "projection_variant": proj64,
+                 "dense_tflops": round(F / hx64_ms / 1e9, 2),
+                 "traffic": measured_hx_traffic(args.workload, W, tile["fp64"], proj64, "fp64")},
         # the BF16 apply moves FP32 multivectors: its bound is HBM, not the
         # BF16 MFMA rate (the MFMA view is kept beside it)
         "bf16": {"bound": "hbm", "achieved": round(bf16_bytes / hxb_best / 1e6, 1),
@@ -557,9 +572,8 @@ def cell_rebuild(prob, op, log, reps=5):
     """Per-SCF rebuild of every cell Hamiltonian on the device from V_eff JxW
     (LDA) and from V_eff JxW plus the GGA vector (C x n_q x 3), timed with HIP
     events on the stream the library launches on; the LDA matrices of the
-    workload are restored afterwards.  Flops: the executed MFMA work of the
-    symmetric build (16 x 16 node-pair blocks with ib <= jb), 2 per pair and
-    quadrature term, FP64."""
+    workload are restored afterwards.  Rate: bytes of the three
+    copies of the matrices that the build stores."""
     import torch
     from dftfe_amd.chfsi import _ptr, _stream
 
@@ -586,17 +600,12 @@ def cell_rebuild(prob, op, log, reps=5):
         e1.record(st)
         e1.synchronize()
         ms = e0.elapsed_time(e1) / reps
-        # MFMA work the kernel issues: the 16 x 16 node-pair blocks with
-        # ib <= jb (the transposed blocks are written from the same sums),
-        # 2 flops per pair and quadrature term (1 term per point for LDA, 4
-        # for GGA); padding not counted
-        nb = (prob.ne + 15) // 16
-        pairs = nb * (nb + 1) // 2 * 256
-        fl = 2 * pairs * prob.nqc * (1 if name == "lda" else 4) * prob.C
-        tf = fl / ms / 1e9
-        assert tf <= PEAK_TFLOPS["fp64"], f"{name} build rate {tf:.1f} above the FP64 peak"
+        # bytes the build must store: FP64, FP32 and BF16 copies of the padded matrices
+        stored = 14 * prob.C * ((prob.ne + 15) // 16 * 16) ** 2
+        rate = stored / ms / 1e6
+        assert rate <= PEAK_HBM_GBPS, f"{name} build stores {rate:.0f} GB/s, above the HBM peak"
         res[f"{name}_ms"] = round(ms, 3)
-        res[f"{name}_fp64_tflops"] = round(tf, 2)
+        res[f"{name}_store_GBps"] = round(rate, 1)
     op.set_potential(prob.vJxW)
     log(f"cell rebuild: {res}")
     return res
@@ -651,8 +660,8 @@ def density_leg(prob, op, X, log, reps=5):
     e1.record(st)
     e1.synchronize()
     ms = e0.elapsed_time(e1) / reps
-    fl = 2 * prob.C * prob.nqc * prob.ne * N
-    res = {"columns": N, "ms": round(ms, 3), "fp64_tflops": round(fl / ms / 1e9, 2)}
+    # the block read once
+    res = {"columns": N, "ms": round(ms, 3), "GBps": round(8 * prob.M * N / ms / 1e6, 1)}
     log(f"density: {res}")
     return res
 
