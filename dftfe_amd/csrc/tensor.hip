@@ -91,10 +91,10 @@ struct TensorTab {
 };
 
 // FP32 operand tables of the 4 x 4 products: [table][row][column], zero beyond
-// the blocks, then the weights
+// the blocks, then the weights.  L: what K's rounding leaves (see tensor_tables)
 enum {
   kTabIe, kTabIo, kTabIeT, kTabIoT, kTabMe, kTabMo, kTabKx, kTabKxo, kTabKy, kTabKyo, kTabKz,
-  kTabKzo, kTabs
+  kTabKzo, kTabLx, kTabLxo, kTabLy, kTabLyo, kTabLz, kTabLzo, kTabs
 };
 
 bool tensor_shape(int ne, int nqc, int *n, int *q) {
@@ -239,10 +239,14 @@ bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, i
         }
     // FP32: a rounding error of a table acts alike in every cell, so it shifts
     // eigenvalues where the rounding of dense cell matrices averages out.  The
-    // even parts of I (sums = 1) and K (sums = 0) are therefore rounded to a
-    // common grid with their row sums kept exact: a constant is interpolated to
-    // itself and has no kinetic energy.  Smooth states at p = 6: shifts of
-    // 2.6e-6 Ha without, 1e-7 with it, 1e-7 in the dense FP32 product.
+    // even part of I (sums = 1) is therefore rounded with its row sums kept
+    // exact, so that a constant is interpolated to itself, and K (sums = 0)
+    // is kept in two parts, the first with exact zero row sums (a constant has
+    // no kinetic energy), the second the rest.  Plane waves of 0.5-1.2 Ha at
+    // p = 5 and 6 shift by 3-7e-7 Ha with the first part alone (as any state
+    // does, in proportion to its kinetic energy) and by at most 2e-8 with
+    // both, which is the rounding of I, M and the weights; the dense FP32
+    // matrices shift them by up to 1e-7.
     const double *e = tab->data() + at;
     double big = 0;
     for (int x = 0; x < rows_e * NE; ++x) big = std::max(big, std::fabs(e[x]));
@@ -256,8 +260,14 @@ bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, i
       }
       for (int c = 0; c < NE; ++c) {
         float *d = tab32->data() + t32 * 16;
+        const double ev = er[c], od = e[(rows_e + r) * NE + c];
         d[r * 4 + c] = (float)v[c];
-        d[16 + r * 4 + c] = (float)e[(rows_e + r) * NE + c];
+        d[16 + r * 4 + c] = (float)od;
+        if (sums == 0) {
+          float *l = d + (kTabLx - kTabKx) * 16;
+          l[r * 4 + c] = (float)(ev - d[r * 4 + c]);
+          l[16 + r * 4 + c] = (float)(od - d[16 + r * 4 + c]);
+        }
         if (t32 == kTabIe)
           for (int p = 0; p < 2; ++p) d[32 + p * 16 + c * 4 + r] = d[p * 16 + r * 4 + c];
       }
@@ -674,17 +684,19 @@ struct Planes<float, N, Q, TC, PX> {
     const f32x4 z = {0, 0, 0, 0};
     const f32x4 my = operand(kTabMe + s), ky = operand(kTabKy + s);
     const f32x4 mx = operand(kTabMe + PX), kx = operand(kTabKx + PX);
+    const f32x4 ly = operand(kTabLy + s), lx = operand(kTabLx + PX);
     f32x4 m[NE], q[NE];
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       auto l = [&](int j) { return x[s][j][i]; };
       m[i] = mat4<ns>(my, l, z);
-      q[i] = mat4<ns>(ky, l, z);
+      q[i] = mat4<ns>(ky, l, mat4<ns>(ly, l, z));
     }
 #pragma unroll
     for (int j = 0; j < ns; ++j) {
+      auto mj = [&](int i) { return m[i][j]; };
       const f32x4 r = mat4<NX>(mx, [&](int i) { return q[i][j]; },
-                               mat4<NX>(kx, [&](int i) { return m[i][j]; }, z));
+                               mat4<NX>(kx, mj, mat4<NX>(lx, mj, z)));
 #pragma unroll
       for (int i = 0; i < NX; ++i)
         if (act) b[((s ? NE + j : j) * N + (PX ? NE : 0) + i) * TC] = r[i];
@@ -802,8 +814,8 @@ struct Lines<float, N, Q> {
     if constexpr (N & 1) E[NO] = u[NO];
     auto Ek = [&](int k) { return E[k]; };
     auto Ok = [&](int k) { return O[k]; };
-    f32x4 rE = mat4<NE>(operand(kTabKz), Ek, z) * wk;
-    f32x4 rO = mat4<NO>(operand(kTabKzo), Ok, z) * wk;
+    f32x4 rE = mat4<NE>(operand(kTabKz), Ek, mat4<NE>(operand(kTabLz), Ek, z)) * wk;
+    f32x4 rO = mat4<NO>(operand(kTabKzo), Ok, mat4<NO>(operand(kTabLzo), Ok, z)) * wk;
     f32x4 e = mat4<NE>(operand(kTabIe), Ek, z);
     f32x4 o = mat4<NO>(operand(kTabIo), Ok, z);
 #pragma unroll
@@ -885,6 +897,7 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
     for (int r = 0; r < 4; ++r) slot0[r] = gload(a.slot_proj, s0 + 4 * (lane >> 4) + r);
   }
   if constexpr (sizeof(T) == 4) {
+    static_assert(kTabs * 16 + QE <= S::NT, "one table entry per thread");
     if (t < kTabs * 16 + QE) tabs[t] = tabp[t];
   }
 
