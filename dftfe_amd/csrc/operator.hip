@@ -84,7 +84,7 @@ chfsi_operator::~chfsi_operator() {
                   d_ones_cons32, d_own_map, d_own_n, d_nlCto64, d_nlCto32, d_nlCtko64,
                   d_nlCtko32, d_ttab64, d_ttab32, d_tprod, d_touch_ptr, d_touch_idx, d_vq64,
                   d_vq32, d_nlCp64,
-                  d_nlCp32};
+                  d_nlCp32, d_cells_out64, d_cells_out32};
   for (void *p : ptrs)
     if (p) hipFree(p);
   ztab_dev.release();
@@ -95,7 +95,6 @@ chfsi_operator::~chfsi_operator() {
   W64.release();
   W32.release();
   tmp.release();
-  cells_out.release();
 }
 
 extern "C" const char *chfsi_last_error(void) { return g_last_error.c_str(); }
@@ -584,6 +583,16 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
       CHFSI_HIP(launch_tensor_projectors(op->d_nlC64, (int64_t)nlC.size(), op->tn, ne, ne_pad,
                                          op->d_nlCp64, op->d_nlCp32, 0));
     }
+    if (op->d_touch_ptr) {
+      // the cells' sums of an apply on all cells at once, for the widest block
+      // that takes it; without room for them the colour launches run (same bits)
+      auto room = [&](bool fp64) {
+        return size_t(C) * ne * tensor_all_cells_columns(op->tn, fp64, op->max_color_cells);
+      };
+      if (dev_alloc(&op->d_cells_out64, room(true)) != CHFSI_OK ||
+          dev_alloc(&op->d_cells_out32, room(false)) != CHFSI_OK)
+        (void)hipGetLastError();
+    }
     CHFSI_TRY(dev_upload(&op->d_proj_ptr, proj_ptr.data(), proj_ptr.size()));
     CHFSI_TRY(dev_upload(&op->d_proj_slots, proj_slots.data(), proj_slots.size()));
     CHFSI_TRY(dev_upload(&op->d_proj_V, d->proj_V, d->n_proj));
@@ -713,6 +722,7 @@ struct OpData<double> {
   static const double *nlC(chfsi_operator *op) { return op->d_nlC64; }
   static const double *ttab(chfsi_operator *op) { return op->d_ttab64; }
   static const double *vq(chfsi_operator *op) { return op->d_vq64; }
+  static double *cells_out(chfsi_operator *op) { return op->d_cells_out64; }
   static const double *nlCp(chfsi_operator *op) { return op->d_nlCp64; }
   static const double *nlCt(chfsi_operator *op) { return op->d_nlCt64; }
   static const double *nlCto(chfsi_operator *op) { return op->d_nlCto64; }
@@ -728,6 +738,7 @@ struct OpData<float> {
   static const float *nlC(chfsi_operator *op) { return op->d_nlC32; }
   static const float *ttab(chfsi_operator *op) { return op->d_ttab32; }
   static const float *vq(chfsi_operator *op) { return op->d_vq32; }
+  static float *cells_out(chfsi_operator *op) { return op->d_cells_out32; }
   static const float *nlCp(chfsi_operator *op) { return op->d_nlCp32; }
   static const float *nlCt(chfsi_operator *op) { return op->d_nlCt32; }
   static const float *nlCto(chfsi_operator *op) { return op->d_nlCto32; }
@@ -855,25 +866,16 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
   }
   if (tensor && !ext_scratch) {
     // small blocks: one launch over all cells and a sum, where the operator
-    // already owns scratch (its projections') and need not grow it in a capture
+    // holds a buffer for it (as its projections' scratch, one per precision)
     TensorTouch touch{op->d_touch_ptr, op->d_touch_idx, op->M};
-    Scratch &co = op->cells_out;
-    const size_t bytes = sizeof(T) * size_t(op->C) * op->ne * B;
-    bool all = op->d_touch_ptr && op->n_slots > 0 &&
-               tensor_all_cells(op->tn, sizeof(T) == 8, op->max_color_cells, B);
-    if (all && bytes > co.size) {
-      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-      CHFSI_HIP(hipStreamIsCapturing(s, &cap));
-      all = cap == hipStreamCaptureStatusNone;
-    }
-    if (all) {
-      CHFSI_TRY(co.ensure(bytes));
+    T *co = OpData<T>::cells_out(op);
+    all_cells = co && tensor_all_cells(op->tn, sizeof(T) == 8, op->max_color_cells, B);
+    if (all_cells) {
       a.cells = op->d_cells_by_color;
       a.ncells = op->C;
       CHFSI_HIP(launch_hx_tensor<T>(a, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq,
-                                    &touch, static_cast<T *>(co.ptr), s));
+                                    &touch, co, s));
     }
-    all_cells = all;
   }
   for (int k = 0; k < (all_cells ? 0 : op->ncolors); ++k) {
     a.cells = op->d_cells_by_color + op->color_off[k];

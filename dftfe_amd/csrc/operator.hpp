@@ -101,9 +101,12 @@ struct chfsi_operator {
   int tn = 0, tq = 0;
   bool tensor_pot = false;
   // touches of every DOF in colour order and the cells' sums of one apply, for
-  // small blocks (nullable)
+  // small blocks (nullable).  The sums of each precision have a buffer of their
+  // own, as the projections do: an FP64 and an FP32 apply may run at once.
+  // It is never moved: a captured apply keeps its address.
   uint32_t *d_touch_ptr = nullptr, *d_touch_idx = nullptr;
-  chfsi::Scratch cells_out;
+  double *d_cells_out64 = nullptr;
+  float *d_cells_out32 = nullptr;
   bool tensor_gga = false;  // the shape gradients are products too
   double *d_ttab64 = nullptr, *d_tprod = nullptr, *d_vq64 = nullptr, *d_nlCp64 = nullptr;
   float *d_ttab32 = nullptr, *d_vq32 = nullptr, *d_nlCp32 = nullptr;

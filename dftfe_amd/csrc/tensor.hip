@@ -1307,8 +1307,10 @@ static hipError_t hx_tensor_vec(const HxLaunch<T> &a, const T *vq, const T *tab,
 //          and wins while a colour does not fill the chip: 512 cells x 64 columns
 //          0.09 / 0.19 FP64, 0.06 / 0.13 FP32, x 200 0.216 / 0.218 and 0.13 / 0.21,
 //          x 1 0.05 / 0.12; 1728 x 256 0.77 / 0.62 and 0.44 / 0.38
+static int tile_columns(int n, bool fp64) { return n == 7 && fp64 ? 16 : 32; }
+
 static int64_t colour_items(int n, bool fp64, int cells, int B) {
-  const int tc = n == 7 && fp64 ? 16 : 32;
+  const int tc = tile_columns(n, fp64);
   return int64_t(cells) * ((B + tc - 1) / tc);
 }
 
@@ -1327,6 +1329,10 @@ bool tensor_wins(int n, bool fp64, int cells, int B) {
 // x 64 0.228 / 0.177, x 128 0.304 / 0.306; 1728 x 16 0.264 / 0.213
 bool tensor_all_cells(int n, bool fp64, int cells, int B) {
   return colour_items(n, fp64, cells, B) <= kAllCellsItems;
+}
+
+int tensor_all_cells_columns(int n, bool fp64, int cells) {
+  return kAllCellsItems / cells * tile_columns(n, fp64);
 }
 
 template <typename T>

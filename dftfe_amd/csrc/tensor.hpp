@@ -24,6 +24,8 @@ bool tensor_wins(int n, bool fp64, int cells, int B);
 constexpr int kAllCellsItems = 448;
 // Whether all cells at once beat the colour launches on B columns
 bool tensor_all_cells(int n, bool fp64, int cells, int B);
+// The widest block for which they do (0: none)
+int tensor_all_cells_columns(int n, bool fp64, int cells);
 
 // Host check of an operator's shape values (nqc x ne) and stiffness (ne x ne):
 // true when every entry is the product of one-dimensional, centro-symmetric
