@@ -73,7 +73,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
 
   const int wid = blockIdx.x;
   const int local = wid >> 3;
-  if (local >= a.per_xcd) return;
+  if (local >= a.per_xcd || other_form(a)) return;
   const int item = (wid & 7) * a.per_xcd + local;
   if (item >= a.ncells * a.ntiles) return;
   const int cell = a.cells[item / a.ntiles];
@@ -328,7 +328,7 @@ __attribute__((amdgpu_waves_per_eu(NW == 8 && S == 2 ? 4 : 1))) void hxp_kernel(
 
   const int wid = blockIdx.x;
   const int local = wid >> 3;
-  if (local >= a.per_xcd) return;
+  if (local >= a.per_xcd || other_form(a)) return;
   const int item = (wid & 7) * a.per_xcd + local;
   if (item >= a.ncells * a.ntiles) return;
   const int cell = a.cells[item / a.ntiles];
@@ -524,7 +524,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 2)
 
   const int wid = blockIdx.x;
   const int local = wid >> 3;
-  if (local >= a.per_xcd) return;
+  if (local >= a.per_xcd || other_form(a)) return;
   const int item = (wid & 7) * a.per_xcd + local;
   if (item >= a.ncells * a.ntiles) return;
   const int cell = a.cells[item / a.ntiles];
@@ -1459,6 +1459,8 @@ __global__ void scale_listed_rows_kernel(const int64_t *rows, int64_t nrows, T a
   X[rows[idx / B] * ld + idx % B] *= a;
 }
 
+__global__ void set_form_kernel(int *form, int v) { *form = v; }
+
 template <typename T>
 __global__ void zero_rows_kernel(const int64_t *rows, int64_t nrows, T *X, int64_t ld, int B) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1710,7 +1712,7 @@ __global__ __launch_bounds__(256) void hx1_kernel(HxLaunch<T> a) {
 
   const int wid = blockIdx.x;
   const int local = wid >> 3;
-  if (local >= a.per_xcd) return;
+  if (local >= a.per_xcd || other_form(a)) return;
   const int item = (wid & 7) * a.per_xcd + local;
   if (item >= a.ncells) return;
   const int cell = a.cells[item];
@@ -2909,6 +2911,11 @@ template hipError_t launch_scale_listed_rows<double>(const int64_t *, int64_t, d
                                                      int64_t, int, hipStream_t);
 template hipError_t launch_scale_listed_rows<float>(const int64_t *, int64_t, float, float *,
                                                     int64_t, int, hipStream_t);
+hipError_t launch_set_form(int *form, int v, hipStream_t s) {
+  hipLaunchKernelGGL(set_form_kernel, dim3(1), dim3(1), 0, s, form, v);
+  return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_zero_rows_t(const int64_t *rows, int64_t nrows, T *X, int64_t ld, int B,
                               hipStream_t st) {

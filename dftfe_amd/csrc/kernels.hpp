@@ -56,7 +56,21 @@ struct HxLaunch {
   // 1: the cell matrices are exactly symmetric (built on the device); the
   // one-column kernel then reads the slices on and below the diagonal only
   int h_sym;
+  // captured applies (else null): the form of the cell operators that holds when
+  // the graph is replayed; launches of the other one (`want`) do nothing
+  const int *form;
+  int want;
 };
+
+// Forms of the cell operators: the dense cell matrices (always up to date), or
+// tensor products, where the potential is an LDA one on product tables
+enum { kDenseForm, kTensorForm };
+template <typename T>
+__device__ __forceinline__ bool other_form(const HxLaunch<T> &a) {
+  return a.form && *a.form != a.want;
+}
+// *form = v
+hipError_t launch_set_form(int *form, int v, hipStream_t s);
 
 // Arguments of the projection C_e^T (s_in * src)_e for all cells with slots.
 template <typename T>

@@ -84,7 +84,7 @@ chfsi_operator::~chfsi_operator() {
                   d_ones_cons32, d_own_map, d_own_n, d_nlCto64, d_nlCto32, d_nlCtko64,
                   d_nlCtko32, d_ttab64, d_ttab32, d_tprod, d_touch_ptr, d_touch_idx, d_vq64,
                   d_vq32, d_nlCp64,
-                  d_nlCp32, d_cells_out64, d_cells_out32};
+                  d_nlCp32, d_cells_out64, d_cells_out32, d_form};
   for (void *p : ptrs)
     if (p) hipFree(p);
   ztab_dev.release();
@@ -330,6 +330,7 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
         CHFSI_TRY(dev_upload(&op->d_touch_ptr, tptr.data(), tptr.size()));
         CHFSI_TRY(dev_upload(&op->d_touch_idx, tidx.data(), tidx.size()));
       }
+      CHFSI_TRY(dev_alloc(&op->d_form, 1));
       CHFSI_TRY(dev_alloc(&op->d_vq64, nv));
       CHFSI_TRY(dev_alloc(&op->d_vq32, nv));
     }
@@ -605,6 +606,14 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
 
 extern "C" void chfsi_operator_destroy(chfsi_operator *op) { delete op; }
 
+// Notes whether the tensor form's weights are those of the cell matrices, here and
+// for the captured applies
+static chfsi_status set_form(chfsi_operator *op, bool tensor, hipStream_t s) {
+  op->tensor_pot = tensor;
+  if (op->d_form) CHFSI_HIP(launch_set_form(op->d_form, tensor ? kTensorForm : kDenseForm, s));
+  return CHFSI_OK;
+}
+
 extern "C" chfsi_status chfsi_operator_set_potential(chfsi_operator *op, const double *vJxW,
                                                      void *stream) {
   CHFSI_ARG(op && vJxW, "null argument");
@@ -620,7 +629,7 @@ extern "C" chfsi_status chfsi_operator_set_potential(chfsi_operator *op, const d
   if (op->tn)
     CHFSI_HIP(launch_tensor_potential(vJxW, op->C, op->tn, op->tq, op->d_vq64, op->d_vq32,
                                       as_stream(stream)));
-  op->tensor_pot = op->tn > 0;
+  CHFSI_TRY(set_form(op, op->tn > 0, as_stream(stream)));
   op->has_H = true;
   op->h_sym = true;  // the build writes each off-diagonal pair block from one sum
   return rebuild_kpoint_matrices(op, as_stream(stream));
@@ -639,7 +648,7 @@ extern "C" chfsi_status chfsi_operator_set_potential_gga(chfsi_operator *op, con
     CHFSI_HIP(launch_build_h(op->d_K, op->d_Nq, vJxW, op->d_Gq, gJxW, op->C, op->ne, op->ne_pad,
                              op->nq, op->d_Ht64, op->d_Ht32, op->d_Ht16, as_stream(stream),
                              op->K_per_cell, op->d_invJ, op->jac));
-  op->tensor_pot = false;
+  CHFSI_TRY(set_form(op, false, as_stream(stream)));
   op->has_H = true;
   op->h_sym = true;
   return rebuild_kpoint_matrices(op, as_stream(stream));
@@ -652,7 +661,7 @@ extern "C" chfsi_status chfsi_operator_set_cell_matrices(chfsi_operator *op, con
                           as_stream(stream)));
   CHFSI_HIP(launch_f64_to_bf16(op->d_Ht64, int64_t(op->C) * op->ne_pad * op->ne_pad, op->d_Ht16,
                                as_stream(stream)));
-  op->tensor_pot = false;
+  CHFSI_TRY(set_form(op, false, as_stream(stream)));
   op->has_H = true;
   op->h_sym = false;  // caller's matrices: not assumed symmetric
   return rebuild_kpoint_matrices(op, as_stream(stream));
@@ -848,7 +857,7 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
   a.beta_mode = beta_mode;
   a.B = B;
   a.variant = sizeof(T) == 8 ? op->hx_variant64 : (bf16 ? op->hx_variant16 : op->hx_variant32);
-  bool all_cells = false;
+  bool all_cells = false, captured = false;
   const bool tensor = a.variant < 0 && !bf16 && op->tensor_pot &&
                       ld_src < (int64_t(1) << 29) && ld_dst < (int64_t(1) << 29) &&
                       ldR < (int64_t(1) << 29) &&  // the kernels' row offsets are 32-bit bytes
@@ -864,6 +873,17 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
     a.W = W;
     a.ldW = B;
   }
+  if (tensor) {
+    // a replay applies the potential of its own time, which need not be of this
+    // form: a captured apply holds the launches of both, and those of the wrong
+    // one end at once (us per replay, one form / both: 512 cells at p = 4 x 64
+    // columns 89 / 103, 1728 at p = 6 x 512 in FP32 1410 / 1432)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+    captured = cap != hipStreamCaptureStatusNone;
+    if (captured) a.form = op->d_form;
+    a.want = kTensorForm;
+  }
   if (tensor && !ext_scratch) {
     // small blocks: one launch over all cells and a sum, where the operator
     // holds a buffer for it (as its projections' scratch, one per precision)
@@ -877,21 +897,30 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
                                     &touch, co, s));
     }
   }
-  for (int k = 0; k < (all_cells ? 0 : op->ncolors); ++k) {
-    a.cells = op->d_cells_by_color + op->color_off[k];
-    a.ncells = op->color_off[k + 1] - op->color_off[k];
-    if (a.ncells == 0) continue;
-    if constexpr (sizeof(T) == 4) {
-      if (bf16) {
-        CHFSI_HIP(launch_hx_bf16(a, op->d_Ht16, op->d_nlC16, s));
-        continue;
+  auto colours = [&](bool product) -> chfsi_status {
+    for (int k = 0; k < op->ncolors; ++k) {
+      a.cells = op->d_cells_by_color + op->color_off[k];
+      a.ncells = op->color_off[k + 1] - op->color_off[k];
+      if (a.ncells == 0) continue;
+      if constexpr (sizeof(T) == 4) {
+        if (bf16) {
+          CHFSI_HIP(launch_hx_bf16(a, op->d_Ht16, op->d_nlC16, s));
+          continue;
+        }
       }
+      if (product)
+        CHFSI_HIP(launch_hx_tensor<T>(a, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq,
+                                      nullptr, nullptr, s));
+      else
+        CHFSI_HIP(launch_hx<T>(a, s));
     }
-    if (tensor)
-      CHFSI_HIP(launch_hx_tensor<T>(a, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq,
-                                    nullptr, nullptr, s));
-    else
-      CHFSI_HIP(launch_hx<T>(a, s));
+    return CHFSI_OK;
+  };
+  if (!all_cells) CHFSI_TRY(colours(tensor));
+  if (captured) {
+    a.want = kDenseForm;
+    if (op->n_slots > 0) a.nl_C = OpData<T>::nlC(op);
+    CHFSI_TRY(colours(false));
   }
   if (op->general_constraints) {
     // distribute_slave_to_master (kohnShamDFTOperatorDevice.cc:3832-3838):

@@ -100,6 +100,7 @@ struct chfsi_operator {
   // the cell matrices are those of the weights held here (an LDA potential)
   int tn = 0, tq = 0;
   bool tensor_pot = false;
+  int *d_form = nullptr;  // the same on the device, for captured applies (operators with tn)
   // touches of every DOF in colour order and the cells' sums of one apply, for
   // small blocks (nullable).  The sums of each precision have a buffer of their
   // own, as the projections do: an FP64 and an FP32 apply may run at once.

@@ -882,7 +882,7 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
 
   // consecutive items (the column tiles of a cell first) on one XCD
   const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-  if (item >= a.ncells * a.ntiles) return;
+  if (item >= a.ncells * a.ntiles || other_form(a)) return;
   const int cell = a.cells[item / a.ntiles];
   const int v0 = (item % a.ntiles) * TC;
   const int t = threadIdx.x, lane = t & 63;
@@ -1223,7 +1223,7 @@ __global__ __launch_bounds__(256) void hx_assemble_kernel(HxLaunch<T> a, const u
   const int per = a.B / VW;
   const int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x;
   const int64_t g = e / per;
-  if (g >= M) return;
+  if (g >= M || other_form(a)) return;
   const int v = (int)(e % per) * VW;
   const uint32_t k0 = ptr[g], k1 = ptr[g + 1];
   if (k0 == k1) return;  // a folded row: no cell writes it

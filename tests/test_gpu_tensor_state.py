@@ -72,3 +72,40 @@ def test_precisions_overlap_on_two_streams(small):
     torch.cuda.synchronize()
     assert all(torch.equal(Y, want64) for Y in got[0])
     assert all(torch.equal(Y, want32) for Y in got[1])
+
+
+@pytest.mark.parametrize("B", [1, 8, 600])      # all cells at once; 513 workgroups a colour
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_replay_applies_the_potential_of_its_time(B, dtype):
+    """An apply captured under an LDA potential, replayed after another LDA potential,
+    a GGA one and the caller's cell matrices: each time the eager apply's result."""
+    from dftfe_amd.chfsi import KohnShamOperatorDevice
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    prob = fe.build_workload("cube18_p5_n64")
+    op = KohnShamOperatorDevice(prob)
+    X = _block(prob, B, 5, dtype)
+    Y = torch.zeros_like(X)
+    first = op.apply(X)
+    graph = _capture(op, X, Y)
+    g = 0.1 * np.random.default_rng(6).uniform(-1, 1, (prob.C, prob.nqc, 3)) * prob.jxw_cells[..., None]
+    op.set_potential_gga(prob.vJxW, g)
+    H = op.cell_matrices()
+    steps = (("gga", lambda: op.set_potential_gga(prob.vJxW, g)),
+             ("lda", lambda: op.set_potential(1.5 * prob.vJxW)),
+             ("matrices", lambda: op.set_cell_matrices(1.25 * H)),
+             ("first", lambda: op.set_potential(prob.vJxW)))
+    for name, change in steps:
+        change()
+        want = op.apply(X)
+        Y.fill_(3.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        if name == "matrices" and B == 1:
+            # symmetric here, which the eager one-column apply does not assume
+            err = ((Y - want).abs().max() / want.abs().max()).item()
+            assert err < (1e-14 if dtype == torch.float64 else 2e-6), err
+        else:
+            assert torch.equal(Y, want), name
+        assert torch.equal(want, first) == (name == "first")
