@@ -343,8 +343,11 @@ static bool pairs(const double *p, int64_t ld, int n) {
 // edge) gets longer chunks, so that the items end together; chunks of at least kMinRows
 // rows, at most 256 of them.  (216k rows, whole CholGS in ms, every block of every tile
 // on equal chunks / so: 500 columns 4.94 / 4.73, 333 columns 3.60 / 3.35.)
-static void gram_plan(int64_t K, int m, int n, int diag_off, std::vector<GramItem> *items,
-                      std::vector<GramItem> *tiles) {
+// whole > 0: equal chunks instead, as many as the lower triangle of whole columns
+// has room for, so that an entry's sum does not depend on the group of columns that
+// the call covers.
+static void gram_plan(int64_t K, int m, int n, int diag_off, int whole,
+                      std::vector<GramItem> *items, std::vector<GramItem> *tiles) {
   const int tm = (m + TT - 1) / TT, tn = (n + TT - 1) / TT;
   items->clear();
   tiles->clear();
@@ -362,20 +365,22 @@ static void gram_plan(int64_t K, int m, int n, int diag_off, std::vector<GramIte
   if (nt == 0 || K <= 0) return;
   // slabs of a chunk of load 18, grown until the items fit
   const int64_t slabs = (K + KS - 1) / KS;
-  auto chunk = [&](int t, int64_t full) {
-    return std::max<int64_t>({full * 18 / load[t], (slabs + 255) / 256, kMinRows / KS});
-  };
+  const int64_t least = std::max<int64_t>((slabs + 255) / 256, kMinRows / KS);
   int64_t full = std::max<int64_t>(1, slabs * sum / (18 * 512));
-  for (;; full += std::max<int64_t>(1, full / 256)) {
-    int64_t count = 0;
-    for (int t = 0; t < nt; ++t) {
-      const int64_t c = chunk(t, full);
-      count += (slabs + c - 1) / c;
+  auto chunk = [&](int t) { return std::max<int64_t>(full * 18 / load[t], least); };
+  if (whole > 0) {
+    const int tw = (whole + TT - 1) / TT, nch = std::max(1, 512 / (tw * (tw + 1) / 2));
+    full = (slabs + nch - 1) / nch;
+    load.assign(nt, 18);
+  } else {
+    for (;; full += std::max<int64_t>(1, full / 256)) {
+      int64_t count = 0;
+      for (int t = 0; t < nt; ++t) count += (slabs + chunk(t) - 1) / chunk(t);
+      if (count <= std::max(512, nt)) break;
     }
-    if (count <= std::max(512, nt)) break;
   }
   for (int t = 0; t < nt; ++t) {
-    const int64_t c = chunk(t, full);
+    const int64_t c = chunk(t);
     const int nch = (int)((slabs + c - 1) / c);
     GramItem &tl = (*tiles)[t];
     tl.part = (int)items->size();
@@ -389,17 +394,17 @@ static void gram_plan(int64_t K, int m, int n, int diag_off, std::vector<GramIte
                    [](const GramItem &x, const GramItem &y) { return x.slab < y.slab; });
 }
 
-size_t gram_partial_bytes(int64_t K, int m, int n, int diag_off) {
+size_t gram_partial_bytes(int64_t K, int m, int n, int diag_off, int whole) {
   std::vector<GramItem> items, tiles;
-  gram_plan(K, m, n, diag_off, &items, &tiles);
+  gram_plan(K, m, n, diag_off, whole, &items, &tiles);
   return sizeof(double) * items.size() * TT * TT;
 }
 
 hipError_t launch_gram(const double *A, int64_t lda, const double *B, int64_t ldb, int m, int n,
-                       int64_t K, int diag_off, double *C, int64_t ldc, double *P,
+                       int64_t K, int diag_off, int whole, double *C, int64_t ldc, double *P,
                        GramItem *table_dev, hipStream_t s) {
   std::vector<GramItem> items, tiles;
-  gram_plan(K, m, n, diag_off, &items, &tiles);
+  gram_plan(K, m, n, diag_off, whole, &items, &tiles);
   const int nt = (int)tiles.size(), nitems = (int)items.size();
   if (nitems == 0) return hipSuccess;
   if (nt > kGramMaxTiles || nt + nitems > kGramMaxTable) return hipErrorInvalidValue;

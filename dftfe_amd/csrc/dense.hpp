@@ -24,13 +24,15 @@ struct GramItem {
 // (A^T B of node-major blocks), split over K with partial tiles in P summed in
 // a fixed order.  diag_off >= 0: only the tiles that reach the lower triangle
 // of C, i >= j + diag_off (16 x 16 blocks above it read as zero there); -1: all.
-// P holds gram_partial_bytes(K, m, n, diag_off) bytes and table_dev
+// whole > 0: the call is one group of columns of the lower triangle of an
+// m x whole product, whose entries have the same bits in every grouping.
+// P holds gram_partial_bytes(K, m, n, diag_off, whole) bytes and table_dev
 // kGramMaxTable entries; synchronises the stream (the table is copied
 // from the host).
 hipError_t launch_gram(const double *A, int64_t lda, const double *B, int64_t ldb, int m, int n,
-                       int64_t K, int diag_off, double *C, int64_t ldc, double *P,
+                       int64_t K, int diag_off, int whole, double *C, int64_t ldc, double *P,
                        GramItem *table_dev, hipStream_t s);
-size_t gram_partial_bytes(int64_t K, int m, int n, int diag_off);
+size_t gram_partial_bytes(int64_t K, int m, int n, int diag_off, int whole);
 
 // column tile of the rotation kernel
 constexpr int kRotateTile = 128;

@@ -2422,13 +2422,15 @@ __global__ __launch_bounds__(64 * NW) void projp_kernel(ProjLaunch<float> a) {
 }
 
 // FP64 projection on the direct-to-LDS ring of hxd_kernel.  A stage holds
-// half of a 16-wide K slice: the cell's slot rows of nl_Ct (8 doubles = 64
-// bytes of each, one 1 KB copy per 16 slots, 16-byte units swizzled as for
-// the cell matrices) and the 8 gathered source rows of TN = 128 columns (one
-// 1 KB copy per row, the copies XG bytes apart so that the B-operand reads of
-// the four lane groups fall in two 128-byte bank windows).  Four waves split
-// the columns (32 each) and hold every slot block of the cell.  In the r-th
-// of the two MFMAs of a half slice lane l supplies K row 2 (l/16) + r.  OWN:
+// half of a 16-wide K slice, the rows 4 g + 2 half + (0, 1) of the four lane
+// groups g: the cell's slot rows of nl_Ct (8 doubles = 64 bytes of each, one 1 KB
+// copy per 16 slots, 16-byte units swizzled as for the cell matrices) and the
+// 8 gathered source rows of TN = 128 columns (one 1 KB copy per row, the copies
+// XG bytes apart so that the B-operand reads of the four lane groups fall in
+// two 128-byte bank windows).  Four waves split the columns (32 each) and hold
+// every slot block of the cell.  In the r-th of the two MFMAs of a half slice
+// lane l supplies row 4 (l/16) + 2 half + r: the order of proj_kernel, which
+// takes blocks that are not aligned, so both give the same bits.  OWN:
 // owned rows instead of the cell's nodes, as in proj_kernel.  Requirements
 // (checked by the launcher): B even, 16-byte aligned src rows (ld_src even)
 // and nl_Ct.
@@ -2491,14 +2493,14 @@ __global__ __launch_bounds__(256) void projd_kernel(ProjLaunch<double> a) {
 
   const uint32_t ring0 = lds_address(ring);
   const int hr = lane >> 2;  // slot row within a copy's 16 rows
-  const int hoff = hr * 16 + 2 * ((lane & 3) ^ (((hr >> 1) ^ (hr >> 3)) & 3));
+  const int hoff = hr * 16 + 4 * ((lane & 3) ^ (((hr >> 1) ^ (hr >> 3)) & 3));
   const int xc = v0 + 2 * lane;
   const int xcl = xc < a.B - 2 ? xc : a.B - 2;  // columns >= B are never stored
   const T *xb = a.src + xcl;
 
   auto issue = [&](int h, int stage) {
     const int t = h >> 1, half = h & 1;
-    const T *tile = Acell + (int64_t)t * nslot * 16 + half * 8;
+    const T *tile = Acell + (int64_t)t * nslot * 16 + half * 2;
     const uint32_t sbase = ring0 + stage * SB;
 #pragma unroll
     for (int j = 0; j < D; ++j) {
@@ -2507,7 +2509,7 @@ __global__ __launch_bounds__(256) void projd_kernel(ProjLaunch<double> a) {
         copy16_to_lds(tile + o * 256 + hoff, sbase + o * 1024);
       } else {
         const int x = o - nsrb;
-        copy16_to_lds(xb + soff[t * 16 + half * 8 + x], sbase + AB + x * XG);
+        copy16_to_lds(xb + soff[t * 16 + 4 * (x >> 1) + 2 * half + (x & 1)], sbase + AB + x * XG);
       }
     }
   };
@@ -2519,15 +2521,15 @@ __global__ __launch_bounds__(256) void projd_kernel(ProjLaunch<double> a) {
     for (int cb = 0; cb < CBW; ++cb) acc[j][cb] = v4{0, 0, 0, 0};
 
   const int arow = lane & 15;
-  const int g = lane >> 4;  // K rows 2g, 2g + 1 of the half slice
+  const int g = lane >> 4;  // copies 2g, 2g + 1 of the half slice
   const int aoff = arow * 64 + ((g ^ (((arow >> 1) ^ (arow >> 3)) & 3)) * 16);  // bytes
-  const int xo0 = 2 * g * XG, xo1 = xo0 + XG;  // copies of K rows 2g, 2g + 1
+  const int xo0 = 2 * g * XG, xo1 = xo0 + XG;
 
   auto compute = [&](int stage, int h) {
     const unsigned char *As = ring + stage * SB;
     const T *X0 = reinterpret_cast<const T *>(ring + stage * SB + AB + xo0);
     const T *X1 = reinterpret_cast<const T *>(ring + stage * SB + AB + xo1);
-    const int k0 = (h >> 1) * 16 + (h & 1) * 8 + 2 * g;
+    const int k0 = (h >> 1) * 16 + 4 * g + 2 * (h & 1);
     const T sc0 = sscl[k0], sc1 = sscl[k0 + 1];
     T b0[CBW], b1[CBW];
 #pragma unroll

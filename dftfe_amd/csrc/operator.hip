@@ -771,7 +771,8 @@ template <typename T>
 chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, int64_t ld_dst,
                       int B, T alpha, T beta, T gamma, int beta_mode, bool scaled,
                       hipStream_t s, bool bf16, const T *R, int64_t ldR, const T *rcoef,
-                      void *ext_scratch) {
+                      void *ext_scratch, int choice) {
+  if (choice <= 0) choice = B;
   CHFSI_ARG(!bf16 || sizeof(T) == 4, "the BF16 apply works on FP32 multivectors");
   CHFSI_ARG(!R || (!bf16 && sizeof(T) == 4 && rcoef && ldR >= B), "bad defect source");
   if (!op->has_H) {
@@ -830,7 +831,7 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
     pl.B = B;
     pl.max_srb = op->max_srb;
     pl.variant = sizeof(T) == 8 ? op->proj_variant64 : op->proj_variant32;
-    if (pl.variant < 0) pl.variant = bf16 ? 0 : proj_default(op->n_nl_cells, B);
+    if (pl.variant < 0) pl.variant = bf16 ? 0 : proj_default(op->n_nl_cells, choice);
     if (pl.variant >= 4) {
       pl.nl_Ct = OpData<T>::nlCto(op);
       pl.own_map = op->d_own_map;
@@ -861,7 +862,7 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
   const bool tensor = a.variant < 0 && !bf16 && op->tensor_pot &&
                       ld_src < (int64_t(1) << 29) && ld_dst < (int64_t(1) << 29) &&
                       ldR < (int64_t(1) << 29) &&  // the kernels' row offsets are 32-bit bytes
-                      tensor_wins(op->tn, sizeof(T) == 8, op->max_color_cells, B);
+                      tensor_wins(op->tn, sizeof(T) == 8, op->max_color_cells, choice);
   a.R = R;
   a.ldR = ldR;
   a.rcoef = rcoef;
@@ -937,10 +938,10 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
 template chfsi_status hx_fused<double>(chfsi_operator *, const double *, int64_t, double *,
                                        int64_t, int, double, double, double, int, bool,
                                        hipStream_t, bool, const double *, int64_t,
-                                       const double *, void *);
+                                       const double *, void *, int);
 template chfsi_status hx_fused<float>(chfsi_operator *, const float *, int64_t, float *, int64_t,
                                       int, float, float, float, int, bool, hipStream_t, bool,
-                                      const float *, int64_t, const float *, void *);
+                                      const float *, int64_t, const float *, void *, int);
 
 }  // namespace chfsi
 

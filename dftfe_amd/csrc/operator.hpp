@@ -23,7 +23,10 @@ struct Scratch {
 // One fused apply  dst <- base + alpha * S H S src  over all colour classes
 // (see HxLaunch for base / beta_mode).  bf16 selects the BF16-input kernel
 // (T = float only).  R (nullable, ld ldR) adds rcoef[v] * R[:, v] to every row
-// once (the defect form of the filter; FP32, not with bf16).
+// once (the defect form of the filter; FP32, not with bf16).  choice (0: B):
+// the block width that the kernels' choice goes by, the same for all the
+// applies of a pass, so that a column's bits do not depend on the group that
+// it is applied in.
 // Layout of a caller-provided HX scratch: projection partials (n_slots x B),
 // then the V-scaled projections (n_proj x B) at the next 256-byte boundary.
 inline size_t noalloc_w_offset(size_t elem, int n_slots, int B) {
@@ -37,7 +40,7 @@ template <typename T>
 chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, int64_t ld_dst,
                       int B, T alpha, T beta, T gamma, int beta_mode, bool scaled, hipStream_t s,
                       bool bf16 = false, const T *R = nullptr, int64_t ldR = 0,
-                      const T *rcoef = nullptr, void *ext_scratch = nullptr);
+                      const T *rcoef = nullptr, void *ext_scratch = nullptr, int choice = 0);
 
 // g (+)= wscale JxW sum_v w_v (N.(s a_v))(N.(s b_v)) per (cell, quadrature
 // point), s = M^{-1/2} when scaled; with general constraints the rows of a and

@@ -152,22 +152,23 @@ ChebState cheb_init(double a, double b, double a0) {
 // degree 1 from X into Y
 template <typename T>
 chfsi_status cheb_first(chfsi_operator *op, const T *X, int64_t ldX, T *Y, int64_t ldY, int B,
-                        const ChebState &cs, hipStream_t st, bool bf16, void *hx_ws = nullptr) {
+                        const ChebState &cs, hipStream_t st, bool bf16, int choice,
+                        void *hx_ws = nullptr) {
   return hx_fused<T>(op, X, ldX, Y, ldY, B, T(cs.sigma / cs.e), T(0), T(-cs.c * cs.sigma / cs.e),
-                     1, true, st, bf16, nullptr, 0, nullptr, hx_ws);
+                     1, true, st, bf16, nullptr, 0, nullptr, hx_ws, choice);
 }
 
 // degrees d0..d1 (d0 >= 2); *cur holds the latest iterate, *prev the one before;
 // hx_ws (nullable): projection scratch of the HX calls in place of the operator's
 template <typename T>
 chfsi_status cheb_steps(chfsi_operator *op, T **cur, int64_t *ldc, T **prev, int64_t *ldp, int B,
-                        int d0, int d1, ChebState &cs, hipStream_t st, bool bf16,
+                        int d0, int d1, ChebState &cs, hipStream_t st, bool bf16, int choice,
                         void *hx_ws = nullptr) {
   for (int degree = d0; degree <= d1; ++degree) {
     const double sigma2 = 1.0 / (cs.gamma - cs.sigma);
     const double alpha1 = 2.0 * sigma2 / cs.e, alpha2 = -(cs.sigma * sigma2);
     CHFSI_TRY(hx_fused<T>(op, *cur, *ldc, *prev, *ldp, B, T(alpha1), T(alpha2),
-                          T(-cs.c * alpha1), 0, true, st, bf16, nullptr, 0, nullptr, hx_ws));
+                          T(-cs.c * alpha1), 0, true, st, bf16, nullptr, 0, nullptr, hx_ws, choice));
     std::swap(*cur, *prev);
     std::swap(*ldc, *ldp);
     cs.sigma = sigma2;
@@ -198,12 +199,14 @@ int filter_group_columns(const chfsi_params &P, int64_t M, int N, int B) {
 // the FP64 eigenvectors' accuracy.  Equal to the plain filter in exact
 // arithmetic.
 chfsi_status filter_block_defect(chfsi_solver *s, chfsi_operator *op, double *X, int64_t ld,
-                                 int B, int m, double a, double b, double a0, hipStream_t st) {
+                                 int B, int m, double a, double b, double a0, int choice,
+                                 hipStream_t st) {
   const int64_t M = op->M;
   const ChebState cs = cheb_init(a, b, a0);
   CHFSI_TRY(s->HXb.ensure(sizeof(double) * M * B));
   double *HX = sptr<double>(s->HXb);
-  CHFSI_TRY(hx_fused<double>(op, X, ld, HX, B, B, 1.0, 0.0, 0.0, 1, true, st));
+  CHFSI_TRY(hx_fused<double>(op, X, ld, HX, B, B, 1.0, 0.0, 0.0, 1, true, st, false, nullptr, 0,
+                             nullptr, nullptr, choice));
   if (op->nc) CHFSI_HIP(launch_zero_rows(op->d_c_rows, op->nc, HX, B, B, st));
   const int nch = 256;
   CHFSI_TRY(s->part.ensure(sizeof(double) * nch * 2 * B));
@@ -257,7 +260,7 @@ chfsi_status filter_block_defect(chfsi_solver *s, chfsi_operator *op, double *X,
     const double alpha1 = 2.0 * sigma2 / cs.e, alpha2 = -(sigma * sigma2);
     CHFSI_TRY(hx_fused<float>(op, Ec, B, Ep, B, B, float(alpha1), float(alpha2),
                               float(-cs.c * alpha1), 0, true, st, false, R, B,
-                              drc + size_t(degree) * B));
+                              drc + size_t(degree) * B, nullptr, choice));
     std::swap(Ec, Ep);
     sigma = sigma2;
   }
@@ -272,20 +275,21 @@ chfsi_status filter_block_defect(chfsi_solver *s, chfsi_operator *op, double *X,
 // degrees run in FP64 from the cast-back pair of iterates, so that the
 // rounding of the low-precision steps is itself filtered.  hx_ws (nullable,
 // FP64 form only): projection scratch of its HX calls in place of the
-// operator's own.
+// operator's own.  choice: see hx_fused.
 chfsi_status filter_block(chfsi_solver *s, chfsi_operator *op, double *X, int64_t ld, int B, int m,
                           double a, double b, double a0, int precision, int tail,
-                          hipStream_t st, void *hx_ws = nullptr) {
+                          hipStream_t st, int choice = 0, void *hx_ws = nullptr) {
   const int64_t M = op->M;
   ChebState cs = cheb_init(a, b, a0);
   CHFSI_TRY(s->Y64.ensure(sizeof(double) * M * B));
   double *Y = sptr<double>(s->Y64);
   if (precision == CHFSI_FP64) {
     CHFSI_HIP(hipMemsetAsync(Y, 0, sizeof(double) * M * B, st));
-    CHFSI_TRY(cheb_first<double>(op, X, ld, Y, B, B, cs, st, false, hx_ws));
+    CHFSI_TRY(cheb_first<double>(op, X, ld, Y, B, B, cs, st, false, choice, hx_ws));
     double *cur = Y, *prev = X;
     int64_t ldc = B, ldp = ld;
-    CHFSI_TRY(cheb_steps<double>(op, &cur, &ldc, &prev, &ldp, B, 2, m, cs, st, false, hx_ws));
+    CHFSI_TRY(
+        cheb_steps<double>(op, &cur, &ldc, &prev, &ldp, B, 2, m, cs, st, false, choice, hx_ws));
     if (cur != X) CHFSI_HIP(launch_copy_block<double, double>(cur, ldc, X, ld, M, B, st));
     return CHFSI_OK;
   }
@@ -295,7 +299,7 @@ chfsi_status filter_block(chfsi_solver *s, chfsi_operator *op, double *X, int64_
   }
   const bool bf16 = precision == CHFSI_BF16;
   if (!bf16 && s->params.mixed_prec_defect_filter)
-    return filter_block_defect(s, op, X, ld, B, m, a, b, a0, st);
+    return filter_block_defect(s, op, X, ld, B, m, a, b, a0, choice, st);
   tail = std::max(0, std::min(tail, m - 1));
   const int mlow = m - tail;
   CHFSI_TRY(s->X32.ensure(sizeof(float) * M * B));
@@ -303,10 +307,10 @@ chfsi_status filter_block(chfsi_solver *s, chfsi_operator *op, double *X, int64_
   float *X32 = sptr<float>(s->X32), *Y32 = sptr<float>(s->Y32);
   CHFSI_HIP(launch_copy_block<double, float>(X, ld, X32, B, M, B, st));
   CHFSI_HIP(hipMemsetAsync(Y32, 0, sizeof(float) * M * B, st));
-  CHFSI_TRY(cheb_first<float>(op, X32, B, Y32, B, B, cs, st, bf16));
+  CHFSI_TRY(cheb_first<float>(op, X32, B, Y32, B, B, cs, st, bf16, choice));
   float *cur = Y32, *prev = X32;
   int64_t ldc = B, ldp = B;
-  CHFSI_TRY(cheb_steps<float>(op, &cur, &ldc, &prev, &ldp, B, 2, mlow, cs, st, bf16));
+  CHFSI_TRY(cheb_steps<float>(op, &cur, &ldc, &prev, &ldp, B, 2, mlow, cs, st, bf16, choice));
   if (tail == 0) {
     CHFSI_HIP(launch_copy_block<float, double>(cur, ldc, X, ld, M, B, st));
     return CHFSI_OK;
@@ -316,7 +320,8 @@ chfsi_status filter_block(chfsi_solver *s, chfsi_operator *op, double *X, int64_
   CHFSI_HIP(launch_copy_block<float, double>(prev, ldp, Y, B, M, B, st));
   double *c64 = X, *p64 = Y;
   int64_t ldc64 = ld, ldp64 = B;
-  CHFSI_TRY(cheb_steps<double>(op, &c64, &ldc64, &p64, &ldp64, B, mlow + 1, m, cs, st, false));
+  CHFSI_TRY(
+      cheb_steps<double>(op, &c64, &ldc64, &p64, &ldp64, B, mlow + 1, m, cs, st, false, choice));
   if (c64 != X) CHFSI_HIP(launch_copy_block<double, double>(c64, ldc64, X, ld, M, B, st));
   return CHFSI_OK;
 }
@@ -456,15 +461,15 @@ int64_t panel_rows(int64_t M, int N) {
 // Mixed (subspaceRotationRRMixedPrecScalapack, :2660-3077): the bs x bs diagonal
 // blocks of Q in FP64, the rest from FP32 copies of Q and X.
 // C = A^T B over M rows with the library's FP64 MFMA kernel (lower-triangle
-// tiles i >= j + diag_off, or all with diag_off = -1)
+// tiles i >= j + diag_off, or all with diag_off = -1); whole: see launch_gram
 chfsi_status gram_fp64(chfsi_solver *s, const double *A, int64_t lda, const double *B,
                        int64_t ldb, int m, int n, int64_t M, int diag_off, double *C,
-                       int64_t ldc, hipStream_t st) {
-  const size_t pb = gram_partial_bytes(M, m, n, diag_off);
+                       int64_t ldc, hipStream_t st, int whole = 0) {
+  const size_t pb = gram_partial_bytes(M, m, n, diag_off, whole);
   if (pb == 0) return CHFSI_OK;
   CHFSI_TRY(s->split.ensure(pb));
   CHFSI_TRY(s->gtiles.ensure(sizeof(GramItem) * kGramMaxTable));
-  CHFSI_HIP(launch_gram(A, lda, B, ldb, m, n, M, diag_off, C, ldc, sptr<double>(s->split),
+  CHFSI_HIP(launch_gram(A, lda, B, ldb, m, n, M, diag_off, whole, C, ldc, sptr<double>(s->split),
                         static_cast<GramItem *>(s->gtiles.ptr), st));
   return CHFSI_OK;
 }
@@ -683,9 +688,10 @@ chfsi_status xthx_lower(chfsi_solver *s, chfsi_operator *op, const double *X, in
     // tiles that reach the lower triangle
     for (g0 = 0; g0 < N; g0 += G) {
       gw = std::min(G, N - g0);
-      CHFSI_TRY(hx_fused<double>(op, X + g0, N, HXg, gw, gw, 1.0, 0.0, 0.0, 1, true, st));
+      CHFSI_TRY(hx_fused<double>(op, X + g0, N, HXg, gw, gw, 1.0, 0.0, 0.0, 1, true, st,
+                                 false, nullptr, 0, nullptr, nullptr, N));
       if (op->nc) CHFSI_HIP(launch_zero_rows(op->d_c_rows, op->nc, HXg, gw, gw, st));
-      CHFSI_TRY(gram_fp64(s, X, N, HXg, gw, N, gw, M, g0, Hp + (int64_t)g0 * N, N, st));
+      CHFSI_TRY(gram_fp64(s, X, N, HXg, gw, N, gw, M, g0, Hp + (int64_t)g0 * N, N, st, N));
     }
     return CHFSI_OK;
   }
@@ -694,7 +700,8 @@ chfsi_status xthx_lower(chfsi_solver *s, chfsi_operator *op, const double *X, in
     if (j >= g0 + gw) {
       g0 = j;
       gw = std::min(G, N - j);
-      CHFSI_TRY(hx_fused<double>(op, X + j, N, HXg, gw, gw, 1.0, 0.0, 0.0, 1, true, st));
+      CHFSI_TRY(hx_fused<double>(op, X + j, N, HXg, gw, gw, 1.0, 0.0, 0.0, 1, true, st,
+                                 false, nullptr, 0, nullptr, nullptr, N));
       if (op->nc) CHFSI_HIP(launch_zero_rows(op->d_c_rows, op->nc, HXg, gw, gw, st));
     }
     const double *HX = HXg + (j - g0);
@@ -812,7 +819,8 @@ chfsi_status residual_impl(chfsi_solver *s, chfsi_operator *op, const double *X,
     if (j >= g0 + gw) {
       g0 = j;
       gw = std::min(G, N - j);
-      CHFSI_TRY(hx_fused<double>(op, X + j, ldX, HX, gw, gw, 1.0, 0.0, 0.0, 1, true, st));
+      CHFSI_TRY(hx_fused<double>(op, X + j, ldX, HX, gw, gw, 1.0, 0.0, 0.0, 1, true, st,
+                                 false, nullptr, 0, nullptr, nullptr, N));
       if (op->nc) CHFSI_HIP(launch_zero_rows(op->d_c_rows, op->nc, HX, gw, gw, st));
     }
     CHFSI_HIP(launch_residual_partial(HX + (j - g0), gw, X + j, ldX, lam + j, M, bw, part, nch,
@@ -861,7 +869,8 @@ chfsi_status rr_split_impl(chfsi_solver *s, chfsi_operator *op, const double *X,
     if (j >= g0 + gw) {
       g0 = j;
       gw = std::min(G, N - j);
-      CHFSI_TRY(hx_fused<double>(op, X + j, N, HXg, gw, gw, 1.0, 0.0, 0.0, 1, true, st));
+      CHFSI_TRY(hx_fused<double>(op, X + j, N, HXg, gw, gw, 1.0, 0.0, 0.0, 1, true, st,
+                                 false, nullptr, 0, nullptr, nullptr, N));
       if (op->nc) CHFSI_HIP(launch_zero_rows(op->d_c_rows, op->nc, HXg, gw, gw, st));
     }
     const double *HX = HXg + (j - g0);
@@ -1275,21 +1284,21 @@ chfsi_status filter_all(chfsi_solver *s, chfsi_operator *op, double *X, int64_t 
     for (int j = nlow; j < N && stl == CHFSI_OK; j += G) {
       const int bw = std::min(G, N - j);
       stl = filter_block(s, op, X + j, N, bw, m, s->bLow, s->bUp, s->a0, CHFSI_FP64, 0, top_st,
-                         top_ws);
+                         N, top_ws);
     }
     for (int j = 0; j < nlow && stl == CHFSI_OK; j += G) {
       const int bw = std::min(G, nlow - j);
-      stl = filter_block(s, op, X + j, N, bw, m, s->bLow, s->bUp, s->a0, prec, tail, st);
+      stl = filter_block(s, op, X + j, N, bw, m, s->bLow, s->bUp, s->a0, prec, tail, st, N);
     }
     return join(stl);
   }
   for (int j = 0; j < nlow; j += G) {
     const int bw = std::min(G, nlow - j);
-    CHFSI_TRY(filter_block(s, op, X + j, N, bw, m, s->bLow, s->bUp, s->a0, prec, tail, st));
+    CHFSI_TRY(filter_block(s, op, X + j, N, bw, m, s->bLow, s->bUp, s->a0, prec, tail, st, N));
   }
   for (int j = nlow; j < N; j += G) {
     const int bw = std::min(G, N - j);
-    CHFSI_TRY(filter_block(s, op, X + j, N, bw, m, s->bLow, s->bUp, s->a0, CHFSI_FP64, 0, st));
+    CHFSI_TRY(filter_block(s, op, X + j, N, bw, m, s->bLow, s->bUp, s->a0, CHFSI_FP64, 0, st, N));
   }
   return CHFSI_OK;
 }
