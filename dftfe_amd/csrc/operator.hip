@@ -1040,7 +1040,7 @@ extern "C" chfsi_status chfsi_operator_set_hx_variant(chfsi_operator *op, int32_
     return CHFSI_OK;
   }
   CHFSI_ARG(precision == CHFSI_FP64 || precision == CHFSI_FP32, "bad precision");
-  CHFSI_ARG(variant >= 0 && variant < hx_variants(precision == CHFSI_FP64), "bad variant");
+  CHFSI_ARG(variant >= -1 && variant < hx_variants(precision == CHFSI_FP64), "bad variant");
   if (precision == CHFSI_FP64)
     op->hx_variant64 = variant;
   else
@@ -1052,7 +1052,7 @@ extern "C" chfsi_status chfsi_operator_set_proj_variant(chfsi_operator *op, int3
                                                        int32_t variant) {
   CHFSI_ARG(op, "null operator");
   CHFSI_ARG(precision == CHFSI_FP64 || precision == CHFSI_FP32, "bad precision");
-  CHFSI_ARG(variant >= 0 && variant < proj_variants(), "bad variant");
+  CHFSI_ARG(variant >= -1 && variant < proj_variants(), "bad variant");
   (precision == CHFSI_FP64 ? op->proj_variant64 : op->proj_variant32) = variant;
   return CHFSI_OK;
 }

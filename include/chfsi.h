@@ -263,11 +263,14 @@ chfsi_status chfsi_operator_set_cell_matrices(chfsi_operator *op, const double *
 chfsi_status chfsi_operator_get_cell_matrices(chfsi_operator *op, double *H_dev, void *stream);
 
 /* Tile-shape selection of the fused HX kernel (no reference counterpart: the
- * reference calls hipBLAS gemmStridedBatched).  chfsi_operator_autotune times
- * every tile variant of both precisions on a B-column block, keeps the fastest
- * (until a variant is set, and after autotuning where it is faster, operators
- * whose cells are products of one-dimensional tables apply an LDA potential
- * direction by direction instead of through the cell matrices), then times the projection-kernel variants with it and keeps the fastest.
+ * reference calls hipBLAS gemmStridedBatched).  Until a variant is set (or with
+ * variant -1, which returns to that), operators whose cells are products of
+ * one-dimensional tables apply an LDA potential direction by direction instead
+ * of through the cell matrices, and the projection's variant goes by the width.
+ * chfsi_operator_autotune times every tile variant of both precisions on a
+ * B-column block, keeps the fastest (that form where it is faster than all of
+ * them), then times the projection-kernel variants with it and keeps the
+ * fastest.
  * times_ms (48 entries) [0..15]: FP64 tile variants, [16..23]: FP64 projection
  * variants, [24..39]: FP32 tile variants, [40..47]: FP32 projection variants
  * (ms per HX; -1 where a variant does not exist).  Projection variants 4
