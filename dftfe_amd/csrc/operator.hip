@@ -732,6 +732,8 @@ struct OpData<double> {
   static const double *ttab(chfsi_operator *op) { return op->d_ttab64; }
   static const double *vq(chfsi_operator *op) { return op->d_vq64; }
   static double *cells_out(chfsi_operator *op) { return op->d_cells_out64; }
+  static int &hx_variant(chfsi_operator *op) { return op->hx_variant64; }
+  static int &hx_tuned(chfsi_operator *op) { return op->hx_tuned64; }
   static const double *nlCp(chfsi_operator *op) { return op->d_nlCp64; }
   static const double *nlCt(chfsi_operator *op) { return op->d_nlCt64; }
   static const double *nlCto(chfsi_operator *op) { return op->d_nlCto64; }
@@ -748,6 +750,8 @@ struct OpData<float> {
   static const float *ttab(chfsi_operator *op) { return op->d_ttab32; }
   static const float *vq(chfsi_operator *op) { return op->d_vq32; }
   static float *cells_out(chfsi_operator *op) { return op->d_cells_out32; }
+  static int &hx_variant(chfsi_operator *op) { return op->hx_variant32; }
+  static int &hx_tuned(chfsi_operator *op) { return op->hx_tuned32; }
   static const float *nlCp(chfsi_operator *op) { return op->d_nlCp32; }
   static const float *nlCt(chfsi_operator *op) { return op->d_nlCt32; }
   static const float *nlCto(chfsi_operator *op) { return op->d_nlCto32; }
@@ -857,9 +861,10 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
   a.gamma = gamma;
   a.beta_mode = beta_mode;
   a.B = B;
-  a.variant = sizeof(T) == 8 ? op->hx_variant64 : (bf16 ? op->hx_variant16 : op->hx_variant32);
+  const int set_tile = OpData<T>::hx_variant(op);
+  a.variant = bf16 ? op->hx_variant16 : set_tile >= 0 ? set_tile : OpData<T>::hx_tuned(op);
   bool all_cells = false, captured = false;
-  const bool tensor = a.variant < 0 && !bf16 && op->tensor_pot &&
+  const bool tensor = set_tile < 0 && !bf16 && op->tensor_pot &&
                       ld_src < (int64_t(1) << 29) && ld_dst < (int64_t(1) << 29) &&
                       ldR < (int64_t(1) << 29) &&  // the kernels' row offsets are 32-bit bytes
                       tensor_wins(op->tn, sizeof(T) == 8, op->max_color_cells, choice);
@@ -1041,10 +1046,7 @@ extern "C" chfsi_status chfsi_operator_set_hx_variant(chfsi_operator *op, int32_
   }
   CHFSI_ARG(precision == CHFSI_FP64 || precision == CHFSI_FP32, "bad precision");
   CHFSI_ARG(variant >= -1 && variant < hx_variants(precision == CHFSI_FP64), "bad variant");
-  if (precision == CHFSI_FP64)
-    op->hx_variant64 = variant;
-  else
-    op->hx_variant32 = variant;
+  (precision == CHFSI_FP64 ? op->hx_variant64 : op->hx_variant32) = variant;
   return CHFSI_OK;
 }
 
@@ -1070,11 +1072,9 @@ chfsi_status time_variants(chfsi_operator *op, int B, int *best, float *times, h
   hipEvent_t e0, e1;
   CHFSI_HIP(hipEventCreate(&e0));
   CHFSI_HIP(hipEventCreate(&e1));
-  int &var = sizeof(T) == 8 ? op->hx_variant64 : op->hx_variant32;
-  float best_t = 1e30f, tensor_t = 1e30f;
-  // v = -1: the tensor form, where the operator has it (kept when it is faster
-  // than every tile variant; *best and times report the tile variants)
-  for (int v = op->tensor_pot ? -1 : 0; v < nv; ++v) {
+  int &var = OpData<T>::hx_variant(op);
+  float best_t = 1e30f;
+  for (int v = 0; v < nv; ++v) {
     var = v;
     const T *xs = static_cast<const T *>(x.ptr);
     T *ys = static_cast<T *>(y.ptr);
@@ -1088,18 +1088,16 @@ chfsi_status time_variants(chfsi_operator *op, int B, int *best, float *times, h
     }
     float ms = 1e30f;
     if (stt == CHFSI_OK) CHFSI_HIP(hipEventElapsedTime(&ms, e0, e1));
-    if (v < 0) {
-      tensor_t = ms;
-      continue;
-    }
     times[v] = stt == CHFSI_OK ? ms / 3 : -1.0f;
     if (stt == CHFSI_OK && ms < best_t) {
       best_t = ms;
       *best = v;
     }
   }
-  var = tensor_t < best_t ? -1 : *best;
-  // projection variants with the chosen tile variant, timed as whole applies
+  OpData<T>::hx_tuned(op) = *best;
+  var = -1;
+  // projection variants with the form that the operator then takes, timed as
+  // whole applies
   if (op->n_slots > 0) {
     int &pv = sizeof(T) == 8 ? op->proj_variant64 : op->proj_variant32;
     float best_p = 1e30f;

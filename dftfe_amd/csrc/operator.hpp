@@ -114,10 +114,11 @@ struct chfsi_operator {
   bool tensor_gga = false;  // the shape gradients are products too
   double *d_ttab64 = nullptr, *d_tprod = nullptr, *d_vq64 = nullptr, *d_nlCp64 = nullptr;
   float *d_ttab32 = nullptr, *d_vq32 = nullptr, *d_nlCp32 = nullptr;
-  // HX tile and projection variants per precision (chosen by
-  // chfsi_operator_autotune); -1: the tensor form where the operator has it,
-  // tile variant 0 otherwise
+  // HX tile variants per precision: the caller's (-1: none set), and the fastest
+  // of the dense form (chfsi_operator_autotune).  Only a tile that the caller set
+  // turns the tensor form off where the operator has it.
   int hx_variant64 = -1, hx_variant32 = -1;
+  int hx_tuned64 = 0, hx_tuned32 = 0;
   int hx_variant16 = 0;  // BF16 apply: 0 K = 32 ring, 1 register-staged K = 16
   int proj_variant64 = -1, proj_variant32 = -1;  // -1: by size (proj_default)
   int max_srb = 1;  // largest slot count of any cell / 16

@@ -268,9 +268,9 @@ chfsi_status chfsi_operator_get_cell_matrices(chfsi_operator *op, double *H_dev,
  * one-dimensional tables apply an LDA potential direction by direction instead
  * of through the cell matrices, and the projection's variant goes by the width.
  * chfsi_operator_autotune times every tile variant of both precisions on a
- * B-column block, keeps the fastest (that form where it is faster than all of
- * them), then times the projection-kernel variants with it and keeps the
- * fastest.
+ * B-column block, keeps the fastest for the applies that go through the cell
+ * matrices (the others stay direction by direction: tiles set before are
+ * unset), then times the projection-kernel variants and keeps the fastest.
  * times_ms (48 entries) [0..15]: FP64 tile variants, [16..23]: FP64 projection
  * variants, [24..39]: FP32 tile variants, [40..47]: FP32 projection variants
  * (ms per HX; -1 where a variant does not exist).  Projection variants 4

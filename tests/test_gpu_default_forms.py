@@ -74,3 +74,33 @@ def test_committed_pass_on_the_default_forms(name):
         out.append((X, lam, res))
     assert torch.equal(out[0][0], out[1][0])
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("name,B", [("cube20_p4_n64", 1024), ("cube18_p5_n64", 64)])
+@pytest.mark.parametrize("prec,dtype", [(L.FP64, torch.float64), (L.FP32, torch.float32)])
+@pytest.mark.parametrize("gga_first", [False, True])
+def test_autotune_keeps_both_forms(name, B, prec, dtype, gga_first):
+    """Autotuning (on a block or under a potential that takes the cell matrices, too)
+    leaves the tensor form to LDA potentials, and applies through the cell matrices
+    run the tile that was the fastest."""
+    prob, op = _operator(name)
+    g = 0.1 * np.random.default_rng(2).uniform(-1, 1, (prob.C, prob.nqc, 3)) * prob.jxw_cells[..., None]
+    X = torch.tensor(prob.initial_guess(N=24, seed_offset=3), device="cuda", dtype=dtype)
+    lda = op.apply(X)
+    if gga_first:
+        op.set_potential_gga(prob.vJxW, g)
+    tuned = op.autotune(B)
+    op.set_proj_variant(prec, -1)
+    op.set_potential(prob.vJxW)
+    assert torch.equal(op.apply(X), lda)
+    op.set_potential_gga(prob.vJxW, g)
+    gga = op.apply(X)
+    op.set_hx_variant(prec, tuned["fp64" if prec == L.FP64 else "fp32"])
+    assert torch.equal(op.apply(X), gga)
+    op.set_hx_variant(prec, 0)
+    err = ((op.apply(X) - gga).abs().max() / gga.abs().max()).item()
+    assert err < (1e-13 if prec == L.FP64 else 2e-6)
+    op.set_hx_variant(prec, -1)
+    assert torch.equal(op.apply(X), gga)
+    op.set_potential(prob.vJxW)
+    assert torch.equal(op.apply(X), lda)
