@@ -775,7 +775,7 @@ template <typename T>
 chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, int64_t ld_dst,
                       int B, T alpha, T beta, T gamma, int beta_mode, bool scaled,
                       hipStream_t s, bool bf16, const T *R, int64_t ldR, const T *rcoef,
-                      void *ext_scratch, int choice) {
+                      void *ext_scratch, int choice, size_t ext_bytes) {
   if (choice <= 0) choice = B;
   CHFSI_ARG(!bf16 || sizeof(T) == 4, "the BF16 apply works on FP32 multivectors");
   CHFSI_ARG(!R || (!bf16 && sizeof(T) == 4 && rcoef && ldR >= B), "bad defect source");
@@ -867,7 +867,8 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
   const bool tensor = set_tile < 0 && !bf16 && op->tensor_pot &&
                       ld_src < (int64_t(1) << 29) && ld_dst < (int64_t(1) << 29) &&
                       ldR < (int64_t(1) << 29) &&  // the kernels' row offsets are 32-bit bytes
-                      tensor_wins(op->tn, sizeof(T) == 8, op->max_color_cells, choice);
+                      tensor_wins(op->tn, sizeof(T) == 8, op->max_color_cells, choice,
+                                  op->d_touch_ptr && op->n_slots > 0);
   a.R = R;
   a.ldR = ldR;
   a.rcoef = rcoef;
@@ -890,16 +891,41 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
     if (captured) a.form = op->d_form;
     a.want = kTensorForm;
   }
-  if (tensor && !ext_scratch) {
-    // small blocks: one launch over all cells and a sum, where the operator
-    // holds a buffer for it (as its projections' scratch, one per precision)
+  // small blocks: one launch over all cells and a sum, where there is a buffer for
+  // the cells' sums (as for the projections: the operator's, one per
+  // precision, or the rest of the caller's scratch, which may take several steps)
+  T *co = nullptr;
+  int step = 0;
+  if (tensor && op->d_touch_ptr && op->n_slots > 0 &&
+      tensor_all_cells(op->tn, sizeof(T) == 8, op->max_color_cells, B)) {
+    if (!ext_scratch) {
+      co = OpData<T>::cells_out(op);
+      step = co ? B : 0;
+    } else {
+      const size_t used =
+          (noalloc_scratch_bytes(sizeof(T), op->n_slots, op->n_proj, B) + 255) / 256 * 256;
+      const size_t fit =
+          ext_bytes > used ? (ext_bytes - used) / (sizeof(T) * size_t(op->C) * op->ne) : 0;
+      co = reinterpret_cast<T *>(static_cast<char *>(ext_scratch) + used);
+      step = fit >= size_t(B) ? B : int(fit / 32 * 32);
+    }
+  }
+  all_cells = step > 0;
+  if (all_cells) {
     TensorTouch touch{op->d_touch_ptr, op->d_touch_idx, op->M};
-    T *co = OpData<T>::cells_out(op);
-    all_cells = co && tensor_all_cells(op->tn, sizeof(T) == 8, op->max_color_cells, B);
-    if (all_cells) {
-      a.cells = op->d_cells_by_color;
-      a.ncells = op->C;
-      CHFSI_HIP(launch_hx_tensor<T>(a, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq,
+    a.cells = op->d_cells_by_color;
+    a.ncells = op->C;
+    for (int c0 = 0; c0 < B; c0 += step) {
+      HxLaunch<T> b = a;
+      b.B = std::min(step, B - c0);
+      b.src += c0;
+      b.dst += c0;
+      b.W += c0;
+      if (R) {
+        b.R += c0;
+        b.rcoef += c0;
+      }
+      CHFSI_HIP(launch_hx_tensor<T>(b, OpData<T>::vq(op), OpData<T>::ttab(op), op->tn, op->tq,
                                     &touch, co, s));
     }
   }
@@ -943,10 +969,11 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
 template chfsi_status hx_fused<double>(chfsi_operator *, const double *, int64_t, double *,
                                        int64_t, int, double, double, double, int, bool,
                                        hipStream_t, bool, const double *, int64_t,
-                                       const double *, void *, int);
+                                       const double *, void *, int, size_t);
 template chfsi_status hx_fused<float>(chfsi_operator *, const float *, int64_t, float *, int64_t,
                                       int, float, float, float, int, bool, hipStream_t, bool,
-                                      const float *, int64_t, const float *, void *, int);
+                                      const float *, int64_t, const float *, void *, int,
+                                      size_t);
 
 }  // namespace chfsi
 
@@ -977,7 +1004,7 @@ extern "C" chfsi_status chfsi_hx_noalloc(chfsi_operator *op, const double *src, 
   }
   CHFSI_TRY(hx_fused<double>(op, src, ld_src, dst, ld_dst, B, scalar, 1.0, 0.0,
                              scale_flag ? 0 : 2, true, as_stream(stream), false, nullptr, 0,
-                             nullptr, ws));
+                             nullptr, ws, 0, kNoAllocScratchBytes));
   if (op->nc > 0) CHFSI_HIP(launch_zero_rows(op->d_c_rows, op->nc, dst, ld_dst, B, as_stream(stream)));
   return CHFSI_OK;
 }

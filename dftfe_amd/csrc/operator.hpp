@@ -40,7 +40,8 @@ template <typename T>
 chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, int64_t ld_dst,
                       int B, T alpha, T beta, T gamma, int beta_mode, bool scaled, hipStream_t s,
                       bool bf16 = false, const T *R = nullptr, int64_t ldR = 0,
-                      const T *rcoef = nullptr, void *ext_scratch = nullptr, int choice = 0);
+                      const T *rcoef = nullptr, void *ext_scratch = nullptr, int choice = 0,
+                      size_t ext_bytes = 0);
 
 // g (+)= wscale JxW sum_v w_v (N.(s a_v))(N.(s b_v)) per (cell, quadrature
 // point), s = M^{-1/2} when scaled; with general constraints the rows of a and

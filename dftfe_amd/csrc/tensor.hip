@@ -1304,9 +1304,14 @@ static hipError_t hx_tensor_vec(const HxLaunch<T> &a, const T *vq, const T *tab,
 //   n = 6: 1728 cells x 256 columns 1.06 / 1.50 FP64, 0.58 / 0.80 FP32, x 1 0.16 / 0.29
 //   n = 5: the dense product is only 1.7 times the operations, on the matrix
 //          pipe; the tensor form has fewer bytes in flight behind its barriers
-//          and wins while a colour does not fill the chip: 512 cells x 64 columns
-//          0.09 / 0.19 FP64, 0.06 / 0.13 FP32, x 200 0.216 / 0.218 and 0.13 / 0.21,
-//          x 1 0.05 / 0.12; 1728 x 256 0.77 / 0.62 and 0.44 / 0.38
+//          and wins while a colour does not fill the chip.  us per apply, tensor /
+//          dense at workgroups a colour: FP64 256 141 / 196, 384 194 / 210, 432
+//          215 / 204, 512 253 / 216; FP32 432 133 / 203, 640 213 / 220, 768
+//          220 / 223, 864 275 / 230, 1024 301 / 229; without projectors FP64
+//          432 150 / 167, 448 149 / 152.  One column, all cells at once:
+//          64 cells a colour 50 / 120; colour by colour (no projectors) the
+//          matrix-vector kernel is faster on few cells: FP64 27 92 / 83, 64 89 / 93;
+//          FP32 64 70 / 69, 216 71 / 83
 static int tile_columns(int n, bool fp64) { return n == 7 && fp64 ? 16 : 32; }
 
 static int64_t colour_items(int n, bool fp64, int cells, int B) {
@@ -1314,10 +1319,11 @@ static int64_t colour_items(int n, bool fp64, int cells, int B) {
   return int64_t(cells) * ((B + tc - 1) / tc);
 }
 
-bool tensor_wins(int n, bool fp64, int cells, int B) {
+bool tensor_wins(int n, bool fp64, int cells, int B, bool all) {
   if (n > 5) return true;
   const int64_t items = colour_items(n, fp64, cells, B);
-  return items <= (fp64 || B == 1 ? kAllCellsItems : 1024);
+  if (B == 1) return items <= kAllCellsItems && (all || cells >= (fp64 ? 64 : 128));
+  return items <= (fp64 ? (all ? 400 : 448) : 640);
 }
 
 // One launch over all cells and a sum (all) against the colour launches: a launch

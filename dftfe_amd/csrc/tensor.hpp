@@ -17,8 +17,8 @@ namespace chfsi {
 bool tensor_shape(int ne, int nqc, int *n, int *q);
 
 // Whether the tensor form is the faster one on B columns, from the cells of the
-// largest colour
-bool tensor_wins(int n, bool fp64, int cells, int B);
+// largest colour; all: the operator can run all cells at once
+bool tensor_wins(int n, bool fp64, int cells, int B, bool all);
 
 // workgroups of a colour up to which one launch over all cells is the faster apply
 constexpr int kAllCellsItems = 448;

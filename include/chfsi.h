@@ -301,12 +301,13 @@ chfsi_status chfsi_hx(chfsi_operator *op, const double *src, int64_t ld_src, dou
 
 /* chfsi_hx without any device allocation.  No counterpart in the reference:
  * for callers that cannot allocate (code under HIP graph capture, tight
- * serving loops, harnesses that forbid hipMalloc).  Same arguments, kernels
- * and results (bit for bit) as chfsi_hx; the nonlocal projection scratch,
+ * serving loops, harnesses that forbid hipMalloc).  Same arguments and
+ * results (bit for bit) as chfsi_hx; the nonlocal projection scratch,
  * n_slots*B + n_proj*B doubles (plus 256-byte alignment), lives in a fixed
- * 64 MiB device array per GPU instead of operator-owned buffers, and larger
- * blocks are rejected with CHFSI_ERR_ARG.  Every call on one GPU shares that
- * array: calls that overlap on one GPU (other streams, other threads) race. */
+ * 64 MiB device array per GPU instead of operator-owned buffers (small blocks
+ * use what is left of it for the cells' sums), and larger blocks are rejected
+ * with CHFSI_ERR_ARG.  Every call on one GPU shares that array: calls that
+ * overlap on one GPU (other streams, other threads) race. */
 chfsi_status chfsi_hx_noalloc(chfsi_operator *op, const double *src, int64_t ld_src,
                               double *dst, int64_t ld_dst, int32_t B, int32_t scale_flag,
                               double scalar, void *stream);

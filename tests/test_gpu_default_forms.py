@@ -1,5 +1,7 @@
 """The apply and the projection that an operator chooses by itself: a caller can return
 to them from a set variant, and the workloads' committed passes hold for them."""
+import ctypes as ct
+import dataclasses
 import json
 import os
 import sys
@@ -104,3 +106,48 @@ def test_autotune_keeps_both_forms(name, B, prec, dtype, gga_first):
     assert torch.equal(op.apply(X), gga)
     op.set_potential(prob.vJxW)
     assert torch.equal(op.apply(X), lda)
+
+
+# (columns, precision, cells per side, projectors, whether the dense form is the faster)
+LINES = [(512, L.FP32, 8, True, True), (320, L.FP32, 8, True, False), (448, L.FP64, 6, True, False),
+         (224, L.FP64, 8, True, True), (192, L.FP64, 8, True, False), (1, L.FP64, 6, False, True),
+         (1, L.FP32, 8, False, True), (1, L.FP64, 8, False, False), (1, L.FP64, 6, True, False),
+         (2, L.FP64, 6, False, False), (224, L.FP64, 8, False, False)]
+
+
+@pytest.mark.parametrize("B,prec,n,projectors,dense", LINES)
+def test_lines_between_the_forms_at_p4(B, prec, n, projectors, dense):
+    """Each side of the lines at which the p = 4 apply leaves the tensor form."""
+    from dftfe_amd.chfsi import KohnShamOperatorDevice
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    prob = fe.build_problem(fe.Workload("lines", 2.5 * n, n, 4, 5, 8, 1, 1, 1, seed=60 + n))
+    if not projectors:
+        prob = dataclasses.replace(prob, pair_atom=prob.pair_atom[:0],
+                                   pair_cell=prob.pair_cell[:0], pair_C=prob.pair_C[:0])
+    op = KohnShamOperatorDevice(prob)
+    dtype = torch.float64 if prec == L.FP64 else torch.float32
+    X = torch.tensor(prob.initial_guess(N=B, seed_offset=B), device="cuda", dtype=dtype)
+    Y = op.apply(X)
+    op.set_hx_variant(prec, 0)
+    tile = op.apply(X)
+    assert torch.equal(Y, tile) == dense
+    assert ((Y - tile).abs().max() / tile.abs().max()).item() < (1e-13 if prec == L.FP64 else 2e-6)
+
+
+@pytest.mark.parametrize("name,B", [("cube20_p4_n64", 1), ("cube20_p4_n64", 33),
+                                    ("cube20_p4_n64", 160), ("cube20_p4_n64", 190),
+                                    ("cube18_p5_n64", 70), ("cube18_p6_n64", 1)])
+def test_no_allocation_form_in_steps(name, B):
+    """chfsi_hx_noalloc runs all cells at once where its scratch holds their sums, in
+    steps of columns if need be, with chfsi_hx's bits."""
+    prob, op = _operator(name)
+    X = torch.tensor(prob.initial_guess(N=B, seed_offset=B), device="cuda")
+    D = torch.tensor(prob.initial_guess(N=B, seed_offset=B + 1), device="cuda")
+    want, got = D.clone(), D.clone()
+    st = ct.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for f, Y in ((op.lib.chfsi_hx, want), (op.lib.chfsi_hx_noalloc, got)):
+        L.check(f(op.handle, ct.c_void_p(X.data_ptr()), B, ct.c_void_p(Y.data_ptr()), B, B, 0,
+                  -0.75, st))
+    assert torch.equal(got, want)
