@@ -124,6 +124,11 @@ class KohnShamOperatorDevice:
             self.lib.chfsi_operator_destroy(self.handle)
             self.handle = None
 
+    def release_workspace(self) -> None:
+        """Gives back the scratch that the calls without a solver keep with the operator
+        (up to 8 GiB each, 32 GiB for all operators of a GPU)."""
+        L.check(self.lib.chfsi_operator_release_workspace(self.handle))
+
     # -- setup --------------------------------------------------------------
     def set_potential(self, vJxW: np.ndarray) -> None:
         """computeHamiltonianMatricesAllkpt: cell matrices from V_eff JxW on device."""

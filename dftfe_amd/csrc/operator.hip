@@ -32,11 +32,20 @@ void set_error(const char *fmt, ...) {
   g_last_error = buf;
 }
 
+hipError_t device_malloc(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && release_idle_workspaces()) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 template <typename T>
 static chfsi_status dev_upload(T **d, const T *h, size_t n) {
   *d = nullptr;
   if (n == 0) return CHFSI_OK;
-  if (hipMalloc(reinterpret_cast<void **>(d), n * sizeof(T)) != hipSuccess) {
+  if (device_malloc(reinterpret_cast<void **>(d), n * sizeof(T)) != hipSuccess) {
     set_error("hipMalloc of %zu bytes failed", n * sizeof(T));
     return CHFSI_ERR_NOMEM;
   }
@@ -54,7 +63,7 @@ chfsi_status Scratch::ensure(size_t bytes) {
   if (ptr) hipFree(ptr);
   ptr = nullptr;
   size = 0;
-  if (hipMalloc(&ptr, bytes) != hipSuccess) {
+  if (device_malloc(&ptr, bytes) != hipSuccess) {
     set_error("hipMalloc of %zu bytes failed", bytes);
     return CHFSI_ERR_NOMEM;
   }

@@ -4,13 +4,16 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <memory>
-#include <mutex>
 #include <vector>
 
 #include "common.hpp"
 
 namespace chfsi {
+
+// hipMalloc; without room it gives back the kept workspaces and tries again
+hipError_t device_malloc(void **p, size_t bytes);
 
 // Grow-only device buffer.
 struct Scratch {
@@ -158,9 +161,11 @@ struct chfsi_operator {
   float *d_nlCtko32 = nullptr;
   int zproj_variant = 1;
   int zhx_variant64 = 0, zhx_variant32 = 0;
-  // workspace of the entry points without a solver (see Workspace)
-  std::mutex work_mutex;
+  // workspace of the entry points without a solver (see Workspace), and its bytes
+  // when it was last put down
+  std::atomic<bool> work_busy{false};
   chfsi_solver *work = nullptr;
+  size_t work_bytes = 0;
   hipEvent_t work_done = nullptr;
   chfsi::Scratch ztab_dev, ztab_W, ztab_P;  // tables and scratch of single complex applies
 
@@ -168,8 +173,10 @@ struct chfsi_operator {
 };
 
 namespace chfsi {
-// Frees the operator's kept workspace
+// Frees the operator's kept workspace (no call may be using it)
 void release_workspace(chfsi_operator *op);
+// Frees the kept workspaces that no call is using; whether there were any
+bool release_idle_workspaces();
 // Rebuilds the complex cell matrices of every k-point from the real tiles.
 chfsi_status rebuild_kpoint_matrices(chfsi_operator *op, hipStream_t s);
 }  // namespace chfsi

@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <new>
 #include <vector>
 
@@ -997,16 +998,36 @@ extern "C" chfsi_status chfsi_solver_set_lanczos_start(chfsi_solver *s, const do
   return CHFSI_OK;
 }
 
+namespace {
+// Operators with a workspace put down, the one used last at the end.  Never
+// destroyed: operators may go at the program's end.
+struct KeptWorkspaces {
+  std::mutex m;
+  std::vector<chfsi_operator *> ops;
+  // of an operator whose workspace no call is using, with m held
+  void drop(chfsi_operator *op) {
+    delete op->work;  // hipFree waits for the work
+    op->work = nullptr;
+    op->work_bytes = 0;
+    ops.erase(std::remove(ops.begin(), ops.end(), op), ops.end());
+  }
+};
+KeptWorkspaces &kept() {
+  static KeptWorkspaces *k = new KeptWorkspaces;
+  return *k;
+}
+}  // namespace
+
 namespace chfsi {
 Workspace::Workspace(chfsi_operator *op, hipStream_t st) : op_(op), st_(st) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
-  if (!op->work_mutex.try_lock()) return;
+  if (op->work_busy.exchange(true)) return;
   if (!op->work_done && hipEventCreateWithFlags(&op->work_done, hipEventDisableTiming) != hipSuccess)
     op->work_done = nullptr;
   if (!op->work) op->work = new (std::nothrow) chfsi_solver();
   if (!op->work_done || !op->work || hipStreamWaitEvent(st, op->work_done, 0) != hipSuccess) {
-    op->work_mutex.unlock();
+    op->work_busy = false;
     return;
   }
   held_ = true;
@@ -1015,22 +1036,72 @@ Workspace::Workspace(chfsi_operator *op, hipStream_t st) : op_(op), st_(st) {
 
 Workspace::~Workspace() {
   if (!held_) return;
-  size_t bytes = 0;
+  bool keep = hipEventRecord(op_->work_done, st_) == hipSuccess;
+  size_t bytes = 0, others = 0, avail = 0, total = 0;
   for (Scratch *b : s_->scratch()) bytes += b->size;
-  if (bytes > kKeep || hipEventRecord(op_->work_done, st_) != hipSuccess) {
-    delete op_->work;  // hipFree waits for the work
-    op_->work = nullptr;
+  keep = keep && bytes <= kKeep;
+  if (keep && bytes > kSmall)
+    keep = hipMemGetInfo(&avail, &total) == hipSuccess && avail >= total / 4;
+  {
+    KeptWorkspaces &k = kept();
+    std::lock_guard<std::mutex> lock(k.m);
+    for (chfsi_operator *o : k.ops)
+      if (o != op_ && o->device == op_->device) others += o->work_bytes;
+    // room for this one: the others go, the one unused for longest first
+    for (size_t i = 0; keep && bytes + others > kKeepAll && i < k.ops.size();) {
+      chfsi_operator *o = k.ops[i];
+      if (o == op_ || o->device != op_->device || o->work_busy.exchange(true)) {
+        ++i;
+        continue;
+      }
+      others -= o->work_bytes;
+      k.drop(o);
+      o->work_busy = false;
+    }
+    k.ops.erase(std::remove(k.ops.begin(), k.ops.end(), op_), k.ops.end());
+    if (keep && bytes + others <= kKeepAll) {
+      op_->work_bytes = bytes;
+      k.ops.push_back(op_);
+    } else {
+      k.drop(op_);
+    }
   }
-  op_->work_mutex.unlock();
+  op_->work_busy = false;
 }
 
 void release_workspace(chfsi_operator *op) {
-  delete op->work;
-  op->work = nullptr;
+  KeptWorkspaces &k = kept();
+  std::lock_guard<std::mutex> lock(k.m);
+  k.drop(op);
   if (op->work_done) (void)hipEventDestroy(op->work_done);
   op->work_done = nullptr;
 }
+
+bool release_idle_workspaces() {
+  KeptWorkspaces &k = kept();
+  std::lock_guard<std::mutex> lock(k.m);
+  const std::vector<chfsi_operator *> ops = k.ops;
+  bool any = false;
+  for (chfsi_operator *o : ops) {
+    if (o->work_busy.exchange(true)) continue;
+    any = any || o->work_bytes > 0;
+    k.drop(o);
+    o->work_busy = false;
+  }
+  return any;
+}
 }  // namespace chfsi
+
+extern "C" chfsi_status chfsi_operator_release_workspace(chfsi_operator *op) {
+  CHFSI_ARG(op, "null operator");
+  if (op->work_busy.exchange(true)) {
+    set_error("the operator's workspace is in use by another thread");
+    return CHFSI_ERR_STATE;
+  }
+  release_workspace(op);
+  op->work_busy = false;
+  return CHFSI_OK;
+}
 
 extern "C" chfsi_status chfsi_chebyshev_filter(chfsi_operator *op, double *X, int64_t ld,
                                                int32_t B, int32_t m, double a, double b,

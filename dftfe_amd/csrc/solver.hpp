@@ -74,8 +74,14 @@ namespace chfsi {
 // blocks and BLAS handle (each hipFree waits for the device; freeing the 6.6 GB
 // of a 256-column reverse pass takes tens of ms).  Another thread's call in the
 // meantime, and calls on a stream under capture, get one of their own; a call on
-// another stream waits for the last one's work.  More than 8 GiB are given back
-// at the end of the call, the rest with the operator.
+// another stream waits for the last one's work, as it did when each call ended
+// with the device idle (hipFree).  A workspace of more than 8 GiB is given back at
+// the end of the call, and one of more than 256 MiB (hipMemGetInfo takes longer than
+// the smaller calls) unless a quarter of the device's memory is free.  The operators
+// of a device keep 32 GiB together, those unused for longest making room: with 8,
+// reverse passes of 256 columns taking turns on three operators freed each other's
+// (39.5 against 37.7 ms).  Workspaces also go when an allocation of the library
+// fails, with chfsi_operator_release_workspace, and with the operator.
 class Workspace {
  public:
   Workspace(chfsi_operator *op, hipStream_t st);
@@ -85,7 +91,8 @@ class Workspace {
   chfsi_solver *get() { return s_; }
 
  private:
-  static constexpr size_t kKeep = size_t(8) << 30;
+  static constexpr size_t kKeep = size_t(8) << 30, kKeepAll = size_t(32) << 30,
+                          kSmall = size_t(256) << 20;
   chfsi_operator *op_;
   hipStream_t st_;
   chfsi_solver local_, *s_ = &local_;

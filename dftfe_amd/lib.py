@@ -86,6 +86,7 @@ SIGNATURES = {
                                           c_int32_p]),
     "chfsi_operator_create": (ct.c_int, [ct.POINTER(OperatorDesc), ct.POINTER(_VP)]),
     "chfsi_operator_destroy": (None, [_VP]),
+    "chfsi_operator_release_workspace": (ct.c_int, [_VP]),
     "chfsi_operator_set_potential": (ct.c_int, [_VP, _VP, _VP]),
     "chfsi_operator_set_potential_gga": (ct.c_int, [_VP, _VP, _VP, _VP]),
     "chfsi_operator_set_cell_matrices": (ct.c_int, [_VP, _VP, _VP]),

@@ -242,6 +242,16 @@ chfsi_status chfsi_chebyshev_degree(const chfsi_params *params, double bUp, int3
 chfsi_status chfsi_operator_create(const chfsi_operator_desc *desc, chfsi_operator **op);
 void chfsi_operator_destroy(chfsi_operator *op);
 
+/* The entry points without a solver (filter, Lanczos, CholGS, Rayleigh-Ritz,
+ * residuals, their complex forms, the filter's reverse pass) keep their scratch
+ * with the operator between calls: up to 8 GiB each and 32 GiB for all operators
+ * of a GPU, those unused for longest giving way; more than 256 MiB only while a
+ * quarter of the GPU's memory is free.  It is given back where an allocation of
+ * the library fails.  This gives the operator's back, for instance before
+ * another allocator needs the memory (CHFSI_ERR_STATE while another thread is in
+ * such a call). */
+chfsi_status chfsi_operator_release_workspace(chfsi_operator *op);
+
 /* Cell Hamiltonian build from V_eff*JxW at quadrature points (device, C*n_q):
  * H_e = 1/2 K_e + N^T diag(vJxW_c) N.  Replaces computeHamiltonianMatricesAllkpt
  * / hamMatrixKernelLDA (hamiltonianMatrixCalculatorFlattenedDevice.cc:61-116, :1073-1375). */
