@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <limits>
 
 #include "mfma.hpp"
 #include "scatter.hpp"
@@ -163,14 +164,114 @@ bool gradient_products(const double *G, const std::vector<ld> &I, int n, int q, 
 }
 }  // namespace
 
+namespace {
+// Corrects the quadrature weights w so that I^T diag(w) I is closest to M: K_z is weighted
+// by w at the points of x and y, where K_x and K_y take M itself, and an error of w
+// acts alike in every cell.
+void fit_weights(const std::vector<ld> &I, const std::vector<ld> &M, int n, int q,
+                 std::vector<ld> &w) {
+  // normal equations [q][q + 1]: A_kl = (I_k . I_l)^2, b_k = I_k^T M I_k - A w
+  std::vector<ld> A(size_t(q) * (q + 1), 0);
+  for (int k = 0; k < q; ++k) {
+    ld *row = &A[k * (q + 1)];
+    for (int a = 0; a < n; ++a)
+      for (int b = 0; b < n; ++b) row[q] += I[k * n + a] * M[a * n + b] * I[k * n + b];
+    for (int l = 0; l < q; ++l) {
+      ld s = 0;
+      for (int a = 0; a < n; ++a) s += I[k * n + a] * I[l * n + a];
+      row[l] = s * s;
+      row[q] -= row[l] * w[l];
+    }
+  }
+  for (int c = 0; c < q; ++c) {
+    int piv = c;
+    for (int r = c + 1; r < q; ++r)
+      if (fabsl(A[r * (q + 1) + c]) > fabsl(A[piv * (q + 1) + c])) piv = r;
+    for (int k = 0; k <= q; ++k) std::swap(A[c * (q + 1) + k], A[piv * (q + 1) + k]);
+    for (int r = 0; r < q; ++r) {
+      if (r == c) continue;
+      const ld f = A[r * (q + 1) + c] / A[c * (q + 1) + c];
+      for (int k = c; k <= q; ++k) A[r * (q + 1) + k] -= f * A[c * (q + 1) + k];
+    }
+  }
+  for (int c = 0; c < q; ++c) w[c] += A[c * (q + 1) + q] / A[c * (q + 1) + c];
+}
+
+// The mass and stiffness tables of K = D_x M M + M D_y M + M M D_z ([a * n + b]) that
+// fit it best, from a start near them: K contracted with M in one direction and with M,
+// or with the part of a D that is orthogonal to M, in another leaves the table of
+// the third (the D up to multiples of M, which are fixed by a constant having no
+// energy).  Two rounds reach rounding.
+void fit_stiffness(const double *K, int n, std::vector<ld> &M, std::vector<ld> (&D)[3]) {
+  const int nn = n * n, ne = nn * n;
+  const Index3 in(n);
+  // rows of A times b, columns of A times b (A: nn x nn)
+  auto right = [nn](const std::vector<ld> &A, const std::vector<ld> &b, ld f, std::vector<ld> &out) {
+    for (int e = 0; e < nn; ++e)
+      for (int k = 0; k < nn; ++k) out[e] += f * A[e * nn + k] * b[k];
+  };
+  auto left = [nn](const std::vector<ld> &A, const std::vector<ld> &b, ld f, std::vector<ld> &out) {
+    for (int k = 0; k < nn; ++k)
+      for (int e = 0; e < nn; ++e) out[e] += f * A[k * nn + e] * b[k];
+  };
+  auto dot = [nn](const std::vector<ld> &a, const std::vector<ld> &b) {
+    ld s = 0;
+    for (int e = 0; e < nn; ++e) s += a[e] * b[e];
+    return s;
+  };
+  const std::vector<ld> one(nn, 1);
+  for (int round = 0; round < 2; ++round) {
+    // K times M in z, y, x: [ex][ey], [ex][ez], [ey][ez]
+    std::vector<ld> xy(nn * nn, 0), xz(nn * nn, 0), yz(nn * nn, 0);
+    for (int i = 0; i < ne; ++i)
+      for (int j = 0; j < ne; ++j) {
+        const int ex = in.x[i] * n + in.x[j], ey = in.y[i] * n + in.y[j],
+                  ez = in.z[i] * n + in.z[j];
+        const ld v = K[size_t(i) * ne + j];
+        xy[ex * nn + ey] += v * M[ez];
+        xz[ex * nn + ez] += v * M[ey];
+        yz[ey * nn + ez] += v * M[ex];
+      }
+    const ld mm = dot(M, M);
+    for (auto &d : D) d.assign(nn, 0);
+    right(xy, M, 1 / (mm * mm), D[0]);
+    left(xy, M, 1 / (mm * mm), D[1]);
+    left(xz, M, 1 / (mm * mm), D[2]);
+    ld off[3], rest = 2 * dot(D[0], M) / mm;
+    for (int d = 0; d < 3; ++d) rest -= off[d] = dot(D[d], one) / dot(M, one);
+    std::vector<ld> P[3], next(nn, 0);
+    for (int d = 0; d < 3; ++d) {
+      for (int e = 0; e < nn; ++e) D[d][e] -= (off[d] + rest / 3) * M[e];
+      const ld f = dot(D[d], M) / mm;
+      P[d] = D[d];
+      for (int e = 0; e < nn; ++e) P[d][e] -= f * M[e];
+    }
+    ld w[3];
+    for (int d = 0; d < 3; ++d) w[d] = 1 / (6 * dot(P[d], P[d]) * mm);
+    right(xy, P[1], w[1], next);
+    right(xz, P[2], w[2], next);
+    left(xy, P[0], w[0], next);
+    right(yz, P[2], w[2], next);
+    left(xz, P[0], w[0], next);
+    left(yz, P[1], w[1], next);
+    M = next;
+  }
+}
+}  // namespace
+
 bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, int nqc,
                    std::vector<double> *tab, std::vector<float> *tab32,
                    std::vector<double> *products) {
   int n = 0, q = 0;
   if (!tensor_shape(ne, nqc, &n, &q)) return false;
-  const double tol = 1e-13;
+  // rounding: products of three tables are within 5 eps of shape values and
+  // gradients evaluated point by point, and within 2-6 eps of a stiffness from
+  // one-dimensional tables or matrix products, 31 of one summed point after point
+  // (512 points)
+  const double eps = std::numeric_limits<double>::epsilon();
+  const double tol = 32 * eps, tol_k = 128 * eps;
   const Index3 in(n), iq(q);
-  const std::vector<ld> w = gauss_weights(q);
+  std::vector<ld> w = gauss_weights(q);
   // I: sums of N over the nodes of the other two directions (which are one),
   // mean over their quadrature points and over the directions; x is the
   // fastest index of nodes and points
@@ -194,19 +295,12 @@ bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, i
   for (int a = 0; a < n; ++a)
     for (int b = 0; b < n; ++b)
       for (int k = 0; k < q; ++k) M[a * n + b] += w[k] * I[k * n + a] * I[k * n + b];
-  // stiffness of each direction: the mass tables sum to one over the other
-  // two, the stiffness tables to zero
-  for (auto &A : Kd) A.assign(size_t(n) * n, 0);
   double kmax = 0;
-  for (int i = 0; i < ne; ++i)
-    for (int j = 0; j < ne; ++j) {
-      const ld v = K[size_t(i) * ne + j];
-      kmax = std::max(kmax, std::fabs((double)v));
-      Kd[0][in.x[i] * n + in.x[j]] += v;
-      Kd[1][in.y[i] * n + in.y[j]] += v;
-      Kd[2][in.z[i] * n + in.z[j]] += v;
-    }
+  for (size_t i = 0; i < size_t(ne) * ne; ++i) kmax = std::max(kmax, std::fabs(K[i]));
+  fit_stiffness(K, n, M, Kd);
+  symmetrise(M);
   for (auto &A : Kd) symmetrise(A);
+  fit_weights(I, M, n, q, w);
   const std::vector<double> Id(I.begin(), I.end()), Md(M.begin(), M.end());
   const std::vector<double> Kd0(Kd[0].begin(), Kd[0].end()), Kd1(Kd[1].begin(), Kd[1].end()),
       Kd2(Kd[2].begin(), Kd[2].end());
@@ -222,7 +316,7 @@ bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, i
                 ez = in.z[i] * n + in.z[j];
       const double v =
           Kd0[ex] * Md[ey] * Md[ez] + Md[ex] * Kd1[ey] * Md[ez] + Md[ex] * Md[ey] * Kd2[ez];
-      if (!(std::fabs(K[size_t(i) * ne + j] - v) <= tol * kmax)) return false;
+      if (!(std::fabs(K[size_t(i) * ne + j] - v) <= tol_k * kmax)) return false;
     }
   // parity tables; the operator applies half the stiffness
   const int NE = (n + 1) / 2, NO = n / 2, QE = (q + 1) / 2, QO = q / 2;

@@ -29,7 +29,7 @@ int tensor_all_cells_columns(int n, bool fp64, int cells);
 
 // Host check of an operator's shape values (nqc x ne) and stiffness (ne x ne):
 // true when every entry is the product of one-dimensional, centro-symmetric
-// tables (Gauss quadrature) to 1e-13 of the largest one.  Fills the kernels'
+// tables (Gauss quadrature) to rounding.  Fills the kernels'
 // tables, FP64 and FP32, and the products of the cell matrix build (n^2 q, or
 // 4 n^2 q when the shape gradients G (nqc x ne x 3, nullable) have that form too).
 bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, int nqc,
