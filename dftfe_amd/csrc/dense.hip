@@ -134,8 +134,9 @@ __global__ __launch_bounds__(NT, 2) void gram_kernel(const double *A, int64_t ld
   const int wi = w & 1, wj = w >> 1;
 
   // staging: thread t loads row t/16 of the slab, the column pairs 2 (t%16) + 32 e (16
-  // lanes a line of memory and all banks of LDS).  Indices past the block are clamped and the values dropped when they are stored, so
-  // nothing waits for a load before the MFMAs of the slab in between.
+  // lanes a line of memory and all banks of LDS).  Indices past the block are clamped
+  // and the values dropped when they are stored, so nothing waits for a load before
+  // the MFMAs of the slab in between.
   const int lr = tid >> 4, lc = (tid & 15) * 2;
   double2 ra[4], rb[4];
   auto load = [&](int64_t k0) {
@@ -427,7 +428,8 @@ hipError_t launch_gram(const double *A, int64_t lda, const double *B, int64_t ld
 }
 
 hipError_t launch_rotate(const double *X, int64_t ldx, const double *Rm, int64_t ldr, int trans,
-                         int K, int diag, int N, int64_t rows, double *Y, int64_t ldy, hipStream_t s) {
+                         int K, int diag, int N, int64_t rows, double *Y, int64_t ldy,
+                         hipStream_t s) {
   if (rows <= 0 || N <= 0 || K <= 0) return hipSuccess;
   const int ntj = (N + TT - 1) / TT;
   const int64_t nti = (rows + TT - 1) / TT;
@@ -438,8 +440,8 @@ hipError_t launch_rotate(const double *X, int64_t ldx, const double *Rm, int64_t
   const bool vec = pairs(X, ldx, K) && pairs(Rm, ldr, trans ? N : K);
   hipLaunchKernelGGL((trans ? (vec ? rotate_kernel<1, true> : rotate_kernel<1, false>)
                             : (vec ? rotate_kernel<0, true> : rotate_kernel<0, false>)),
-                     dim3(8 * per_xcd), dim3(NT), 0, s, X, ldx, Rm, ldr, K, diag, N, rows, Y, ldy, ntj,
-                     per_xcd, nitems);
+                     dim3(8 * per_xcd), dim3(NT), 0, s, X, ldx, Rm, ldr, K, diag, N, rows, Y, ldy,
+                     ntj, per_xcd, nitems);
   return hipGetLastError();
 }
 

@@ -42,6 +42,7 @@ constexpr int kRotateTile = 128;
 // for i > diag + j (diag >= K: none need be).  Y must not overlap X unless N <= kRotateTile
 // and Y's columns are among the K of X (row for row: in place).
 hipError_t launch_rotate(const double *X, int64_t ldx, const double *Rm, int64_t ldr, int trans,
-                         int K, int diag, int N, int64_t rows, double *Y, int64_t ldy, hipStream_t s);
+                         int K, int diag, int N, int64_t rows, double *Y, int64_t ldy,
+                         hipStream_t s);
 
 }  // namespace chfsi

@@ -334,8 +334,10 @@ extern "C" chfsi_status chfsi_operator_create(const chfsi_operator_desc *d, chfs
         for (int64_t g = 0; g < M; ++g) tptr[g + 1] += tptr[g];
         std::vector<uint32_t> fill(tptr.begin(), tptr.end() - 1);
         for (int k = 0; k < C; ++k)
-          for (int i = 0; i < ne; ++i)
-            tidx[fill[map[size_t(cells_sorted[k]) * ne + i] & 0x7fffffffu]++] = uint32_t(k * ne + i);
+          for (int i = 0; i < ne; ++i) {
+            const uint32_t g = map[size_t(cells_sorted[k]) * ne + i] & 0x7fffffffu;
+            tidx[fill[g]++] = uint32_t(k * ne + i);
+          }
         CHFSI_TRY(dev_upload(&op->d_touch_ptr, tptr.data(), tptr.size()));
         CHFSI_TRY(dev_upload(&op->d_touch_idx, tidx.data(), tidx.size()));
       }

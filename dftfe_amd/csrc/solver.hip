@@ -169,7 +169,8 @@ chfsi_status cheb_steps(chfsi_operator *op, T **cur, int64_t *ldc, T **prev, int
     const double sigma2 = 1.0 / (cs.gamma - cs.sigma);
     const double alpha1 = 2.0 * sigma2 / cs.e, alpha2 = -(cs.sigma * sigma2);
     CHFSI_TRY(hx_fused<T>(op, *cur, *ldc, *prev, *ldp, B, T(alpha1), T(alpha2),
-                          T(-cs.c * alpha1), 0, true, st, bf16, nullptr, 0, nullptr, hx_ws, choice));
+                          T(-cs.c * alpha1), 0, true, st, bf16, nullptr, 0, nullptr, hx_ws,
+                          choice));
     std::swap(*cur, *prev);
     std::swap(*ldc, *ldp);
     cs.sigma = sigma2;
@@ -1021,9 +1022,11 @@ KeptWorkspaces &kept() {
 namespace chfsi {
 Workspace::Workspace(chfsi_operator *op, hipStream_t st) : op_(op), st_(st) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
+  if (cap != hipStreamCaptureStatusNone) return;
   if (op->work_busy.exchange(true)) return;
-  if (!op->work_done && hipEventCreateWithFlags(&op->work_done, hipEventDisableTiming) != hipSuccess)
+  if (!op->work_done &&
+      hipEventCreateWithFlags(&op->work_done, hipEventDisableTiming) != hipSuccess)
     op->work_done = nullptr;
   if (!op->work) op->work = new (std::nothrow) chfsi_solver();
   if (!op->work_done || !op->work || hipStreamWaitEvent(st, op->work_done, 0) != hipSuccess) {
@@ -1122,8 +1125,8 @@ extern "C" chfsi_status chfsi_chebyshev_filter(chfsi_operator *op, double *X, in
 // accumulated in FP64 from FP64 interpolations of the FP32 vectors.
 namespace {
 template <typename T>
-chfsi_status filter_backward_impl(chfsi_solver *s, chfsi_operator *op, const double *X0, int64_t ldx,
-                                  const double *Ybar, int64_t ldy, int B, int m, double a,
+chfsi_status filter_backward_impl(chfsi_solver *s, chfsi_operator *op, const double *X0,
+                                  int64_t ldx, const double *Ybar, int64_t ldy, int B, int m, double a,
                                   double b, double a0, int every, double *Xbar, int64_t ldxb,
                                   double *g, hipStream_t st) {
   const int64_t M = op->M;
@@ -1223,11 +1226,11 @@ extern "C" chfsi_status chfsi_chebyshev_filter_backward(
   hipStream_t st = as_stream(stream);
   Workspace ws(op, st);
   if (precision == CHFSI_FP64)
-    return filter_backward_impl<double>(ws.get(), op, X0, ldx, Ybar, ldy, B, m, a, b, a0, every, Xbar, ldxb,
-                                        g, st);
+    return filter_backward_impl<double>(ws.get(), op, X0, ldx, Ybar, ldy, B, m, a, b, a0, every,
+                                        Xbar, ldxb, g, st);
   CHFSI_ARG(precision == CHFSI_FP32, "filter backward precision must be CHFSI_FP64 or CHFSI_FP32");
-  return filter_backward_impl<float>(ws.get(), op, X0, ldx, Ybar, ldy, B, m, a, b, a0, every, Xbar, ldxb, g,
-                                     st);
+  return filter_backward_impl<float>(ws.get(), op, X0, ldx, Ybar, ldy, B, m, a, b, a0, every, Xbar,
+                                     ldxb, g, st);
 }
 
 extern "C" chfsi_status chfsi_lanczos_bounds(chfsi_operator *op, const double *v0, int32_t steps,
@@ -1273,7 +1276,8 @@ extern "C" chfsi_status chfsi_rayleigh_ritz_spectrum_split(chfsi_operator *op, d
   Workspace ws(op, st);
   const int B = std::min<int>(block, N);
   CHFSI_TRY(cholgs_impl(ws.get(), X, M, N, B, false, false, st));
-  return rr_split_impl(ws.get(), op, X, M, N, n_core, B, Xfrac, ld_frac, eig_host, mixed_xthx != 0, st);
+  return rr_split_impl(ws.get(), op, X, M, N, n_core, B, Xfrac, ld_frac, eig_host, mixed_xthx != 0,
+                       st);
 }
 
 namespace {

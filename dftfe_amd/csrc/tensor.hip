@@ -23,8 +23,9 @@
 #include "scatter.hpp"
 #include "tensor.hpp"
 
-// Fused multiply-adds are written out: an instantiation for other widths must
-// not contract other sums, a column has the same bits in every block
+// Fused multiply-adds are written out: an instantiation for other widths must not
+// contract other sums.  Within this form a column has the same bits in every
+// block; the form, and the projection's tile, go by the columns of a whole pass.
 #pragma clang fp contract(off)
 
 namespace chfsi {
@@ -206,11 +207,13 @@ void fit_stiffness(const double *K, int n, std::vector<ld> &M, std::vector<ld> (
   const int nn = n * n, ne = nn * n;
   const Index3 in(n);
   // rows of A times b, columns of A times b (A: nn x nn)
-  auto right = [nn](const std::vector<ld> &A, const std::vector<ld> &b, ld f, std::vector<ld> &out) {
+  auto right = [nn](const std::vector<ld> &A, const std::vector<ld> &b, ld f,
+                    std::vector<ld> &out) {
     for (int e = 0; e < nn; ++e)
       for (int k = 0; k < nn; ++k) out[e] += f * A[e * nn + k] * b[k];
   };
-  auto left = [nn](const std::vector<ld> &A, const std::vector<ld> &b, ld f, std::vector<ld> &out) {
+  auto left = [nn](const std::vector<ld> &A, const std::vector<ld> &b, ld f,
+                   std::vector<ld> &out) {
     for (int k = 0; k < nn; ++k)
       for (int e = 0; e < nn; ++e) out[e] += f * A[k * nn + e] * b[k];
   };
@@ -485,11 +488,11 @@ struct TensorShape : TensorTab<N, Q> {
 typedef const __attribute__((address_space(4))) double *ctab;
 
 // (I_z^T diag(v) I_z + wk K_z) u on one line, in place
-template <typename T, int N, int Q>
-__device__ __forceinline__ void tensor_line(T (&u)[N], const T *v, T wk, ctab tab) {
+template <int N, int Q>
+__device__ __forceinline__ void tensor_line(double (&u)[N], const double *v, double wk, ctab tab) {
   using S = TensorTab<N, Q>;
   constexpr int NE = S::NE, NO = S::NO, QE = S::QE, QO = S::QO;
-  T E[NE], O[NE], rE[NE], rO[NE];
+  double E[NE], O[NE], rE[NE], rO[NE];
 #pragma unroll
   for (int i = 0; i < NO; ++i) {
     E[i] = u[i] + u[N - 1 - i];
@@ -498,28 +501,28 @@ __device__ __forceinline__ void tensor_line(T (&u)[N], const T *v, T wk, ctab ta
   if constexpr (N & 1) E[NO] = u[NO];
 #pragma unroll
   for (int i = 0; i < NE; ++i) {
-    T t = tab[S::oKz + i * NE] * E[0];
+    double t = tab[S::oKz + i * NE] * E[0];
 #pragma unroll
     for (int j = 1; j < NE; ++j) t = fmadd(tab[S::oKz + i * NE + j], E[j], t);
     rE[i] = wk * t;
   }
 #pragma unroll
   for (int i = 0; i < NO; ++i) {
-    T t = tab[S::oKz + (NE + i) * NE] * O[0];
+    double t = tab[S::oKz + (NE + i) * NE] * O[0];
 #pragma unroll
     for (int j = 1; j < NO; ++j) t = fmadd(tab[S::oKz + (NE + i) * NE + j], O[j], t);
     rO[i] = wk * t;
   }
 #pragma unroll
   for (int k = 0; k < QE; ++k) {
-    T e = tab[S::oI + k * NE] * E[0], o = T(0);
+    double e = tab[S::oI + k * NE] * E[0], o = 0.0;
 #pragma unroll
     for (int i = 1; i < NE; ++i) e = fmadd(tab[S::oI + k * NE + i], E[i], e);
     if (k < QO) {
       o = tab[S::oI + (QE + k) * NE] * O[0];
 #pragma unroll
       for (int i = 1; i < NO; ++i) o = fmadd(tab[S::oI + (QE + k) * NE + i], O[i], o);
-      const T p = v[k] * (e + o), m = v[Q - 1 - k] * (e - o);
+      const double p = v[k] * (e + o), m = v[Q - 1 - k] * (e - o);
       e = p + m;
       o = p - m;
     } else {
@@ -722,7 +725,7 @@ struct Lines {
   }
   __device__ __forceinline__ T weight(int i) const { return tab[S::oW + i]; }
   __device__ __forceinline__ void potential(T (&u)[N], const T *v, T wk) const {
-    tensor_line<T, N, Q>(u, v, wk, tab);
+    tensor_line<N, Q>(u, v, wk, tab);
   }
 };
 
@@ -949,6 +952,26 @@ template <typename T>
 __device__ __forceinline__ T *row_ptr(T *p, uint32_t g, uint32_t ldb) {
   return (T *)((char *)p + (uint64_t)g * ldb);
 }
+// The four z lines mirrored in x and y, from their parity values at b<y><x>; hx, hy:
+// whether the index has an odd value (a middle one does not, it counts as zero)
+template <typename T, int N, int Q, int TC>
+__device__ __forceinline__ void pencil(const T *b00, const T *b01, const T *b10, const T *b11,
+                                       bool hx, bool hy, T (&u)[4][N]) {
+#pragma unroll
+  for (int z = 0; z < N; ++z) {
+    const int f = z * Q * Q * TC;
+    const T ee = b00[f];
+    const T oe = (Q & 1) && !hx ? T(0) : b01[f];
+    const T eo = (Q & 1) && !hy ? T(0) : b10[f];
+    const T oo = (Q & 1) && !(hx && hy) ? T(0) : b11[f];
+    const T s0 = ee + oe, d0 = ee - oe, s1 = eo + oo, d1 = eo - oo;
+    u[0][z] = s0 + s1;
+    u[1][z] = d0 + d1;
+    u[2][z] = s0 - s1;
+    u[3][z] = d0 - d1;
+  }
+}
+
 // CELLS: all cells in one launch, each writing its own sums to cells_out
 // [cell position in a.cells][node][column]; hx_assemble_kernel adds them up
 template <typename T, int N, int Q, int TC, int VW, bool CELLS>
@@ -1159,25 +1182,12 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
   // ---- z lines of u: four mirrored lines per thread
   for (int id = grp; id < QE * QE; id += GR) {
     const int ix = id % QE, iy = id / QE;
-    // the odd value of a middle index does not exist (and is zero)
     const bool hx = ix < QO, hy = iy < QO;
     T *b00 = buf + (iy * Q + ix) * TC + col;
     T *b01 = b00 + (hx ? QE : 0) * TC, *b10 = b00 + (hy ? QE : 0) * Q * TC,
       *b11 = b10 + (hx ? QE : 0) * TC;
     T u[4][N];
-#pragma unroll
-    for (int z = 0; z < N; ++z) {
-      const int f = z * Q * Q * TC;
-      const T ee = b00[f];
-      const T oe = (Q & 1) && !hx ? T(0) : b01[f];
-      const T eo = (Q & 1) && !hy ? T(0) : b10[f];
-      const T oo = (Q & 1) && !(hx && hy) ? T(0) : b11[f];
-      const T s0 = ee + oe, d0 = ee - oe, s1 = eo + oo, d1 = eo - oo;
-      u[0][z] = s0 + s1;
-      u[1][z] = d0 + d1;
-      u[2][z] = s0 - s1;
-      u[3][z] = d0 - d1;
-    }
+    pencil<T, N, Q, TC>(b00, b01, b10, b11, hx, hy, u);
     const T wk = lines.weight(ix) * lines.weight(iy);
     const T *v = svq + id * (4 * Q);
 #pragma unroll
@@ -1199,8 +1209,8 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
     }
   }
 
-  // ---- the destination's rows: loaded here so
-  // that they arrive while the last plane stages run
+  // ---- the destination's rows: loaded here so that they arrive while the last
+  // plane stages run
   vec dv[S::LT][N];
   if constexpr (!CELLS) {
 #pragma unroll
@@ -1210,7 +1220,7 @@ __attribute__((amdgpu_waves_per_eu(TensorShape<T, N, Q, TC, VW>::WPE))) void hx_
       for (int i = 0; i < N; ++i)
         dv[l][i] = vload<T, VW>(row_ptr(a.dst + vc, smap[lc * N + i] & 0x7fffffffu, ldd_b));
     }
-}
+  }
   __syncthreads();
   if (px) p1.collect(bq, o); else p0.collect(bq, o);
   __syncthreads();
@@ -1557,19 +1567,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void quad_tensor_kernel(
         const double *b01 = b00 + (hx ? QE : 0) * TC, *b10 = b00 + (hy ? QE : 0) * Q * TC,
                      *b11 = b10 + (hx ? QE : 0) * TC;
         double u[4][N];
-#pragma unroll
-        for (int z = 0; z < N; ++z) {
-          const int f = z * Q * Q * TC;
-          const double ee = b00[f];
-          const double oe = (Q & 1) && !hx ? 0.0 : b01[f];
-          const double eo = (Q & 1) && !hy ? 0.0 : b10[f];
-          const double oo = (Q & 1) && !(hx && hy) ? 0.0 : b11[f];
-          const double s0 = ee + oe, d0 = ee - oe, s1 = eo + oo, d1 = eo - oo;
-          u[0][z] = s0 + s1;
-          u[1][z] = d0 + d1;
-          u[2][z] = s0 - s1;
-          u[3][z] = d0 - d1;
-        }
+        pencil<double, N, Q, TC>(b00, b01, b10, b11, hx, hy, u);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           double E[NE], O[NE];
