@@ -133,15 +133,18 @@ bool gradient_products(const double *G, const std::vector<ld> &I, int n, int q, 
   const Index3 in(n), iq(q);
   std::vector<ld> D[3];
   for (auto &d : D) d.assign(size_t(q) * n, 0);
+  // means as for I (tensor_tables)
   double gmax = 0;
   for (int k = 0; k < nqc; ++k)
     for (int i = 0; i < ne; ++i) {
       const double *g = G + (size_t(k) * ne + i) * 3;
       for (int d = 0; d < 3; ++d) gmax = std::max(gmax, std::fabs(g[d]));
-      D[0][iq.x[k] * n + in.x[i]] += g[0] / ld(q * q);
-      D[1][iq.y[k] * n + in.y[i]] += g[1] / ld(q * q);
-      D[2][iq.z[k] * n + in.z[i]] += g[2] / ld(q * q);
+      if (iq.y[k] == iq.z[k]) D[0][iq.x[k] * n + in.x[i]] += g[0];
+      if (iq.z[k] == iq.x[k]) D[1][iq.y[k] * n + in.y[i]] += g[1];
+      if (iq.x[k] == iq.y[k]) D[2][iq.z[k] * n + in.z[i]] += g[2];
     }
+  for (auto &d : D)
+    for (ld &v : d) v /= q;
   const std::vector<double> Id(I.begin(), I.end());
   std::vector<double> Dd[3];
   for (int d = 0; d < 3; ++d) Dd[d].assign(D[d].begin(), D[d].end());
@@ -227,13 +230,17 @@ void fit_stiffness(const double *K, int n, std::vector<ld> &M, std::vector<ld> (
     // K times M in z, y, x: [ex][ey], [ex][ez], [ey][ez]
     std::vector<ld> xy(nn * nn, 0), xz(nn * nn, 0), yz(nn * nn, 0);
     for (int i = 0; i < ne; ++i)
-      for (int j = 0; j < ne; ++j) {
-        const int ex = in.x[i] * n + in.x[j], ey = in.y[i] * n + in.y[j],
-                  ez = in.z[i] * n + in.z[j];
-        const ld v = K[size_t(i) * ne + j];
-        xy[ex * nn + ey] += v * M[ez];
-        xz[ex * nn + ez] += v * M[ey];
-        yz[ey * nn + ez] += v * M[ex];
+      for (int j = 0; j < ne; j += n) {
+        const int xi = in.x[i] * n, ey = in.y[i] * n + in.y[j], ez = in.z[i] * n + in.z[j];
+        const double *k = K + size_t(i) * ne + j;
+        ld sum = 0;  // over x
+        for (int x = 0; x < n; ++x) {
+          const ld v = k[x];
+          xy[(xi + x) * nn + ey] += v * M[ez];
+          xz[(xi + x) * nn + ez] += v * M[ey];
+          sum += v * M[xi + x];
+        }
+        yz[ey * nn + ez] += sum;
       }
     const ld mm = dot(M, M);
     for (auto &d : D) d.assign(nn, 0);
@@ -275,17 +282,21 @@ bool tensor_tables(const double *Nq, const double *K, const double *G, int ne, i
   const double tol = 32 * eps, tol_k = 128 * eps;
   const Index3 in(n), iq(q);
   std::vector<ld> w = gauss_weights(q);
-  // I: sums of N over the nodes of the other two directions (which are one),
-  // mean over their quadrature points and over the directions; x is the
-  // fastest index of nodes and points
+  // I: sums of N over the nodes of the other two directions (which are one), mean
+  // over their points with two equal indices (q n^2 entries: far below rounding)
+  // and over the directions; x is the fastest index of nodes and points
   std::vector<ld> I(size_t(q) * n, 0), M(size_t(n) * n, 0), Kd[3];
-  for (int k = 0; k < nqc; ++k)
+  for (int k = 0; k < nqc; ++k) {
+    const bool yz = iq.y[k] == iq.z[k], zx = iq.z[k] == iq.x[k], xy = iq.x[k] == iq.y[k];
+    if (!(yz || zx || xy)) continue;
     for (int i = 0; i < ne; ++i) {
-      const ld v = Nq[size_t(k) * ne + i] / ld(3 * q * q);
-      I[iq.x[k] * n + in.x[i]] += v;
-      I[iq.y[k] * n + in.y[i]] += v;
-      I[iq.z[k] * n + in.z[i]] += v;
+      const ld v = Nq[size_t(k) * ne + i];
+      if (yz) I[iq.x[k] * n + in.x[i]] += v;
+      if (zx) I[iq.y[k] * n + in.y[i]] += v;
+      if (xy) I[iq.z[k] * n + in.z[i]] += v;
     }
+  }
+  for (ld &v : I) v /= 3 * q;
   // products of the cell matrix build: I I, and with shape gradients (nqc x ne x
   // 3, of the same form) 2 (D_d I + I D_d), [a][b][q], symmetric in a and b
   products->assign(size_t(n) * n * q, 0.0);
