@@ -773,9 +773,9 @@ struct OpData<float> {
   static const float *ones_cons(chfsi_operator *op) { return op->d_ones_cons32; }
 };
 
-// Projection of an operator whose variant was not set: owned rows on wide tiles
-// (variant 4) where their workgroups fill the chip, the cell form on 64 columns
-// (0) for less.  ms per apply, 0 / 4: p = 6, 4096 cells x 1024 columns FP32 6.07 / 5.79,
+// Projection of an operator whose variant was not set, by the columns of the whole
+// pass: owned rows on wide tiles (variant 4) where their workgroups fill the chip,
+// the cell form on 64 columns (0) for less.  ms per apply, 0 / 4: p = 6, 4096 cells x 1024 columns FP32 6.25 / 5.98,
 // 1728 cells x 333 FP64 2.29 / 2.14, x 1 0.27 / 0.26; p = 5, 1728 x 250 1.15 / 1.07;
 // p = 6, 216 cells x 16 0.175 / 0.189; p = 4, 512 x 64 0.141 / 0.147
 static int proj_default(int cells, int B) {

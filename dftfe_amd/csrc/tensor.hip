@@ -746,7 +746,9 @@ struct Lines {
 // of the result in four registers.  With the table entry A[l % 4][k] in the
 // first operand, four of them multiply each lane's own 4-vector by a 4 x 4
 // table: the parity blocks here, at twice the rate of 16 vector FMAs and beside
-// the vector pipe.
+// the vector pipe.  The second part of the stiffness tables is 84 more of them a wave:
+// 619 -> 657 us per colour launch on 1024 columns (512 cells, n = 7), the time of
+// these instructions alone.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
@@ -1414,9 +1416,9 @@ static hipError_t hx_tensor_vec(const HxLaunch<T> &a, const T *vq, const T *tab,
 
 // Where the tensor form is taken (cells: of the largest colour; one MI355X, ms per
 // apply, tensor / best tile variant or, for one column, the matrix-vector kernel):
-//   n = 7: 4096 cells x 1024 columns 5.8 / 11.0 FP32, 1728 x 1024 5.2 / 9.9 FP64,
+//   n = 7: 4096 cells x 1024 columns 6.1 / 11.0 FP32, 1728 x 1024 5.2 / 9.9 FP64,
 //          1728 x 16 0.21 / 0.86, x 1 0.16 / 0.48
-//   n = 6: 1728 cells x 256 columns 1.06 / 1.50 FP64, 0.58 / 0.80 FP32, x 1 0.16 / 0.29
+//   n = 6: 1728 cells x 256 columns 1.07 / 1.34 FP64, 0.61 / 0.79 FP32, x 1 0.16 / 0.29
 //   n = 5: the dense product is only 1.7 times the operations, on the matrix
 //          pipe; the tensor form has fewer bytes in flight behind its barriers
 //          and wins while a colour does not fill the chip.  us per apply, tensor /
