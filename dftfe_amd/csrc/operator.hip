@@ -903,8 +903,10 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
     a.want = kTensorForm;
   }
   // small blocks: one launch over all cells and a sum, where there is a buffer for
-  // the cells' sums (as for the projections: the operator's, one per
-  // precision, or the rest of the caller's scratch, which may take several steps)
+  // the cells' sums (as for the projections: the operator's, one per precision, or
+  // the rest of the caller's scratch).  Where the rest holds some of the columns
+  // only, p = 4 goes in steps (512 cells x 160 columns 185 us, colours 233), and
+  // larger cells by colours (p = 5, 512 x 192 302 us, in steps 350)
   T *co = nullptr;
   int step = 0;
   if (tensor && op->d_touch_ptr && op->n_slots > 0 &&
@@ -918,7 +920,7 @@ chfsi_status hx_fused(chfsi_operator *op, const T *src, int64_t ld_src, T *dst, 
       const size_t fit =
           ext_bytes > used ? (ext_bytes - used) / (sizeof(T) * size_t(op->C) * op->ne) : 0;
       co = reinterpret_cast<T *>(static_cast<char *>(ext_scratch) + used);
-      step = fit >= size_t(B) ? B : int(fit / 32 * 32);
+      step = fit >= size_t(B) ? B : op->tn == 5 ? int(fit / 32 * 32) : 0;
     }
   }
   all_cells = step > 0;
